@@ -120,6 +120,46 @@ __device__ __forceinline__ void zfmac(zc& acc, zc a, zc b) {
 }
 __device__ __forceinline__ double zabs2(zc a) { return a.x * a.x + a.y * a.y; }
 
+// Lane exchanges of a wave without the LDS crossbar (a __shfl_xor of a double is two of its round
+// trips, about 250 cycles): lane ^ M by data-parallel primitives inside a row of 16 lanes, and the
+// sums of the two halves of a wave or of each pair of rows by the lane-swap instructions.
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int M>
+__device__ __forceinline__ double lane_xor(double v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "inside a row of 16 lanes");
+  if constexpr (M == 1) return dpp_mov<0xb1>(v);                  // quad_perm 1 0 3 2
+  else if constexpr (M == 2) return dpp_mov<0x4e>(v);             // quad_perm 2 3 0 1
+  else if constexpr (M == 4) return dpp_mov<0x1b>(dpp_mov<0x141>(v));  // half-row mirror, then quad_perm 3 2 1 0
+  else return dpp_mov<0x128>(v);                                  // row rotate by 8
+}
+// Lanes 0..31 (M = 32) or the even rows of 16 (M = 16): a + a(lane ^ M); the others: b + b(lane ^ M).
+template <int M>
+__device__ __forceinline__ double swap_sum(double a, double b) {
+  static_assert(M == 16 || M == 32, "rows or halves");
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  auto sw = [](unsigned u, unsigned v) {
+    if constexpr (M == 32) return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+    else return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+  };
+  const auto lo = sw((unsigned)x, (unsigned)y), hi = sw((unsigned)(x >> 32), (unsigned)(y >> 32));
+  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) + __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+// Sum over the wave, in every lane (the order of a butterfly from distance 32 down to 1).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = swap_sum<32>(v, v);
+  v = swap_sum<16>(v, v);
+  v += lane_xor<8>(v);
+  v += lane_xor<4>(v);
+  v += lane_xor<2>(v);
+  return v + lane_xor<1>(v);
+}
+
 // Jacobi block geometry: pairs of JB-column blocks, i.e. JC = 2*JB columns
 // are orthogonalised together by one workgroup.
 constexpr int JB = 16;

@@ -17,7 +17,7 @@
 //   k_qrp_colnorms     column norms (one wave per column)
 //   k_qrp_begin        ||W||_F, identity pivot, rank := running
 //   k_qrp_panel_reg    panel j0 for Rb <= 1024: the QB largest remaining columns are
-//                      gathered into registers (512 threads, one or two rows each),
+//                      gathered into registers (two to eight waves, one or two rows a thread),
 //                      factorised there (one 32-value reduce-scatter per reflector
 //                      gives the reflector's products with the later panel columns
 //                      and the earlier reflectors at once) and stored in place, with
@@ -43,8 +43,7 @@ namespace {
 
 constexpr int QB = 16;          // panel width
 constexpr int kMaxCols = 4096;  // largest Cb (d chi_max <= 4096)
-constexpr int PT = 512;         // threads of the register-resident panel kernel
-constexpr int PW = PT / 64;     // its waves
+constexpr int PW = 8;           // most waves of the register-resident panel kernel
 
 // Calls f(std::integral_constant<int, i>) for i = 0 .. N-1 in order (a loop whose index is
 // a compile-time constant in every iteration).
@@ -58,11 +57,6 @@ __device__ __forceinline__ void static_for_impl(F&& f) {
 template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl<0, N>(f);
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
 }
 
 // Fixed-order sum over the 256 threads of a workgroup (bitwise reproducible).
@@ -215,10 +209,11 @@ __device__ __forceinline__ bool householder(zc alpha, double xn2, zc& tau, doubl
   if (xn2 == 0.0 && alpha.y == 0.0) return false;
   const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
   beta = alpha.x >= 0.0 ? -nrm : nrm;
-  tau = zmk((beta - alpha.x) / beta, -alpha.y / beta);
+  const double ib = 1.0 / beta;
+  tau = zmk((beta - alpha.x) * ib, -alpha.y * ib);
   const zc am = zmk(alpha.x - beta, alpha.y);
-  const double den = zabs2(am);
-  scale = zmk(am.x / den, -am.y / den);
+  const double id = 1.0 / zabs2(am);
+  scale = zmk(am.x * id, -am.y * id);
   return true;
 }
 
@@ -340,9 +335,22 @@ __device__ __forceinline__ void move_rows(zc* Wq, size_t ld, int i, int nmv, con
   }
 }
 
-// Panel j0 with the panel in registers (Rb <= RPT * PT; one workgroup of PT threads per
-// task, thread t owns rows t + PT s, s < RPT):
-//  1. wave 0 picks the nbp = min(QB, kmax - j0) columns of largest remaining norm in
+// LDS of the register-resident panel.
+struct PanelLds {
+  double snrm[kMaxCols + 1];
+  int sel[QB], mv_src[QB], mv_dst[QB];
+  int snmv, sstop;
+  double red[PW][32];
+  double wsum[PW][32];
+  double rnorm[PW];
+  zc salpha;
+  zc G[QB][QB + 1];
+  zc stau[QB];
+};
+
+// Panel j0 with the panel in registers (Rb <= RPT * 64 NW, NW waves; thread t owns rows
+// t + 64 NW s, s < RPT):
+//  1. the nbp = min(QB, kmax - j0) columns of largest remaining norm are picked in
 //     descending order (ties: lowest index); if even the largest is below the stop
 //     threshold the numerical rank is j0 and the factorisation ends;
 //  2. the picked columns are loaded into registers; the displaced ones are moved;
@@ -350,52 +358,44 @@ __device__ __forceinline__ void move_rows(zc* Wq, size_t ld, int i, int nmv, con
 //     reflector q one fixed-order reduction yields w_k = v_q^H a_k (k > q, for the
 //     update) and G[p][q] = v_p^H v_q (p < q, for T);
 //  4. the panel is stored back and T formed.
-template <int RPT>
-__global__ __launch_bounds__(PT) void k_qrp_panel_reg(const BondTask* __restrict__ tasks, int j0) {
-  const BondTask t = tasks[blockIdx.x];
-  if (t.qstate[0] >= 0.0) return;
+// The 16 reflectors are one dependent chain, bound by the instructions each SIMD issues for
+// it: per reflector a wave spends about 300 on the norm, the Householder scalars and the
+// 32-value reduction and 120 RPT on its rows, so few waves with two rows per thread beat
+// many with one; exchanging lanes by data-parallel moves and lane swaps instead of the LDS
+// crossbar, and one barrier less, shorten the rest.  With eight waves for every row count a
+// panel took 52 us at 128 rows, 65 at 225 and 73 at 400; now 32, 44 and 62.
+template <int RPT, int NW>
+__device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S) {
+  constexpr int NT = 64 * NW;
   const int Rb = t.Rb, Cb = t.Cb;
   const int kmax = Rb < Cb ? Rb : Cb;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (j0 >= kmax) {
-    if (tid == 0) t.qstate[0] = (double)kmax;
-    return;
-  }
   const int nbp = (kmax - j0) < QB ? (kmax - j0) : QB;
   const int ncand = Cb - j0;
   const size_t ld = Rb;
-  __shared__ double snrm[kMaxCols + 1];
-  __shared__ int sel[QB], mv_src[QB], mv_dst[QB];
-  __shared__ int snmv, sstop;
-  __shared__ double red[PW][32];
-  __shared__ double wsum[32];
-  __shared__ double rnorm[PW];
-  __shared__ zc salpha;
-  __shared__ zc G[QB][QB + 1];
-  __shared__ zc stau[QB];
 
   // 1. selection
-  for (int k = tid; k < ncand; k += PT) snrm[k] = t.qnrm[j0 + k];
-  select_panel<PT>(snrm, ncand, nbp, t.qstate[1], j0, sel, &sstop, tid);
-  if (sstop) {
-    if (tid == 0) t.qstate[0] = sstop == 1 ? (double)j0 : 0.0;
+  for (int k = tid; k < ncand; k += NT) S.snrm[k] = t.qnrm[j0 + k];
+  select_panel<NT>(S.snrm, ncand, nbp, t.qstate[1], j0, S.sel, &S.sstop, tid);
+  if (S.sstop) {
+    if (tid == 0) t.qstate[0] = S.sstop == 1 ? (double)j0 : 0.0;
     return;
   }
   if (wave == 0) {
-    const int n = panel_moves(t, j0, nbp, sel, mv_src, mv_dst, lane);
-    if (lane == 0) snmv = n;
+    const int n = panel_moves(t, j0, nbp, S.sel, S.mv_src, S.mv_dst, lane);
+    if (lane == 0) S.snmv = n;
   }
   __syncthreads();
 
   // 2. gather the panel; each thread moves its own rows of the displaced columns
   zc a[RPT][QB];
-  const int nmv = snmv;
+  const int nmv = S.snmv;
 #pragma unroll
   for (int s = 0; s < RPT; ++s) {
-    const int i = tid + PT * s;
+    const int i = tid + NT * s;
 #pragma unroll
-    for (int q = 0; q < QB; ++q) a[s][q] = (i < Rb && q < nbp) ? t.Wq[i + ld * sel[q]] : zmk(0.0, 0.0);
-    if (i < Rb) move_rows(t.Wq, ld, i, nmv, mv_src, mv_dst);
+    for (int q = 0; q < QB; ++q) a[s][q] = (i < Rb && q < nbp) ? t.Wq[i + ld * S.sel[q]] : zmk(0.0, 0.0);
+    if (i < Rb) move_rows(t.Wq, ld, i, nmv, S.mv_src, S.mv_dst);
   }
 
   // 3. Householder QR of the panel, the column loop unrolled so that every register
@@ -408,24 +408,24 @@ __global__ __launch_bounds__(PT) void k_qrp_panel_reg(const BondTask* __restrict
     double part = 0.0;
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
-      const int i = tid + PT * s;
+      const int i = tid + NT * s;
       if (i > j && i < Rb) part += zabs2(a[s][q]);
-      if (i == j) salpha = a[s][q];
+      if (i == j) S.salpha = a[s][q];
     }
     part = wave_sum(part);
-    if (lane == 0) rnorm[wave] = part;
+    if (lane == 0) S.rnorm[wave] = part;
     __syncthreads();
     double xn2 = 0.0;
 #pragma unroll
-    for (int w = 0; w < PW; ++w) xn2 += rnorm[w];
+    for (int w = 0; w < NW; ++w) xn2 += S.rnorm[w];
     zc tau, scale = zmk(1.0, 0.0);
     double beta = 0.0;
-    const bool refl = householder(salpha, xn2, tau, beta, scale);
+    const bool refl = householder(S.salpha, xn2, tau, beta, scale);
     // v_q (rows > j; v_j = 1 implicitly) and R(j, j)
     if (refl) {
 #pragma unroll
       for (int s = 0; s < RPT; ++s) {
-        const int i = tid + PT * s;
+        const int i = tid + NT * s;
         if (i > j && i < Rb) a[s][q] = zmul(a[s][q], scale);
         if (i == j) a[s][q] = zmk(beta, 0.0);
       }
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(PT) void k_qrp_panel_reg(const BondTask* __restrict
     zc vq[RPT];
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
-      const int i = tid + PT * s;
+      const int i = tid + NT * s;
       vq[s] = (i == j) ? zmk(1.0, 0.0) : ((i > j && i < Rb) ? a[s][q] : zmk(0.0, 0.0));
     }
 #pragma unroll
@@ -458,44 +458,41 @@ __global__ __launch_bounds__(PT) void k_qrp_panel_reg(const BondTask* __restrict
     // 16 b5 + 8 b4 + 4 b3 + 2 b2 + b1 (b = bits of l), summed over all 64 lanes
     {
       double y16[16], y8[8], y4[4], y2[2];
-      const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
+      const bool h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
 #pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        const double lo = x[m], hi = x[m + 16];
-        y16[m] = (h5 ? hi : lo) + __shfl_xor(h5 ? lo : hi, 32, 64);
-      }
+      for (int m = 0; m < 16; ++m) y16[m] = swap_sum<32>(x[m], x[m + 16]);
 #pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const double lo = y16[m], hi = y16[m + 8];
-        y8[m] = (h4 ? hi : lo) + __shfl_xor(h4 ? lo : hi, 16, 64);
-      }
+      for (int m = 0; m < 8; ++m) y8[m] = swap_sum<16>(y16[m], y16[m + 8]);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const double lo = y8[m], hi = y8[m + 4];
-        y4[m] = (h3 ? hi : lo) + __shfl_xor(h3 ? lo : hi, 8, 64);
+        y4[m] = (h3 ? hi : lo) + lane_xor<8>(h3 ? lo : hi);
       }
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
         const double lo = y4[m], hi = y4[m + 2];
-        y2[m] = (h2 ? hi : lo) + __shfl_xor(h2 ? lo : hi, 4, 64);
+        y2[m] = (h2 ? hi : lo) + lane_xor<4>(h2 ? lo : hi);
       }
-      double y1 = (h1 ? y2[1] : y2[0]) + __shfl_xor(h1 ? y2[0] : y2[1], 2, 64);
-      y1 += __shfl_xor(y1, 1, 64);
+      double y1 = (h1 ? y2[1] : y2[0]) + lane_xor<2>(h1 ? y2[0] : y2[1]);
+      y1 += lane_xor<1>(y1);
       const int idx = 16 * ((lane >> 5) & 1) + 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) +
                       2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
-      if ((lane & 1) == 0) red[wave][idx] = y1;
+      if ((lane & 1) == 0) S.red[wave][idx] = y1;
     }
     __syncthreads();
-    if (tid < 32) {
+    // every wave sums the waves' partials for itself, which saves a barrier
+    if (lane < 32) {
       double sum = 0.0;
 #pragma unroll
-      for (int w = 0; w < PW; ++w) sum += red[w][tid];
-      wsum[tid] = sum;
+      for (int w = 0; w < NW; ++w) sum += S.red[w][lane];
+      S.wsum[wave][lane] = sum;
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const double* const wsum = S.wsum[wave];
     if (tid == 0) {
-      for (int m = QB - q; m < QB; ++m) G[m - QB + q][q] = zmk(wsum[2 * m], wsum[2 * m + 1]);
-      stau[q] = tau;
+      for (int m = QB - q; m < QB; ++m) S.G[m - QB + q][q] = zmk(wsum[2 * m], wsum[2 * m + 1]);
+      S.stau[q] = tau;
       t.tau[j] = tau;
     }
     if (refl) {
@@ -512,15 +509,40 @@ __global__ __launch_bounds__(PT) void k_qrp_panel_reg(const BondTask* __restrict
   // 4. store the panel (R above and on the diagonal, reflectors below) and T
 #pragma unroll
   for (int s = 0; s < RPT; ++s) {
-    const int i = tid + PT * s;
+    const int i = tid + NT * s;
     if (i < Rb) {
 #pragma unroll
       for (int c = 0; c < QB; ++c)
         if (c < nbp) t.Wq[i + ld * (j0 + c)] = a[s][c];
     }
   }
-  form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
+}
+
+// One workgroup per task; the shape of its panel depends on the task's own row count, so a
+// task is factorised the same way whatever batch it is in.  Waves that a task does not need
+// leave at once.
+template <int NWMAX>
+__global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __restrict__ tasks, int j0) {
+  const BondTask t = tasks[blockIdx.x];
+  if (t.qstate[0] >= 0.0) return;
+  const int kmax = t.Rb < t.Cb ? t.Rb : t.Cb;
+  if (j0 >= kmax) {
+    if (threadIdx.x == 0) t.qstate[0] = (double)kmax;
+    return;
+  }
+  __shared__ PanelLds S;
+  const int wave = threadIdx.x >> 6;
+  if (t.Rb <= 128) {
+    if (wave < 2) panel_reg<1, 2>(t, j0, S);
+  } else if (NWMAX >= 4 && t.Rb <= 256) {
+    if (wave < 4) panel_reg<1, NWMAX < 4 ? NWMAX : 4>(t, j0, S);
+  } else if (NWMAX >= 8 && t.Rb <= 512) {
+    if (wave < 4) panel_reg<2, NWMAX < 4 ? NWMAX : 4>(t, j0, S);
+  } else if (NWMAX >= 8) {
+    panel_reg<2, NWMAX>(t, j0, S);
+  }
 }
 
 // Panel j0 through global memory (any Rb; one workgroup of 256 threads per task): the
@@ -1065,8 +1087,9 @@ hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, dou
 
 hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, hipStream_t st) {
   if (max_cb > kMaxCols) return hipErrorInvalidValue;
-  if (max_rb <= PT) hipLaunchKernelGGL(k_qrp_panel_reg<1>, dim3(ntasks), dim3(PT), 0, st, d_tasks, j0);
-  else if (max_rb <= 2 * PT) hipLaunchKernelGGL(k_qrp_panel_reg<2>, dim3(ntasks), dim3(PT), 0, st, d_tasks, j0);
+  if (max_rb <= 128) hipLaunchKernelGGL(k_qrp_panel_reg<2>, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
+  else if (max_rb <= 256) hipLaunchKernelGGL(k_qrp_panel_reg<4>, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+  else if (max_rb <= 1024) hipLaunchKernelGGL(k_qrp_panel_reg<8>, dim3(ntasks), dim3(512), 0, st, d_tasks, j0);
   else hipLaunchKernelGGL(k_qrp_panel, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
   return hipGetLastError();
 }
