@@ -31,13 +31,16 @@ constexpr int kGemmRegions = 8;  // GEMM descriptor arrays per batch (learned pa
 // 1/kProbeSafety of the true value with probability
 // P(Gamma(16, 1) < 1.6) = P(Poisson(1.6) >= 16) < 2e-11.
 constexpr double kProbeSafety = 10.0;
-constexpr int kSweepHist = 16;                      // sweeps tallied one by one in the histograms
+constexpr int kSweepHist = kSweepBins;              // sweeps tallied one by one in the histograms
 constexpr int kNumStats = 14 + 2 * kSweepHist;
 constexpr int kNumProf = 28;
 constexpr double kQrTol = 1e-17;  // QR stops when every remaining column norm is <= kQrTol ||theta||_F
 constexpr int kQrPanel = 16;      // panel width of the blocked pivoted QR (tebd_qrp.hip)
 constexpr int kQrCheck = 8;       // panels between checks whether every task has stopped
-constexpr int kQrMinCols = 64;    // bond matrices with fewer columns go straight to the Jacobi
+// Bond matrices with no side of at least kQrMinSide go straight to the Jacobi, solved in one
+// launch (tebd_jacobi_small.hip).  A chain's edge bonds (4 x 256, say) are preconditioned with the
+// bulk's: on their own they held up the half-sweep by 160-320 us.
+constexpr int kQrMinSide = 64;
 constexpr int kMaxSweeps = 40;
 constexpr double kTolRel = 1e-13;   // relative orthogonality of converged column pairs
 constexpr double kTolAbs = 1e-13;   // rounding floor: |A_pq| <= kTolAbs ||theta|| (|w_p| + |w_q|)
@@ -101,7 +104,7 @@ struct tebd_ctx {
   double* h_qstate = nullptr;    // pinned, 2 per task slot
   double* s = nullptr;
   int* perm = nullptr;
-  int* counters = nullptr;       // 4 per task slot (BondTask::counter)
+  int* counters = nullptr;       // kCounters per task slot (BondTask::counter)
   unsigned* blkver = nullptr;    // nblk_max per task slot
   unsigned long long* pairseen = nullptr;  // nblk_max^2 per task slot
   int nblk_max = 0;
@@ -192,7 +195,7 @@ struct tebd_ctx {
   std::vector<int> last_rank;    // kept rank of each bond's last update (rank model input)
   std::vector<double> last_trunc;  // discarded weight (fraction) of each bond's last update
   double* h_results = nullptr;   // pinned
-  int* h_counters = nullptr;     // pinned, 4 per task slot
+  int* h_counters = nullptr;     // pinned, kCounters per task slot
   std::vector<zc> staging;
   std::string err;
   // [0] bond updates, [1] Jacobi sweeps, [2] sketch fallbacks, [3] device ms of trotter steps,
@@ -312,7 +315,7 @@ hipError_t theta_gate(tebd_ctx* c, const BondTask* d_t, int nb, int max_chil, in
 
 // Gives task `slot` of a batch its Jacobi counters and block bookkeeping.
 void attach_jacobi(tebd_ctx* c, BondTask& t, int slot) {
-  t.counter = c->counters + 4 * slot;
+  t.counter = c->counters + kCounters * slot;
   t.blkver = c->blkver + (size_t)slot * c->nblk_max;
   t.pairseen = c->pairseen + (size_t)slot * c->nblk_max * c->nblk_max;
   t.Qg = c->Qg + (size_t)slot * (c->nblk_max / 2) * JC * JC;
@@ -346,14 +349,71 @@ hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int c
   return ge;
 }
 
-// Jacobi sweeps over the tasks of one stage (task i uses slot i) until a sweep
-// rotates nothing.
-int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, int Pmax) {
-  HIPCHK(c, launch_jacobi_begin(d_t, nb, c->st));
-  int rows_w = 1, rows_v = 0;
+// Tasks solved by k_jacobi_small: bond matrices of at most 2 pairs of column blocks that skip
+// the QR preconditioning.
+bool small_solve(const BondTask& t) { return !t.qr && t.P <= kSmallPairs; }
+
+// After the tasks' counters have reached h_counters: checks that the small solves converged
+// and adds every task's work to the statistics.  `sweeps`: sweeps of the large solves, which
+// have already entered their rotations per sweep.
+int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, int sweeps, bool converged) {
   for (int i = 0; i < nb; ++i) {
+    if (!small_solve(h_t[i])) continue;
+    const int* cnt = c->h_counters + kCounters * i;
+    if (cnt[4] < 1) converged = false;
+    sweeps = std::max(sweeps, cnt[4]);
+    for (int s = 0; s < kSweepHist; ++s) c->stats[14 + s] += cnt[8 + s];
+  }
+  c->stats[1] += sweeps;
+  if (sweeps > 0) c->stats[14 + kSweepHist + std::min(sweeps, kSweepHist) - 1] += 1;
+  for (int i = 0; i < nb; ++i) {
+    const BondTask& t = h_t[i];
+    const double visits = c->h_counters[kCounters * i + 2], rots = c->h_counters[kCounters * i + 3];
+    const double rows = t.R + (t.V ? t.NV : 0);
+    c->stats[8] += visits;
+    c->stats[9] += rots;
+    c->stats[10] += (double)(small_solve(t) ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
+    if (c->profiling && !small_solve(t)) {
+      // k_jacobi_round, per formed Gram: the 16x16 cross block over R rows (8 flops per
+      // complex MAC) reading the pair's JC columns once, and per rotated pair its JC x JC
+      // rotation written; k_jacobi_rotate, per rotated pair: the JC columns of W and V
+      // read and written once, JC complex MACs per element
+      c->prof[6] += visits * 8.0 * t.R * JB * JB;
+      c->prof[7] += visits * 16.0 * t.R * JC + rots * 16.0 * JC * JC;
+      c->prof[22] += rots * 8.0 * rows * JC * JC;
+      c->prof[23] += rots * 32.0 * rows * JC;
+    }
+  }
+  if (!converged) return fail(c, TEBD_ERR_NOCONV, "one-sided Jacobi did not converge");
+  return TEBD_OK;
+}
+
+hipError_t fetch_counters(tebd_ctx* c, int nb) {
+  return hipMemcpyAsync(c->h_counters, c->counters, sizeof(int) * kCounters * nb, hipMemcpyDeviceToHost, c->st);
+}
+
+// Jacobi SVDs of the tasks of one stage (task i uses slot i): the small ones in one launch,
+// the others sweep by sweep until one rotates nothing.  When every task is small nothing is
+// waited for: *deferred is set, the counters' copy to the host is queued, and the caller
+// calls jacobi_account after its next wait.
+int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool* deferred) {
+  HIPCHK(c, launch_jacobi_begin(d_t, nb, c->st));
+  int rows_w = 1, rows_v = 0, Pmax = 0;
+  bool one = false, two = false;
+  for (int i = 0; i < nb; ++i) {
+    if (small_solve(h_t[i])) {
+      (h_t[i].P == 1 ? one : two) = true;
+      continue;
+    }
+    Pmax = std::max(Pmax, h_t[i].P);
     rows_w = std::max(rows_w, h_t[i].R);
     if (h_t[i].V) rows_v = std::max(rows_v, h_t[i].NV);
+  }
+  if (one || two) HIPCHK(c, launch_jacobi_small(d_t, nb, one, two, kTolRel, kTolAbs, kMaxSweeps, c->st));
+  *deferred = Pmax == 0;
+  if (*deferred) {
+    HIPCHK(c, fetch_counters(c, nb));
+    return TEBD_OK;
   }
   // The rotation kernel reads the rows only as a count of 64-row slabs and every slab
   // checks its task's own row count, so rounding up to whole slabs launches the same
@@ -396,36 +456,15 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, int P
         HIPCHK(c, launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st));
       }
     }
-    HIPCHK(c, hipMemcpyAsync(c->h_counters, c->counters, sizeof(int) * 4 * nb, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, fetch_counters(c, nb));
     HIPCHK(c, hipStreamSynchronize(c->st));
     int rot = 0;
-    for (int i = 0; i < nb; ++i) rot += c->h_counters[4 * i + (sweeps & 1)];
+    for (int i = 0; i < nb; ++i) rot += c->h_counters[kCounters * i + (sweeps & 1)];
     converged = rot == 0;
     c->stats[14 + std::min(sweeps, kSweepHist - 1)] += rot;
     ++sweeps;
   }
-  c->stats[1] += sweeps;
-  c->stats[14 + kSweepHist + std::min(sweeps, kSweepHist) - 1] += 1;
-  for (int i = 0; i < nb; ++i) {
-    const BondTask& t = h_t[i];
-    const double visits = c->h_counters[4 * i + 2], rots = c->h_counters[4 * i + 3];
-    const double rows = t.R + (t.V ? t.NV : 0);
-    c->stats[8] += visits;
-    c->stats[9] += rots;
-    c->stats[10] += (double)sweeps * t.P * (2 * t.P - 1);
-    if (c->profiling) {
-      // k_jacobi_round, per formed Gram: the 16x16 cross block over R rows (8 flops per
-      // complex MAC) reading the pair's JC columns once, and per rotated pair its JC x JC
-      // rotation written; k_jacobi_rotate, per rotated pair: the JC columns of W and V
-      // read and written once, JC complex MACs per element
-      c->prof[6] += visits * 8.0 * t.R * JB * JB;
-      c->prof[7] += visits * 16.0 * t.R * JC + rots * 16.0 * JC * JC;
-      c->prof[22] += rots * 8.0 * rows * JC * JC;
-      c->prof[23] += rots * 32.0 * rows * JC;
-    }
-  }
-  if (!converged) return fail(c, TEBD_ERR_NOCONV, "one-sided Jacobi did not converge");
-  return TEBD_OK;
+  return jacobi_account(c, h_t, nb, sweeps, converged);
 }
 
 // Compact-WY factors kept per slot: one kQrPanel^2 block per panel, min(Rb, Cb) <= Cpmax.
@@ -501,23 +540,23 @@ int qrp_factor(tebd_ctx* c, BondTask* D, const BondTask* H, int nb, int max_cb, 
 
 // SVD + truncation of the tasks' bond matrices (in W; tasks D / H, task i uses slot
 // i and results[i]): singular values, kept rank, lambda (into lc_out) and truncerr.
-// Bond matrices with at least kQrMinCols columns are first reduced by the pivoted
+// Bond matrices with a side of at least kQrMinSide are first reduced by the pivoted
 // QR; the one-sided Jacobi then runs on R^dagger and the kept singular vectors are
 // formed into Yr / Zc.  On return h_results holds every task's results and *max_k
 // the largest kept rank.
-int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, int Cpmax, int Pmax, bool force_qr,
-               bool* used_qr, int* max_k) {
+int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, int Cpmax, bool force_qr, bool* used_qr,
+               int* max_k) {
   int max_cb = 1, max_rb = 1;
   for (int i = 0; i < nb; ++i) {
     max_cb = std::max(max_cb, H[i].Cb);
     max_rb = std::max(max_rb, H[i].Rb);
   }
-  // The QR preconditioning is decided per task (bond matrices with at least
-  // kQrMinCols columns, or all with force_qr), so a bond's result does not depend on
+  // The QR preconditioning is decided per task (bond matrices with a side of at least
+  // kQrMinSide, or all with force_qr), so a bond's result does not depend on
   // which other bonds share its batch.
   std::vector<int> qidx;
   for (int i = 0; i < nb; ++i)
-    if (force_qr || H[i].Cb >= kQrMinCols) qidx.push_back(i);
+    if (force_qr || H[i].Rb >= kQrMinSide) qidx.push_back(i);
   const int nq = (int)qidx.size();
   const bool use_qr = nq > 0;
   int max_rank = 1;
@@ -553,18 +592,15 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
       t.NV = t.Cpad;
     }
     Cpmax = 1;
-    Pmax = 1;
-    for (int i = 0; i < nb; ++i) {
-      Cpmax = std::max(Cpmax, H[i].Cpad);
-      Pmax = std::max(Pmax, H[i].P);
-    }
+    for (int i = 0; i < nb; ++i) Cpmax = std::max(Cpmax, H[i].Cpad);
     HIPCHK(c, hipMemcpyAsync(D, H, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
     HIPCHK(c, launch_qrp_build_x(D, nb, c->st));
   }
   HIPCHK(c, launch_prepare_svd(D, nb, c->st));
   HIPCHK(c, launch_frobenius(D, nb, Cpmax, c->st, 0));
+  bool deferred = false;
   {
-    int e = jacobi_sweeps(c, D, H, nb, Pmax);
+    int e = jacobi_sweeps(c, D, H, nb, &deferred);
     if (e) return e;
   }
   {
@@ -573,6 +609,10 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
   }
   HIPCHK(c, hipMemcpyAsync(c->h_results, c->results, sizeof(double) * RESULT_STRIDE * nb, hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
+  if (deferred) {
+    int e = jacobi_account(c, H, nb, 0, true);
+    if (e) return e;
+  }
   *max_k = 1;
   for (int i = 0; i < nb; ++i) {
     const double* r = c->h_results + RESULT_STRIDE * i;
@@ -598,10 +638,10 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
 }
 
 // svd_factor of the batch (stage-0 tasks) followed by the new Gammas and lambda.
-int svd_truncate(tebd_ctx* c, const int* links, int nb, int Cpmax, int Pmax) {
+int svd_truncate(tebd_ctx* c, const int* links, int nb, int Cpmax) {
   bool used_qr = false;
   int max_k = 1;
-  int e = svd_factor(c, c->d_tasks, c->h_tasks, links, nb, Cpmax, Pmax, false, &used_qr, &max_k);
+  int e = svd_factor(c, c->d_tasks, c->h_tasks, links, nb, Cpmax, false, &used_qr, &max_k);
   if (e) return e;
   {
     ProfScope ps(c, 2);
@@ -722,13 +762,12 @@ void account_theta(tebd_ctx* c, const BondTask* h, int nb) {
 }
 
 int run_bonds_full(tebd_ctx* c, const int* links, int nb, const zc* const* gate_ptrs, double* trunc_sum) {
-  int max_chil = 1, max_chir = 1, Pmax = 1, Cpmax = 1;
+  int max_chil = 1, max_chir = 1, Cpmax = 1;
   for (int i = 0; i < nb; ++i) {
     BondTask& t = c->h_tasks[i];
     make_full_task(c, t, links[i], gate_ptrs[i], i);
     max_chil = std::max(max_chil, t.chil);
     max_chir = std::max(max_chir, t.chir);
-    Pmax = std::max(Pmax, t.P);
     Cpmax = std::max(Cpmax, t.Cpad);
   }
   HIPCHK(c, hipMemcpyAsync(c->d_tasks, c->h_tasks, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
@@ -737,7 +776,7 @@ int run_bonds_full(tebd_ctx* c, const int* links, int nb, const zc* const* gate_
     HIPCHK(c, theta_gate(c, c->d_tasks, nb, max_chil, max_chir));
   }
   account_theta(c, c->h_tasks, nb);
-  int e = svd_truncate(c, links, nb, Cpmax, Pmax);
+  int e = svd_truncate(c, links, nb, Cpmax);
   if (e) return e;
   double tsum = 0.0;
   for (int i = 0; i < nb; ++i) {
@@ -819,8 +858,8 @@ int run_bonds_learned(tebd_ctx* c, const int* links, int nb, const zc* const* ga
   std::vector<const zc*> fb_gates;
   for (int i : full) {
     const int link = links[i];
-    const int C = d * std::min(c->chi[link], c->chi[link + 2]);
-    if (ns > 0 && C >= kQrMinCols) {
+    const int R = d * std::max(c->chi[link], c->chi[link + 2]);
+    if (ns > 0 && R >= kQrMinSide) {
       merged.push_back(i);
     } else {
       fb_links.push_back(link);
@@ -948,7 +987,7 @@ int run_bonds_learned(tebd_ctx* c, const int* links, int nb, const zc* const* ga
     account_theta(c, S3 + ns, nf);
     int max_k = 1;
     bool used_qr = false;
-    e = svd_factor(c, D3, S3, all_links.data(), ns + nf, round_up(max_ry, JC), round_up(max_ry, JC) / JC, true,
+    e = svd_factor(c, D3, S3, all_links.data(), ns + nf, round_up(max_ry, JC), true,
                    &used_qr, &max_k);
     if (e) return e;
     for (int j = 0; j < nf; ++j) {
@@ -1137,7 +1176,7 @@ struct SvdJob {
 };
 
 int device_svd_batch(tebd_ctx* c, const SvdJob* jobs, int nb) {
-  int Pmax = 1, Cpmax = 1;
+  int Cpmax = 1;
   for (int i = 0; i < nb; ++i) {
     BondTask& t = c->h_tasks[i];
     std::memset(&t, 0, sizeof(t));
@@ -1147,14 +1186,18 @@ int device_svd_batch(tebd_ctx* c, const SvdJob* jobs, int nb) {
     t.result = c->results + (size_t)RESULT_STRIDE * i;
     t.chi_max = t.C;
     t.lc_out = jobs[i].lam_scratch;
-    Pmax = std::max(Pmax, t.P);
     Cpmax = std::max(Cpmax, t.Cpad);
   }
   HIPCHK(c, hipMemcpyAsync(c->d_tasks, c->h_tasks, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, launch_prepare_svd(c->d_tasks, nb, c->st));
   HIPCHK(c, launch_frobenius(c->d_tasks, nb, Cpmax, c->st, 0));
-  int e = jacobi_sweeps(c, c->d_tasks, c->h_tasks, nb, Pmax);
+  bool deferred = false;
+  int e = jacobi_sweeps(c, c->d_tasks, c->h_tasks, nb, &deferred);
   if (e) return e;
+  if (deferred) {  // the task descriptors are rewritten by the next batch: wait here as after a sweep
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    if ((e = jacobi_account(c, c->h_tasks, nb, 0, true))) return e;
+  }
   HIPCHK(c, launch_col_norms(c->d_tasks, nb, Cpmax, c->st));
   HIPCHK(c, launch_truncate(c->d_tasks, nb, 0.0, c->st));
   return TEBD_OK;
@@ -1545,7 +1588,7 @@ int run_bonds_nc(tebd_ctx* c, const int* links, int nb, const zc* const* gate_pt
       const int n = (int)std::min(live.size() - q0, (size_t)wn);
       chunk_blk.assign(n, NcBlock{});
       err_links.assign(n, 0);
-      int Cpm = 1, Pm = 1;
+      int Cpm = 1;
       for (int q = 0; q < n; ++q) {
         const NcBlock& b = blocks[live[q0 + q]];
         BondTask& t = S[q];
@@ -1572,14 +1615,13 @@ int run_bonds_nc(tebd_ctx* c, const int* links, int nb, const zc* const* gate_pt
         chunk_blk[q].W = t.W;
         err_links[q] = t.link;
         Cpm = std::max(Cpm, t.Cpad);
-        Pm = std::max(Pm, t.P);
       }
       HIPCHK(c, hipMemcpyAsync(c->d_nc_blk, chunk_blk.data(), sizeof(NcBlock) * n, hipMemcpyHostToDevice, w->st));
       HIPCHK(c, hipMemcpyAsync(DS, S, sizeof(BondTask) * n, hipMemcpyHostToDevice, w->st));
       HIPCHK(c, launch_nc_gather(c->d_nc_blk, n, c->d_nc_part, w->st));
       bool used_qr = false;
       int max_k = 1;
-      int ef = svd_factor(w, DS, S, err_links.data(), n, Cpm, Pm, false, &used_qr, &max_k);
+      int ef = svd_factor(w, DS, S, err_links.data(), n, Cpm, true, &used_qr, &max_k);
       if (!ef) {
         HIPCHK(c, launch_nc_vectors(c->d_nc_blk, DS, n, max_k, w->st));
         HIPCHK(c, hipMemcpyAsync(w->h_nc_s, w->s, sizeof(double) * w->Cpmax * n, hipMemcpyDeviceToHost, w->st));
@@ -1764,8 +1806,8 @@ tebd_ctx* make_lane(tebd_ctx* c, int lane, int slot0, int nslots) {
   l->qstate = c->qstate + 2 * s0;
   l->h_qstate = c->h_qstate + 2 * s0;
   l->Tq = c->Tq + s0 * tq_stride(c);
-  l->counters = c->counters + 4 * s0;
-  l->h_counters = c->h_counters + 4 * s0;
+  l->counters = c->counters + kCounters * s0;
+  l->h_counters = c->h_counters + kCounters * s0;
   l->blkver = c->blkver + s0 * c->nblk_max;
   l->pairseen = c->pairseen + s0 * c->nblk_max * c->nblk_max;
   l->Qg = c->Qg + s0 * (c->nblk_max / 2) * JC * JC;
@@ -2313,7 +2355,7 @@ constexpr size_t kNoAllocBytes =
     5 * na_up(sizeof(zc) * kNoAllocSide * kNoAllocSide) +                      // W, V, X, Yr, Zc
     2 * na_up(sizeof(double) * kNoAllocSide) + 2 * na_up(sizeof(int) * kNoAllocSide) +  // s, qnrm, perm, qpiv
     na_up(sizeof(zc) * kNoAllocSide) + na_up(sizeof(double) * 2) +              // tau, qstate
-    na_up(sizeof(zc) * kNoAllocTq) + na_up(sizeof(int) * 4) +                   // Tq, counters
+    na_up(sizeof(zc) * kNoAllocTq) + na_up(sizeof(int) * kCounters) +                   // Tq, counters
     na_up(sizeof(unsigned) * kNoAllocNblk) + na_up(sizeof(unsigned long long) * kNoAllocNblk * kNoAllocNblk) +
     na_up(sizeof(zc) * (kNoAllocNblk / 2) * JC * JC) + na_up(sizeof(int) * 2) +  // Qg, wl_count
     na_up(sizeof(int2) * 2 * (kNoAllocNblk / 2)) + 2 * na_up(sizeof(double) * RESULT_STRIDE) +
@@ -2352,7 +2394,7 @@ void noalloc_layout(tebd_ctx* c, unsigned char* base) {
   c->tau = (zc*)take(sizeof(zc) * n);
   c->qstate = (double*)take(sizeof(double) * 2);
   c->Tq = (zc*)take(sizeof(zc) * kNoAllocTq);
-  c->counters = (int*)take(sizeof(int) * 4);
+  c->counters = (int*)take(sizeof(int) * kCounters);
   c->blkver = (unsigned*)take(sizeof(unsigned) * kNoAllocNblk);
   c->pairseen = (unsigned long long*)take(sizeof(unsigned long long) * kNoAllocNblk * kNoAllocNblk);
   c->Qg = (zc*)take(sizeof(zc) * (kNoAllocNblk / 2) * JC * JC);
@@ -2373,7 +2415,7 @@ size_t split_stride(const tebd_ctx* c) { return (size_t)2 * kSplitSlices * split
 double slot_bytes(const tebd_ctx* c) {
   const double R = c->Rmax, Cp = c->Cpmax, chi = c->chi_max, nblk = c->nblk_max, z = sizeof(zc);
   double b = z * (R * Cp + 2.0 * Cp * Cp + R * chi + Cp * chi + Cp) + 8.0 * Cp * 2 + 4.0 * Cp * 2 + 16.0 +
-             z * (double)tq_stride(c) + 16.0 + 4.0 * nblk + 8.0 * nblk * nblk + z * (nblk / 2) * JC * JC +
+             z * (double)tq_stride(c) + 4.0 * kCounters + 4.0 * nblk + 8.0 * nblk * nblk + z * (nblk / 2) * JC * JC +
              16.0 * (nblk / 2) + 2.0 * 8 * RESULT_STRIDE + 4.0 * TEBD_MLP_INPUTS + 4.0 +
              2.0 * kStages * sizeof(BondTask);
   if (c->mode & TEBD_MODE_LEARNED_RANK)
@@ -2455,7 +2497,7 @@ int create_impl(tebd_ctx** out, int nchain, int Lc, int d, int chi_max, int orde
   if (bad(hipMalloc(&c->qstate, sizeof(double) * 2 * nt))) return TEBD_ERR_HIP;
   if (bad(hipMalloc(&c->Tq, sizeof(zc) * tq_stride(c) * nt))) return TEBD_ERR_HIP;
   if (bad(hipHostMalloc(&c->h_qstate, sizeof(double) * 2 * nt))) return TEBD_ERR_HIP;
-  if (bad(hipMalloc(&c->counters, sizeof(int) * 4 * nt))) return TEBD_ERR_HIP;
+  if (bad(hipMalloc(&c->counters, sizeof(int) * kCounters * nt))) return TEBD_ERR_HIP;
   if (bad(hipMalloc(&c->blkver, sizeof(unsigned) * c->nblk_max * nt))) return TEBD_ERR_HIP;
   if (bad(hipMalloc(&c->pairseen, sizeof(unsigned long long) * c->nblk_max * c->nblk_max * nt))) return TEBD_ERR_HIP;
   if (bad(hipMalloc(&c->Qg, sizeof(zc) * (size_t)(c->nblk_max / 2) * JC * JC * nt))) return TEBD_ERR_HIP;
@@ -2496,7 +2538,7 @@ int create_impl(tebd_ctx** out, int nchain, int Lc, int d, int chi_max, int orde
   c->last_rank.assign(L + 1, 0);
   c->last_trunc.assign(L + 1, 0.0);
   if (bad(hipHostMalloc(&c->h_results, sizeof(double) * RESULT_STRIDE * nt))) return TEBD_ERR_HIP;
-  if (bad(hipHostMalloc(&c->h_counters, sizeof(int) * 4 * nt))) return TEBD_ERR_HIP;
+  if (bad(hipHostMalloc(&c->h_counters, sizeof(int) * kCounters * nt))) return TEBD_ERR_HIP;
   *out = c;
   return TEBD_OK;
 }
@@ -3059,7 +3101,7 @@ int tebd_two_site_op_noalloc(int d, int chi_l, int chi_c, int chi_r, int chi_cap
   // host staging of the one task (pageable: no pinned allocation either)
   static BondTask h_tasks[kStages];
   static double h_results[RESULT_STRIDE], h_qstate[2];
-  static int h_counters[4];
+  static int h_counters[kCounters];
   tebd_ctx c;
   c.d = d;
   c.chi_max = chi_cap;
@@ -3115,7 +3157,7 @@ int tebd_two_site_op_noalloc(int d, int chi_l, int chi_c, int chi_r, int chi_cap
     return TEBD_ERR_HIP;
   }
   const int link = 0;
-  int e = svd_truncate(&c, &link, 1, t.Cpad, t.P);
+  int e = svd_truncate(&c, &link, 1, t.Cpad);
   if (e) {
     (void)hipStreamSynchronize(c.st);  // nothing of this call may still run when the next one starts
     return e;

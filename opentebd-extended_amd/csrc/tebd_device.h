@@ -164,6 +164,11 @@ __device__ __forceinline__ double wave_sum(double v) {
 // are orthogonalised together by one workgroup.
 constexpr int JB = 16;
 constexpr int JC = 2 * JB;
+// Ints per task of BondTask::counter: [0..1] rotated pairs per sweep parity, [2] Gram visits,
+// [3] rotations; of a small solve (tebd_jacobi_small.hip) [4] sweeps run (0: not converged)
+// and [8 + s] pairs rotated in sweep s (the last bin: that sweep and later ones).
+constexpr int kSweepBins = 16;
+constexpr int kCounters = 8 + kSweepBins;
 
 // One bond update ("task") as the kernels see it.
 struct BondTask {
@@ -185,7 +190,7 @@ struct BondTask {
   int NV;
   double* s;         // Cpad: sorted singular values (descending)
   int* perm;         // Cpad: original column of each sorted value
-  int* counter;      // Jacobi counters: [0..1] rotated pairs per sweep parity, [2] Gram visits, [3] rotations
+  int* counter;      // kCounters Jacobi counters
   unsigned* blkver;  // 2P: rotations of each column block in the current solve
   unsigned long long* pairseen;  // (2P)^2: block versions when a pair was last verified orthogonal
   zc* Qg;            // P x 32 x 32: each pair's rotation of the current round, row-major

@@ -347,6 +347,7 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   const BondTask t = tasks[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= t.P || round >= 2 * t.P - 1) return;
+  if (!t.qr && t.P <= kSmallPairs) return;  // solved by k_jacobi_small
   int* cnt = t.counter;
   if (sweep > 0 && cnt[(sweep - 1) & 1] == 0) return;  // converged in the previous sweep
   const int nblk = 2 * t.P;
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(256) void k_jacobi_rotate(const BondTask* __restric
 __global__ void k_jacobi_begin(const BondTask* __restrict__ tasks) {
   const BondTask t = tasks[blockIdx.x];
   const int nblk = 2 * t.P;
-  if (threadIdx.x < 4) t.counter[threadIdx.x] = 0;
+  if (threadIdx.x < kCounters) t.counter[threadIdx.x] = 0;
   for (int e = threadIdx.x; e < nblk; e += blockDim.x) t.blkver[e] = 0u;
   for (int e = threadIdx.x; e < nblk * nblk; e += blockDim.x) t.pairseen[e] = ~0ull;
 }
