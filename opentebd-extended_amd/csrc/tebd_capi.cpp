@@ -44,12 +44,6 @@ constexpr int kQrMinSide = 64;
 constexpr int kMaxSweeps = 40;
 constexpr double kTolRel = 1e-13;   // relative orthogonality of converged column pairs
 constexpr double kTolAbs = 1e-13;   // rounding floor: |A_pq| <= kTolAbs ||theta|| (|w_p| + |w_q|)
-// Every outer sweep solves each pair's 32 x 32 problem with at most kInnerSweepCap inner
-// sweeps (fewer when one finds nothing to rotate): a pair left coupled is revisited by the
-// next outer sweep.  Measured on Fermi-Hubbard bonds at 1024 x 288: one inner sweep per
-// visit doubles the outer sweeps; three take 4.9 outer sweeps per solve against 6.0 with
-// two, and more than three add inner rounds without saving outer sweeps.
-constexpr int kInnerSweepCap = 3;
 constexpr double kSlotBudget = 48.0 * (1ull << 30);  // bytes of per-bond workspace slots per context
 constexpr size_t kMaxSweepGraphs = 512;  // executable Jacobi sweep graphs kept per context or lane
 constexpr int kGraphRowQuantum = 64;     // = the rotation kernel's slab height (tebd_jacobi.hip)
@@ -227,7 +221,7 @@ struct tebd_ctx {
   // hipGraphs of whole Jacobi sweeps (sweep start, every round and rotation), keyed by
   // the launch arguments; used while per-launch profiling is off
   bool graphs = true;
-  std::map<std::array<long long, 7>, hipGraphExec_t> sweep_graphs;
+  std::map<std::array<long long, 6>, hipGraphExec_t> sweep_graphs;
   bool is_lane = false;
   bool owns_gemm = false;  // a lane that allocated its own GEMM descriptors
   bool owns_stream = true;  // false for lane 0, which runs on its context's stream
@@ -329,13 +323,12 @@ void clear_graphs(tebd_ctx* c) {
 // One Jacobi sweep (sweep start, then every round's Gram/eigenproblem kernel and its
 // rotation kernel) captured from the context's stream as an executable graph; null if
 // the capture fails.  The captured launches are the eager ones with the same arguments.
-hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int cls, int inner, int rows_w,
-                             int rows_v) {
+hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int cls, int rows_w, int rows_v) {
   if (hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
   hipError_t e = launch_jacobi_sweep_begin(d_t, nb, cls, c->wl_count, c->st);
   for (int r = 0; r < 2 * Pmax - 1 && e == hipSuccess; ++r) {
     e = launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count, c->wl_items,
-                            c->wl_cap, inner, c->st);
+                            c->wl_cap, c->st);
     if (e == hipSuccess)
       e = launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st);
   }
@@ -423,19 +416,18 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
   int sweeps = 0;
   bool converged = false;
   while (sweeps < kMaxSweeps && !converged) {
-    const int inner = kInnerSweepCap;
     // the kernels read the sweep index only as (sweep > 0) and its parity, so 0, 1 and 2
     // stand for every sweep of their class and one graph serves the whole class
     const int cls = sweeps == 0 ? 0 : ((sweeps & 1) ? 1 : 2);
     bool done = false;
     if (c->graphs && !c->profiling) {
-      const std::array<long long, 7> key = {(long long)(uintptr_t)d_t, nb, Pmax, rows_w, rows_v, cls, inner};
+      const std::array<long long, 6> key = {(long long)(uintptr_t)d_t, nb, Pmax, rows_w, rows_v, cls};
       auto it = c->sweep_graphs.find(key);
       // A full cache is not emptied while the context runs: executable graphs are
       // destroyed only when the context (or its lane) is freed, after its stream has
       // drained.  Sweeps of shapes beyond the cap launch eagerly.
       if (it == c->sweep_graphs.end() && c->sweep_graphs.size() < kMaxSweepGraphs) {
-        hipGraphExec_t ge = capture_sweep(c, d_t, nb, Pmax, cls, inner, rows_w, rows_v);
+        hipGraphExec_t ge = capture_sweep(c, d_t, nb, Pmax, cls, rows_w, rows_v);
         if (ge) it = c->sweep_graphs.emplace(key, ge).first;
         else c->graphs = false;  // capture unavailable: launch eagerly from now on
       }
@@ -450,7 +442,7 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
         {
           ProfScope ps(c, 1);
           HIPCHK(c, launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count,
-                                        c->wl_items, c->wl_cap, inner, c->st));
+                                        c->wl_items, c->wl_cap, c->st));
         }
         ProfScope ps(c, 5);
         HIPCHK(c, launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st));

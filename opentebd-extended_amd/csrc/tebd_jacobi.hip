@@ -6,18 +6,24 @@
 // other (round-robin "circle" order, 2P-1 rounds per sweep).  A round is two kernels:
 //   k_jacobi_round   one workgroup per pair: the pair's Gram matrix on FP64 MFMA
 //                    (v_mfma_f64_16x16x4f64), the decision whether it needs a
-//                    rotation, and the 32x32 Hermitian eigenproblem by cyclic Jacobi
-//                    in LDS -> Q (32x32, to global memory); rotated pairs are queued;
+//                    rotation, and one pass of rotations over its index pairs in LDS
+//                    (tebd_jacobi_inner.h) -> Q (32x32, to global memory); rotated pairs are
+//                    queued;
 //   k_jacobi_rotate  [W; V](:, pair) <- [W; V](:, pair) Q for every queued pair, on
 //                    MFMA, spread over 64-row slabs so a rotation costs one memory
 //                    round trip of the whole GPU instead of one workgroup's stream.
-// After a block has been part of a rotated (or verified) pair its columns are
-// mutually orthogonal, so after the first round of a sweep only the 16x16 cross
-// block and the 32 column norms are formed (4x less Gram work than the full 32x32).
-// The first round of every sweep forms the full Gram of each pair: with a strongly
-// graded spectrum the rounding of rotations lets the small columns of a block drift
-// away from orthogonality, and that round restores it (a cross-only iteration does
-// not converge there).
+// Only the first round of a sweep forms the full Gram of each pair and rotates the pairs
+// within the blocks too; the other rounds form the 16x16 cross block and the 32 column norms
+// (4x less Gram work), take the columns of a block as orthogonal and rotate the cross pairs
+// once.  With a strongly graded spectrum the rounding of rotations lets the small columns of
+// a block drift away from orthogonality, and the first round restores it (a cross-only
+// iteration does not converge there).
+//
+// A pair visit is bound by the latency of its rounds of rotations: three cyclic sweeps over
+// all index pairs per visit (93 rounds, two barriers each) took 59 us at 400 x 400
+// (Fermi-Hubbard, chi = 100) and 54 at 225 x 225 (Bose-Hubbard, chi = 45); one pass over the
+// cross pairs (16 rounds of one barrier) takes 17 and 15, for 6 to 7 outer sweeps instead of 5
+// to 6.
 //
 // Work that cannot change the result is skipped exactly:
 //   * a task whose previous sweep rotated nothing has converged: its workgroups exit;
@@ -27,7 +33,10 @@
 // sweep parity), counter[2] pairs whose Gram was formed and counter[3] rotated pairs
 // over the whole SVD; blkver[b] counts rotations of block b and pairseen[lo*2P+hi]
 // holds (blkver[lo], blkver[hi]) from the last time that pair was verified.
+#include <type_traits>
+
 #include "tebd_device.h"
+#include "tebd_jacobi_inner.h"
 #include "tebd_kernels.h"
 
 namespace {
@@ -41,9 +50,7 @@ __device__ __forceinline__ d4 mfma4(double a, double b, d4 c) {
 }
 
 // k_jacobi_round runs 8 waves: all of them form the Gram matrix; in the inner solve
-// waves 0-3 update one 2x2 block of A per thread and waves 4-7 the rotation
-// accumulator Q, so that no wave issues both (a round costs about the longest wave's
-// instruction stream).
+// waves 0-3 update A and waves 4-7 the rotation accumulator Q.
 constexpr int kRoundThreads = 512;
 constexpr int kGramWaves = kRoundThreads / 64;
 
@@ -55,43 +62,32 @@ __device__ __forceinline__ void rr_pair(int nb, int round, int p, int& bi, int& 
   bj = pos(nb - 1 - p);
 }
 
-// 1/sqrt(x) and 1/x to full FP64 precision: the hardware estimate refined by two
-// Newton-Raphson steps (y <- y (3 - x y^2) / 2, r <- r (2 - x r)).
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  return y * fma(-0.5 * x * y, y, 1.5);
-}
-__device__ __forceinline__ double rcp_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = r * fma(-x, r, 2.0);
-  return r * fma(-x, r, 2.0);
-}
-
 // Hermitian 2x2 Jacobi rotation J = [[c, s w], [-s conj(w), c]], w = g/|g|, that
 // zeroes g in [[a, g], [conj(g), b]] via J^dagger H J, with the inner angle
-// (|theta| <= pi/4, Rutishauser's smaller root).  With e = sqrt((b - a)^2 + 4|g|^2),
-// cos 2theta = |b - a| / e and sin 2theta = 2|g| / e, and the half-angle formulas give
-// c = sqrt((1 + cos 2theta) / 2) = (1 + cos 2theta) r and |s| = sin 2theta / (2c) =
-// sin 2theta r with r = 1/sqrt(2 (1 + cos 2theta)); s takes the sign of b - a.  Every
-// step is well conditioned (1 + cos 2theta lies in [1, 2]) and nothing overflows for tiny
-// |g|.  The two first reciprocal square roots are independent, so the rotation's
-// critical path holds two refined estimates.  Returns c, s w and t|g|, t = s / c =
-// sign(b - a) sin 2theta / (1 + cos 2theta) = sign(b - a) sin 2theta 2 r^2: the rotated
-// diagonal is (a - t|g|, b + t|g|).
-__device__ __forceinline__ void jrot(double a, double b, zc g, double& c, zc& sw, double& tg) {
-  const double g2 = zabs2(g);
-  if (g2 == 0.0) { c = 1.0; sw = zmk(0.0, 0.0); tg = 0.0; return; }
+// (|theta| <= pi/4, Rutishauser's smaller root).  tan theta = t = 2|g| sign(b - a) /
+// (|b - a| + sqrt((b - a)^2 + 4|g|^2)); t w is formed without |g|.  The hardware
+// estimates of the square root and the quotient (about 2^-24, one Newton-Raphson step on
+// the quotient) suffice for t: an angle that is off by 1e-7 of itself leaves 1e-7 of
+// the coupling for the next sweep.  c = 1/sqrt(1 + t^2) is refined to full precision (two
+// steps) and s = c t, so the rotation is unitary to rounding whatever t's error.
+// a and b become the rotated diagonal a - t|g|, b + t|g|.
+__device__ __forceinline__ void jrot(double& a, double& b, zc g, double g2, double& c, zc& sw) {
   const double dd = b - a;
-  const double inv = rsqrt_nr(g2);
-  const double re = rsqrt_nr(fma(dd, dd, 4.0 * g2));
-  const double h = fma(fabs(dd), re, 1.0);  // 1 + cos 2theta
-  const double sin2 = (2.0 * g2 * inv) * re;
-  const double r = rsqrt_nr(2.0 * h);
-  c = h * r;
-  const double s = dd < 0.0 ? -sin2 * r : sin2 * r;
-  sw = zmk(s * (g.x * inv), s * (g.y * inv));
-  tg = (dd < 0.0 ? -sin2 : sin2) * (2.0 * r * r) * (g2 * inv);
+  const double e2 = fma(dd, dd, 4.0 * g2);
+  const double den = fma(e2, __builtin_amdgcn_rsq(e2), fabs(dd));
+  double inv = __builtin_amdgcn_rcp(den);
+  inv = inv * fma(-den, inv, 2.0);
+  const double f = dd < 0.0 ? -2.0 * inv : 2.0 * inv;
+  const double tx = f * g.x, ty = f * g.y;
+  const double h = fma(tx, tx, fma(ty, ty, 1.0));
+  double r = __builtin_amdgcn_rsq(h);
+  const double hh = 0.5 * h;
+  r = r * fma(-hh * r, r, 1.5);
+  r = r * fma(-hh * r, r, 1.5);
+  c = r;
+  sw = zmk(tx * r, ty * r);
+  a = fma(-f, g2, a);
+  b = fma(f, g2, b);
 }
 
 // Gram block D = X^H Y (16 x 16) of two 16-column blocks over rows [0, R), as
@@ -132,218 +128,168 @@ __device__ __forceinline__ void gram_block(const zc* __restrict__ X, const zc* _
 }
 
 // Sums the Gram waves' partial 16x16 blocks in a fixed order (bitwise reproducible)
-// and stores rows [ro, ro+16) x cols [co, co+16) of A.  With `diag` the block is a
-// diagonal block of the Hermitian A: only the upper triangle is taken and mirrored.
-// The real and the imaginary parts go through the scratch `red` ((kGramWaves - 1) x 256
-// doubles) one after the other, so that it fits in the rotation accumulator's LDS, which
-// is free until the inner solve starts.  Called by every thread of the workgroup.
-__device__ __forceinline__ void reduce_block(zc (*A)[JC + 1], double (*red)[256], d4 gre, d4 gim, int wave, int lane,
-                                             int ro, int co, bool diag) {
-  double xr[4];
-  if (wave > 0 && wave < kGramWaves) {
+// and stores rows [ro, ro+16) x cols [co, co+16) of the upper triangle of A (diagonal
+// blocks: the real diagonal goes to dg).  Every thread sums one real or imaginary part from
+// the scratch `red`, which shares its storage with the rotation accumulator.  Called by
+// every thread of the workgroup.
+__device__ __forceinline__ void reduce_block(zc (*A)[kInnerLd], double* dg, double (*red)[512], d4 gre, d4 gim, int wave,
+                                             int lane, int ro, int co, bool diag) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) red[wave - 1][g * 64 + lane] = gre[g];
+  for (int g = 0; g < 4; ++g) {
+    red[wave][g * 64 + lane] = gre[g];
+    red[wave][256 + g * 64 + lane] = gim[g];
   }
   __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      xr[g] = gre[g];
-      for (int w = 0; w < kGramWaves - 1; ++w) xr[g] += red[w][g * 64 + lane];
-    }
+  {
+    const int e = threadIdx.x, idx = e & 255, l = idx & 63, im = e >> 8;
+    double v = red[0][e];
+    for (int w = 1; w < kGramWaves; ++w) v += red[w][e];
+    const int p = (l >> 4) + 4 * (idx >> 6), q = l & 15;
+    if (!diag || p < q) reinterpret_cast<double*>(&A[ro + p][co + q])[im] = v;
+    else if (p == q && !im) dg[ro + p] = v;
   }
   __syncthreads();
-  if (wave > 0 && wave < kGramWaves) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) red[wave - 1][g * 64 + lane] = gim[g];
-  }
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      double xi = gim[g];
-      for (int w = 0; w < kGramWaves - 1; ++w) xi += red[w][g * 64 + lane];
-      const int p = (lane >> 4) + 4 * g, q = lane & 15;
-      if (!diag) {
-        A[ro + p][co + q] = zmk(xr[g], xi);
-        A[co + q][ro + p] = zmk(xr[g], -xi);
-      } else if (p < q) {
-        A[ro + p][co + q] = zmk(xr[g], xi);
-        A[co + q][ro + p] = zmk(xr[g], -xi);
-      } else if (p == q) {
-        A[ro + p][co + p] = zmk(xr[g], 0.0);
+}
+
+static_assert(kRoundThreads == 512 && JB == kInnerPairs, "the inner solve's thread roles");
+
+// Index pair t (t < 16) of round r of level h (h = 1, 2, 4, 8 or 16): the 32 indices in
+// groups of 2h, the lower half of a group against its upper half shifted by r.  Level 16
+// pairs the two column blocks with each other; levels 8, 4, 2 and 1 pair each block within
+// itself.  Over rounds 0 .. h-1 of every level each index pair meets exactly once.
+__host__ __device__ constexpr int level_p(int h, int t) { return 2 * t - (t & (h - 1)); }
+__host__ __device__ constexpr int level_q(int h, int r, int t) {
+  return level_p(h, t) - (t & (h - 1)) + h + (((t & (h - 1)) + r) & (h - 1));
+}
+
+// The schedules: kCross the 16 rounds of level 16 (pair t's next entry lies in block (t, t + 1),
+// the last one's in block (0, 15)), kFull the 15 rounds of levels 8, 4, 2, 1 and then kCross.
+constexpr int kWithinRounds = JB - 1;
+using CrossTable = InnerTable<JB, 2 * kInnerPairs>;
+using FullTable = InnerTable<kAllRounds, 2 * kOffBlocks>;
+template <class Table>
+constexpr Table level_table(int first_level) {
+  Table t{};
+  int rd = 0;
+  for (int lv = 0; lv < 5; ++lv) {
+    const int h = lv < 4 ? 8 >> lv : 16;
+    if (lv < first_level) continue;
+    for (int r = 0; r < h; ++r, ++rd)
+      for (int x = 0; x < kInnerPairs; ++x) {
+        t.p[rd][x] = (unsigned char)level_p(h, x);
+        t.q[rd][x] = (unsigned char)level_q(h, r, x);
       }
+  }
+  int br[16] = {}, bk[16] = {};
+  for (int x = 0; x < 16; ++x) {
+    br[x] = x < 15 ? x : 0;
+    bk[x] = x < 15 ? x + 1 : 15;
+  }
+  return complete_table(t, br, bk);
+}
+__device__ constexpr CrossTable kCross = level_table<CrossTable>(4);
+__device__ constexpr FullTable kFull = level_table<FullTable>(0);
+
+// Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
+// sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
+// blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
+// includes the blocks' own couplings, the pairs within the blocks too, in two passes.
+// Measured on Hubbard and Bose-Hubbard bonds (numpy restatement, 225 x 225 and 256 x 256):
+// 6 outer sweeps and 1300-1400 inner rounds in sequence per solve; three cyclic sweeps over
+// all 496 pairs per visit take 5 outer sweeps but 4400-4650 rounds in sequence.
+// Waves 0..3 update A; waves 4..7 apply the rotations to Q: in level 16 from registers (lane t
+// of a 16-lane row has two rows' entries at p_t, which stays, and q_t, which comes from the next
+// lane in every round), in the other levels in LDS.
+template <bool FULL, class Rounds>
+__device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1], double* dg, RotBuf* rb, const Rounds& T,
+                                             int tid) {
+  constexpr int NN = FULL ? 2 * kOffBlocks : 2 * kInnerPairs, RW = FULL ? kWithinRounds : 0;
+  const bool is_a = tid < 2 * kOffBlocks, is_q = tid >= 256;
+  const int tr = is_a ? kCross.tr[tid] : 0, tk = is_a ? kCross.tk[tid] : 0, half = tid & 1;
+  const int qt = tid & 15, qk = (tid >> 4) & 15;
+  if (FULL) {
+    for (int e = tid; e < JC * JC; e += kRoundThreads) Q[e / JC][e % JC] = zmk(e / JC == e % JC ? 1.0 : 0.0, 0.0);
+    __syncthreads();
+  }
+  zc f[2], s[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    f[u] = zmk(qk + 16 * u == qt ? 1.0 : 0.0, 0.0);
+    s[u] = zmk(qk + 16 * u == qt + 16 ? 1.0 : 0.0, 0.0);
+  }
+  int buf = 0;
+#pragma unroll 1
+  for (int pass = 0; pass < (FULL ? 2 : 1); ++pass) {
+    if (tid < kInnerPairs) {
+      const int p = level_p(FULL ? 8 : 16, tid), q = level_q(FULL ? 8 : 16, 0, tid);
+      A[p][q] = make_rotation(rb[buf], dg[p], dg[q], &dg[p], &dg[q], nullptr, tid, A[p][q], jrot);
     }
-  }
-  __syncthreads();
-}
-
-constexpr int kInnerSweeps = 30;
-
-// Index pair t (t < JC/2) of inner round rd (rd < JC - 1), lower index first: rr_pair
-// on JC indices, with its reduction mod JC - 1 done by one compare (the argument is
-// below 2 (JC - 1)) instead of a general modulo, which costs several multiplies per
-// use inside the inner rounds.
-__device__ __forceinline__ void inner_pair(int rd, int t, int& p, int& q) {
-  auto pos = [rd](int k) {
-    int x = k - 1 + rd;
-    x = x >= JC - 1 ? x - (JC - 1) : x;
-    return k == 0 ? 0 : 1 + x;
-  };
-  const int a = pos(t), b = pos(JC - 1 - t);
-  p = a < b ? a : b;
-  q = a < b ? b : a;
-}
-
-// Cyclic Jacobi on A (JC x JC Hermitian, LDS); Q (LDS) accumulates the rotations.
-// A round rotates 16 disjoint index pairs (round-robin order) in two phases:
-//   phase 1  lanes 0..15 of wave 0 compute the round's rotations into one of two
-//            buffers and write each rotated pair's own 2x2 block of A, which the
-//            rotation makes diagonal: a' = a - t|g|, b' = b + t|g| (t = s / c), the
-//            annihilated entries exactly zero.  Meanwhile waves 1..7 apply the previous
-//            round's rotations to Q (Q_:p <- c Q_:p - s conj(w) Q_:q,
-//            Q_:q <- s w Q_:p + c Q_:q; 512 (row, pair) groups), which nothing in this
-//            round reads;
-//   phase 2  the 240 threads of waves 0..3 update the off-diagonal blocks
-//            [p_r, q_r] x [p_k, q_k], r < k, of A (J^H A J acts on each such block on
-//            its own, so the update is in place): two threads per block, one per row,
-//            each also writing the mirrored entries of block (k, r) (A is Hermitian).
-// Blocks whose two pairs both stay put are skipped, and so is phase 2 of a round that
-// rotates nothing.  The last round's Q update runs after the loop.  A Gram entry is
-// accurate relative to sqrt(A_pp A_qq), so the solve uses a purely relative test (no
-// rotation when |A_pq| <= 1e-15 sqrt(A_pp A_qq)) and ends when a sweep would rotate
-// nothing.  That is decided by testing every pair once after a sweep: a sweep that
-// rotates nothing leaves A unchanged, so it rotates nothing iff no pair passes the test
-// now.
-__device__ __forceinline__ bool needs_rotation(zc g, double a, double b) {
-  const double g2 = zabs2(g);
-  return !(g2 <= 1e-30 * fabs(a * b) || g2 == 0.0);
-}
-
-static_assert(kRoundThreads == JC * JC / 2, "one thread per group of Q after the last round");
-constexpr int kOffBlocks = (JC / 2) * (JC / 2 - 1) / 2;  // 2x2 blocks above the diagonal
-static_assert(2 * kOffBlocks <= 256, "phase 2 runs on waves 0..3");
-
-// Rotations of one round, pair t: c, s w, and p | q << 8 | (rotates) << 16.
-struct RotBuf {
-  double c[JC / 2];
-  zc sw[JC / 2];
-  int pq[JC / 2];
-};
-
-// Applies the rotations of buffer rb to group grp = 16 k + t of Q: row k, pair t.
-__device__ __forceinline__ void q_rotate(zc (*Q)[JC + 1], const RotBuf& rb, int grp) {
-  const int k = grp >> 4, tp = grp & 15;
-  const int pq = rb.pq[tp];
-  const double c = rb.c[tp];
-  const zc sw = rb.sw[tp];
-  if (!(pq >> 16)) return;
-  const int p = pq & 255, q = (pq >> 8) & 255;
-  const zc xp = Q[k][p], xq = Q[k][q];
-  Q[k][p] = zsub(zscale(xp, c), zmul(zconj(sw), xq));
-  Q[k][q] = zadd(zmul(sw, xp), zscale(xq, c));
-}
-
-__device__ void inner_jacobi(zc (*A)[JC + 1], zc (*Q)[JC + 1], RotBuf* rb, int* s_round, int* s_sweep,
-                             int* s_more, int tid, int max_sweeps) {
-  for (int e = tid; e < JC * JC; e += kRoundThreads) {
-    const int r = e % JC, c = e / JC;
-    Q[r][c] = zmk(r == c ? 1.0 : 0.0, 0.0);
-  }
-  // phase 2 owner: block (tr, tk), tr < tk, of the upper triangle, row `half` of it
-  const int ob = tid >> 1, half = tid & 1;
-  int tr = 0, tk = 0;
-  if (ob < kOffBlocks) {
-    int rem = ob;
-    while (rem >= JC / 2 - 1 - tr) {
-      rem -= JC / 2 - 1 - tr;
-      ++tr;
-    }
-    tk = tr + 1 + rem;
-  }
-  int g = 0;  // rounds started, over all sweeps: round g uses buffer g & 1
-  for (int isw = 0; isw < max_sweeps; ++isw) {
-    if (tid == 0) s_sweep[isw & 1] = 0;
-    for (int rd = 0; rd < JC - 1; ++rd, ++g) {
-      const int cur = g & 1;
-      if (tid < 64) {
-        if (tid == 0) s_round[cur] = 0;
-        if (tid < JC / 2) {
-          int pp, qq;
-          inner_pair(rd, tid, pp, qq);
-          const zc gv = A[pp][qq];
-          const double a = A[pp][pp].x, b = A[qq][qq].x;
-          double c = 1.0;
-          zc sw = zmk(0.0, 0.0);
-          int rot = 0;
-          if (needs_rotation(gv, a, b)) {
-            double tg;
-            jrot(a, b, gv, c, sw, tg);
-            A[pp][pp] = zmk(a - tg, 0.0);
-            A[qq][qq] = zmk(b + tg, 0.0);
-            A[pp][qq] = zmk(0.0, 0.0);
-            A[qq][pp] = zmk(0.0, 0.0);
-            rot = 1;
-            s_round[cur] = 1;
-            s_sweep[isw & 1] = 1;
+    __syncthreads();
+    if (FULL) {
+      int rd = 0;
+#pragma unroll 1
+      for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll 1
+        for (int r = 0; r < h; ++r, ++rd, buf ^= 1) {
+          const RotBuf& R = rb[buf];
+          if (is_a) {
+            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, T.entry[rd][tid], T.next[rd][tid], tr, tk, half, jrot);
+          } else if (is_q) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const zc sw = R.sw[qt];
+              const double c = R.c[qt];
+              const int k = qk + 16 * u, p = level_p(h, qt), q = level_q(h, r, qt);
+              const zc xp = Q[k][p], xq = Q[k][q];
+              Q[k][p] = zsub(zscale(xp, c), zmul(zconj(sw), xq));
+              Q[k][q] = zadd(zmul(sw, xp), zscale(xq, c));
+            }
           }
-          rb[cur].c[tid] = c;
-          rb[cur].sw[tid] = sw;
-          rb[cur].pq[tid] = pp | qq << 8 | rot << 16;
+          __syncthreads();
         }
-      } else if (g > 0 && s_round[cur ^ 1]) {
-        const int u = tid - 64;  // 448 threads for the 512 groups
-        q_rotate(Q, rb[cur ^ 1], u);
-        if (u < JC * JC / 2 - (kRoundThreads - 64)) q_rotate(Q, rb[cur ^ 1], u + (kRoundThreads - 64));
+      if (is_q) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f[u] = Q[qk + 16 * u][qt];
+          s[u] = Q[qk + 16 * u][qt + 16];
+        }
       }
-      __syncthreads();
-      if (!s_round[cur]) continue;
-      if (ob < kOffBlocks) {
-        const RotBuf& R = rb[cur];
-        const int pqr = R.pq[tr], pqk = R.pq[tk];
-        const double cr = R.c[tr], ck = R.c[tk];
-        const zc swr = R.sw[tr], swk = R.sw[tk];
-        if ((pqr | pqk) >> 16) {
-          const int pr = pqr & 255, qr = (pqr >> 8) & 255, pk = pqk & 255, qk = (pqk >> 8) & 255;
-          const int own = half ? qr : pr, oth = half ? pr : qr;
-          const zc own0 = A[own][pk], own1 = A[own][qk], oth0 = A[oth][pk], oth1 = A[oth][qk];
-          // this thread's row after the row rotation (a pair that stays put has c = 1,
-          // s w = 0: the identity): A_p <- c A_p - s w A_q ; A_q <- s conj(w) A_p + c A_q
-          const zc f = half ? zconj(swr) : zmk(-swr.x, -swr.y);
-          const zc x0 = zadd(zscale(own0, cr), zmul(f, oth0));
-          const zc x1 = zadd(zscale(own1, cr), zmul(f, oth1));
-          // then the column rotation: A_:p <- c A_:p - s conj(w) A_:q ; A_:q <- s w A_:p + c A_:q
-          const zc n0 = zsub(zscale(x0, ck), zmul(zconj(swk), x1));
-          const zc n1 = zadd(zmul(swk, x0), zscale(x1, ck));
-          A[own][pk] = n0;
-          A[own][qk] = n1;
-          A[pk][own] = zconj(n0);
-          A[qk][own] = zconj(n1);
+    }
+#pragma unroll 1
+    for (int r = 0; r < JB; ++r, buf ^= 1) {
+      const RotBuf& R = rb[buf];
+      if (is_a) {
+        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, T.entry[RW + r][tid], tid < NN ? T.next[RW + r][tid] : 0u, tr,
+                     tk, half, jrot);
+      } else if (is_q) {
+        const double c = R.c[qt];
+        const zc sw = R.sw[qt];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          // Q_:p <- c Q_:p - s conj(w) Q_:q ; Q_:q <- s w Q_:p + c Q_:q
+          const zc xp = f[u], xq = s[u];
+          f[u] = zsub(zscale(xp, c), zmul(zconj(sw), xq));
+          const zc nq = zadd(zmul(sw, xp), zscale(xq, c));
+          s[u] = zdpp<kDppRotate>(nq, nq);
         }
       }
       __syncthreads();
     }
-    if (!s_sweep[isw & 1]) break;
-    if (isw + 1 < max_sweeps) {  // would the next sweep rotate anything?
-      if (tid == 0) *s_more = 0;
-      __syncthreads();
-      for (int e = tid; e < JC * JC; e += kRoundThreads) {
-        const int pp = e % JC, qq = e / JC;
-        if (pp < qq && needs_rotation(A[pp][qq], A[pp][pp].x, A[qq][qq].x)) *s_more = 1;
+    if (is_q) {  // after 16 rounds every q is back at its lane
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        Q[qk + 16 * u][qt] = f[u];
+        Q[qk + 16 * u][qt + 16] = s[u];
       }
-      __syncthreads();
-      if (!*s_more) break;
     }
+    __syncthreads();
   }
-  __syncthreads();
-  if (g > 0 && s_round[(g - 1) & 1]) q_rotate(Q, rb[(g - 1) & 1], tid);
-  __syncthreads();
 }
 
 template <bool FULL>
 __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* __restrict__ tasks, int sweep, int round,
                                                       double tol_rel, double tol_abs, int* __restrict__ wl_count,
-                                                      int2* __restrict__ wl_items, int wl_cap, int inner_sweeps) {
+                                                      int2* __restrict__ wl_items, int wl_cap) {
   const BondTask t = tasks[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= t.P || round >= 2 * t.P - 1) return;
@@ -359,21 +305,28 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   unsigned long long* seen = t.pairseen + (size_t)lo * nblk + hi;
   if (!FULL && *seen == stamp) return;  // unchanged since it was verified orthogonal
 
-  __shared__ zc A[JC][JC + 1];
+  __shared__ zc A[JC][kInnerLd];  // the pair's Gram matrix: its upper triangle; its diagonal is in dg
+  __shared__ double dg[JC];
   // The rotation accumulator Q; until the inner solve starts, its storage holds the
-  // Gram's reduction scratch (red) and the column-norm partials (nred), which keeps
-  // the workgroup at ~35 KB of LDS: registers, not LDS, bound the workgroups per CU.
-  __shared__ zc Q[JC][JC + 1];
-  double (*red)[256] = reinterpret_cast<double (*)[256]>(&Q[0][0]);
-  double (*nred)[2][16] = reinterpret_cast<double (*)[2][16]>(reinterpret_cast<double*>(&Q[0][0]) + (kGramWaves - 1) * 256);
-  static_assert(((kGramWaves - 1) * 256 + kGramWaves * 2 * 16) * sizeof(double) <= sizeof(zc) * JC * (JC + 1),
-                "the Gram scratch must fit in Q's storage");
+  // Gram's reduction scratch (red) and the column-norm partials (nred).
+  union Scratch {
+    zc Q[JC][JC + 1];
+    struct {
+      double red[kGramWaves][512];
+      double nred[kGramWaves][2][16];
+    } g;
+  };
+  __shared__ Scratch sc;
   __shared__ RotBuf rb[2];
-  __shared__ int s_flag, s_round[2], s_sweep[2], s_more;
+  __shared__ typename std::conditional<FULL, decltype(FullTable::rounds), decltype(CrossTable::rounds)>::type table;
+  __shared__ int s_flag;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const zc* Wi = t.W + (size_t)t.R * (bi * JB);
   const zc* Wj = t.W + (size_t)t.R * (bj * JB);
+  if (tid == 0) s_flag = 0;
+  if constexpr (FULL) load_rounds(table, kFull.rounds, tid, kRoundThreads);
+  else load_rounds(table, kCross.rounds, tid, kRoundThreads);
 
   // ---- Gram: A = [Wi Wj]^H [Wi Wj]
   {
@@ -381,32 +334,33 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
     double nx, ny;
     auto gram = [&](const zc* X, const zc* Y) { gram_block(X, Y, t.R, wave, lane, gre, gim, nx, ny); };
     gram(Wi, Wj);
-    reduce_block(A, red, gre, gim, wave, lane, 0, JB, false);
-    if (FULL) {
-      gram(Wi, Wi);
-      reduce_block(A, red, gre, gim, wave, lane, 0, 0, true);
-      gram(Wj, Wj);
-      reduce_block(A, red, gre, gim, wave, lane, JB, JB, true);
-    } else {
+    if (!FULL) {
       nx += __shfl_xor(nx, 16, 64);
       nx += __shfl_xor(nx, 32, 64);
       ny += __shfl_xor(ny, 16, 64);
       ny += __shfl_xor(ny, 32, 64);
-      if (lane < 16 && wave < kGramWaves) {
-        nred[wave][0][lane] = nx;
-        nred[wave][1][lane] = ny;
+      if (lane < 16) {
+        sc.g.nred[wave][0][lane] = nx;
+        sc.g.nred[wave][1][lane] = ny;
       }
-      // within-block entries: zero (the blocks' columns are orthogonal)
-      for (int e = tid; e < 2 * JB * JB; e += kRoundThreads) {
-        const int blk = e / (JB * JB), r = (e / JB) % JB, c = e % JB;
-        if (r != c) A[blk * JB + r][blk * JB + c] = zmk(0.0, 0.0);
+      // within-block entries: zero (the blocks' columns are nearly orthogonal)
+      {
+        const int blk = tid / (JB * JB), r = (tid / JB) % JB, c = tid % JB;
+        A[blk * JB + r][blk * JB + c] = zmk(0.0, 0.0);
       }
-      __syncthreads();
+    }
+    reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, 0, JB, false);
+    if (FULL) {
+      gram(Wi, Wi);
+      reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, 0, 0, true);
+      gram(Wj, Wj);
+      reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, JB, JB, true);
+    } else {
       if (tid < JC) {
         const int side = tid / JB, col = tid % JB;
         double v = 0.0;
-        for (int w = 0; w < kGramWaves; ++w) v += nred[w][side][col];
-        A[tid][tid] = zmk(v, 0.0);
+        for (int w = 0; w < kGramWaves; ++w) v += sc.g.nred[w][side][col];
+        dg[tid] = v;
       }
       __syncthreads();
     }
@@ -418,16 +372,14 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   {
     const double fnorm = sqrt(t.result[2]);  // largest column norm
     int need = 0;
-    for (int e = tid; e < JC * JC; e += kRoundThreads) {
-      const int pp = e % JC, qq = e / JC;
+    for (int e = tid; e < (FULL ? JC * JC : JB * JB); e += kRoundThreads) {
+      const int pp = FULL ? e % JC : e % JB, qq = FULL ? e / JC : JB + e / JB;
       if (pp >= qq) continue;
       const double g2 = zabs2(A[pp][qq]);
-      const double app = fmax(A[pp][pp].x, 0.0), aqq = fmax(A[qq][qq].x, 0.0);
+      const double app = fmax(dg[pp], 0.0), aqq = fmax(dg[qq], 0.0);
       const double fl = tol_abs * fnorm * (sqrt(app) + sqrt(aqq));
       if (g2 > tol_rel * tol_rel * app * aqq && g2 > fl * fl) need = 1;
     }
-    if (tid == 0) s_flag = 0;
-    __syncthreads();
     if (need) s_flag = 1;
     __syncthreads();
     if (!s_flag) {
@@ -439,8 +391,9 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
     }
   }
 
-  // ---- eigenvectors of A -> Q, to the pair's slot; queue the pair for rotation
-  inner_jacobi(A, Q, rb, s_round, s_sweep, &s_more, tid, inner_sweeps);
+  // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
+  zc (*Q)[JC + 1] = sc.Q;
+  inner_jacobi<FULL>(A, Q, dg, rb, table, tid);
   zc* qg = t.Qg + (size_t)p * JC * JC;
   for (int e = tid; e < JC * JC; e += kRoundThreads) qg[e] = Q[e / JC][e % JC];  // qg[k JC + c] = Q[k][c]
   if (tid == 0) {
@@ -553,14 +506,13 @@ hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sw
 
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
                                double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
-                               int2* wl_items, int wl_cap, int inner_sweeps, hipStream_t st) {
-  if (inner_sweeps < 1 || inner_sweeps > kInnerSweeps) inner_sweeps = kInnerSweeps;
+                               int2* wl_items, int wl_cap, hipStream_t st) {
   if (round == 0)
     hipLaunchKernelGGL(k_jacobi_round<true>, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round,
-                       tol_rel, tol_abs, wl_count, wl_items, wl_cap, inner_sweeps);
+                       tol_rel, tol_abs, wl_count, wl_items, wl_cap);
   else
     hipLaunchKernelGGL(k_jacobi_round<false>, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round,
-                       tol_rel, tol_abs, wl_count, wl_items, wl_cap, inner_sweeps);
+                       tol_rel, tol_abs, wl_count, wl_items, wl_cap);
   return hipGetLastError();
 }
 

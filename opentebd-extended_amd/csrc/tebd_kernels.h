@@ -19,7 +19,7 @@ hipError_t launch_jacobi_begin(const BondTask* d_tasks, int ntasks, hipStream_t 
 hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sweep, int* wl_count, hipStream_t st);
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
                                double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
-                               int2* wl_items, int wl_cap, int inner_sweeps, hipStream_t st);
+                               int2* wl_items, int wl_cap, hipStream_t st);
 hipError_t launch_jacobi_rotate(const BondTask* d_tasks, int round, int max_rows_w, int max_rows_v, int* wl_count,
                                 int2* wl_items, int wl_cap, hipStream_t st);
 // The whole solve of every task without QR preconditioning and with at most two pairs
