@@ -45,6 +45,7 @@ constexpr int kMaxSweeps = 40;
 constexpr double kTolRel = 1e-13;   // relative orthogonality of converged column pairs
 constexpr double kTolAbs = 1e-13;   // rounding floor: |A_pq| <= kTolAbs ||theta|| (|w_p| + |w_q|)
 constexpr double kSlotBudget = 48.0 * (1ull << 30);  // bytes of per-bond workspace slots per context
+constexpr double kCrBudget = 4.0 * (1ull << 30);     // bytes of environments of the all-pairs density matrices
 constexpr size_t kMaxSweepGraphs = 512;  // executable Jacobi sweep graphs kept per context or lane
 constexpr int kGraphRowQuantum = 64;     // = the rotation kernel's slab height (tebd_jacobi.hip)
 // The number-conserving update's block SVDs in the batched mode: blocks of up to
@@ -110,11 +111,15 @@ struct tebd_ctx {
   double* results2 = nullptr;    // learned-rank path: per task ||theta||^2 and column norms of theta
   zc* obs_ops = nullptr;         // (L-1) x d^4 operators of tebd_expval_two_site, allocated on first use
   // all-pairs reduced density matrices (tebd_two_point_rdms), allocated on first use:
-  // environments Theta (two, chi^2 d^2), T (chi^2 d^3), three chi d chi factors, row scales,
-  // the phase, and the device copies of the pair (d^4) and site (d^2) matrices
+  // environments of cr_envs right sites (two, chi^2 d^2, and T, chi^2 d^3, each), the left
+  // factors of every chain (chi d chi), the phase, the device copies of the pair (d^4) and
+  // site (d^2) matrices, and the descriptors of a group of right sites (device and pinned)
   zc* cr_theta[2] = {nullptr, nullptr};
-  zc *cr_T = nullptr, *cr_K = nullptr, *cr_B = nullptr, *cr_A = nullptr, *cr_rho2 = nullptr, *cr_rho1 = nullptr;
-  double *cr_s = nullptr, *cr_phase = nullptr;
+  zc *cr_T = nullptr, *cr_B = nullptr, *cr_A = nullptr, *cr_rho2 = nullptr, *cr_rho1 = nullptr;
+  double* cr_phase = nullptr;
+  int cr_envs = 0;
+  unsigned char *cr_desc = nullptr, *cr_hdesc = nullptr;
+  size_t cr_desc_bytes = 0;
   zc* ident = nullptr;           // d^4 identity gate
   // rank model (learned-rank path) and the training record of the full path
   float* mlp = nullptr;          // TEBD_MLP_PARAMS on the device
@@ -1766,8 +1771,9 @@ tebd_ctx* make_lane(tebd_ctx* c, int lane, int slot0, int nslots) {
   l->cf_lam = nullptr;
   l->cf_perm = nullptr;
   l->cf_sets = 0;
-  l->cr_theta[0] = l->cr_theta[1] = l->cr_T = l->cr_K = l->cr_B = l->cr_A = l->cr_rho2 = l->cr_rho1 = nullptr;
-  l->cr_s = l->cr_phase = nullptr;
+  l->cr_theta[0] = l->cr_theta[1] = l->cr_T = l->cr_B = l->cr_A = l->cr_rho2 = l->cr_rho1 = nullptr;
+  l->cr_phase = nullptr;
+  l->cr_desc = l->cr_hdesc = nullptr;
   l->nc_theta = l->nc_vec = nullptr;   // the number-conserving update runs on the context only
   l->nc_small = nullptr;
   l->d_nc_idx = nullptr;
@@ -2085,9 +2091,9 @@ void free_all(tebd_ctx* c) {
   (void)hipFree(c->results);
   (void)hipFree(c->results2);
   (void)hipFree(c->obs_ops);
-  for (zc* p : {c->cr_theta[0], c->cr_theta[1], c->cr_T, c->cr_K, c->cr_B, c->cr_A, c->cr_rho2, c->cr_rho1})
-    (void)hipFree(p);
-  (void)hipFree(c->cr_s);
+  for (zc* p : {c->cr_theta[0], c->cr_theta[1], c->cr_T, c->cr_B, c->cr_A, c->cr_rho2, c->cr_rho1}) (void)hipFree(p);
+  (void)hipFree(c->cr_desc);
+  (void)hipHostFree(c->cr_hdesc);
   (void)hipFree(c->cr_phase);
   (void)hipFree(c->mlp);
   (void)hipFree(c->d_feat);
@@ -3189,77 +3195,132 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
   int e = ensure_state(c, false);
   if (e) return e;
   if (!rho2) return fail(c, TEBD_ERR_ARG, "two_point_rdms: null output");
-  const int d = c->d, Lc = c->chain_len, chi = c->chi_max, d2 = d * d;
+  const int d = c->d, Lc = c->chain_len, chi = c->chi_max, d2 = d * d, nch = c->nchain;
   const size_t np = (size_t)Lc * (Lc - 1) / 2, d4 = (size_t)d2 * d2;
-  if (!c->cr_T) {
-    const size_t th = (size_t)chi * chi * d2, fac = (size_t)chi * d * chi;
-    HIPCHK(c, hipMalloc(&c->cr_theta[0], sizeof(zc) * th));
-    HIPCHK(c, hipMalloc(&c->cr_theta[1], sizeof(zc) * th));
-    HIPCHK(c, hipMalloc(&c->cr_T, sizeof(zc) * th * d));
-    HIPCHK(c, hipMalloc(&c->cr_K, sizeof(zc) * fac));
-    HIPCHK(c, hipMalloc(&c->cr_B, sizeof(zc) * fac));
-    HIPCHK(c, hipMalloc(&c->cr_A, sizeof(zc) * fac));
-    HIPCHK(c, hipMalloc(&c->cr_s, sizeof(double) * chi * d));
+  const size_t th = (size_t)chi * chi * d2, fac = (size_t)chi * d * chi;
+  if (!c->cr_rho1) {
+    // every right site at once, up to the budget of environments
+    const double per = sizeof(zc) * (double)th * (2 + d);
+    c->cr_envs = (int)std::max(1.0, std::min((double)c->L, std::floor(kCrBudget / per)));
+    HIPCHK(c, hipMalloc(&c->cr_theta[0], sizeof(zc) * th * c->cr_envs));
+    HIPCHK(c, hipMalloc(&c->cr_theta[1], sizeof(zc) * th * c->cr_envs));
+    HIPCHK(c, hipMalloc(&c->cr_T, sizeof(zc) * th * d * c->cr_envs));
+    HIPCHK(c, hipMalloc(&c->cr_B, sizeof(zc) * fac * nch));
+    HIPCHK(c, hipMalloc(&c->cr_A, sizeof(zc) * fac * nch));
     HIPCHK(c, hipMalloc(&c->cr_phase, sizeof(double) * d));
-    HIPCHK(c, hipMalloc(&c->cr_rho2, sizeof(zc) * d4 * np * c->nchain));
+    HIPCHK(c, hipMalloc(&c->cr_rho2, sizeof(zc) * d4 * np * nch));
     HIPCHK(c, hipMalloc(&c->cr_rho1, sizeof(zc) * d2 * c->L));
-  }
-  if (!c->h_gemm) {
-    HIPCHK(c, hipMalloc(&c->d_gemm, sizeof(GemmTask) * c->ntask_max * kGemmRegions));
-    HIPCHK(c, hipHostMalloc(&c->h_gemm, sizeof(GemmTask) * c->ntask_max * kGemmRegions));
   }
   const double* ph = nullptr;
   if (phase) {
     HIPCHK(c, hipMemcpy(c->cr_phase, phase, sizeof(double) * d, hipMemcpyHostToDevice));
     ph = c->cr_phase;
   }
-  // one GEMM at a time; the pinned descriptors of a region are rewritten only after the
-  // stream has consumed them
-  int region = 0;
-  auto gemm = [&](const zc* A, const zc* B, zc* C, int M, int N, int K, int lda, int ldb, int ldc, int acc) {
-    if (region == 5) {
-      HIPCHK(c, hipStreamSynchronize(c->st));
-      region = 0;
-    }
-    GemmTask t = {A, B, C, M, N, K, lda, ldb, ldc, 1.0, acc};
-    return gemm_batch(c, &t, 1, region++, false);
-  };
   auto slab = [&](int s) { return c->gam + (size_t)s * c->gslab(); };
   auto lam = [&](int b) { return c->lam + (size_t)b * chi; };
-  for (int r = 0; r < c->nchain; ++r) {
-    const int base = r * Lc;
-    zc* rho2_chain = c->cr_rho2 + d4 * np * r;
-    for (int l2 = Lc - 1; l2 >= 0; --l2) {
-      const int s2 = base + l2, chl = c->chi[s2], chr = c->chi[s2 + 1];
-      // ThetaKernal of site l2 (observables_module.f90:704-730): ket factor (lambda Gamma
-      // lambda as a (chi_l d) x chi_r matrix) times its bra counterpart
-      HIPCHK(c, launch_scaled_copy(slab(s2), chl * d, c->cr_K, chl * d, chl * d, chr, lam(s2), chl, lam(s2 + 1), 1, 0,
-                                   c->st));
-      HIPCHK(c, launch_bra_kernal(slab(s2), lam(s2), lam(s2 + 1), chl, d, chr, c->cr_B, c->st));
-      int cur = 0;
-      if ((e = gemm(c->cr_K, c->cr_B, c->cr_theta[cur], chl * d, d * chl, chr, chl * d, chr, chl * d, 0))) return e;
-      HIPCHK(c, launch_rho1_trace(c->cr_theta[cur], chl, d, c->cr_rho1 + (size_t)d2 * s2, c->st));
-      for (int l1 = l2 - 1; l1 >= 0; --l1) {
-        const int s1 = base + l1, ca = c->chi[s1], cb = c->chi[s1 + 1];
-        // rows of the left site's ket Gamma scaled by lambda(a) phase(i)
-        HIPCHK(c, launch_scale_vec(lam(s1), ph, ca, d, c->cr_s, c->st));
-        // bra Gamma, conjugate-transposed with lambda(a): Gbar(eta, a + chi_a l)
-        HIPCHK(c, launch_scaled_copy(slab(s1), ca * d, c->cr_B, cb, ca * d, cb, lam(s1), ca, nullptr, 1, 1, c->st));
-        // T = Theta Gbar (ThetaNext's / TwoSiteRho's first contraction)
-        if ((e = gemm(c->cr_theta[cur], c->cr_B, c->cr_T, cb * d2, ca * d, cb, cb * d2, cb, cb * d2, 0))) return e;
-        const size_t pair = (size_t)l1 * Lc - (size_t)l1 * (l1 + 1) / 2 + (l2 - l1 - 1);
-        HIPCHK(c, launch_rho_reduce(slab(s1), c->cr_s, c->cr_T, ca, cb, d, rho2_chain + d4 * pair, c->st));
-        if (l1 == 0) break;  // no site further left: the environment is not needed
-        // ket Gamma scaled by lambda(a) phase(k), then Theta' = sum_k A_k T_k
-        HIPCHK(c, launch_scaled_copy(slab(s1), ca * d, c->cr_A, ca * d, ca * d, cb, c->cr_s, ca * d, nullptr, 1, 0,
-                                     c->st));
-        for (int k = 0; k < d; ++k)
-          if ((e = gemm(c->cr_A + (size_t)ca * k, c->cr_T + (size_t)cb * d2 * ca * k, c->cr_theta[1 - cur], ca,
-                        d2 * ca, cb, ca * d, cb, ca, k > 0)))
-            return e;
-        cur = 1 - cur;
-      }
+  // right sites (chain r, site l2), the rightmost first, in groups of cr_envs environments; a
+  // group's environments are stepped together over the left sites l1 of their chains
+  std::vector<std::pair<int, int>> all;
+  for (int l2 = Lc - 1; l2 >= 0; --l2)
+    for (int r = 0; r < nch; ++r) all.push_back({r, l2});
+  struct Step { size_t left, pair, gemm, next; int nleft, npair, max_ca, max_cb; };
+  for (size_t g0 = 0; g0 < all.size(); g0 += c->cr_envs) {
+    const int ng = (int)std::min(all.size() - g0, (size_t)c->cr_envs);
+    std::vector<CrRight> right(ng);
+    std::vector<GemmTask> first(ng);
+    std::vector<CrLeft> left;
+    std::vector<CrPair> pairs;
+    std::vector<GemmTask> gemms;  // per step: T = Theta Gbar of every pair, then A_k T_k of every pair, k < d
+    std::vector<Step> steps;
+    int max_ml = 1, max_l2 = 0;
+    size_t max_r = 1;
+    for (int q = 0; q < ng; ++q) {
+      const auto [r, l2] = all[g0 + q];
+      const int s2 = r * Lc + l2, chl = c->chi[s2], chr = c->chi[s2 + 1];
+      // K and B, which only start the environment, lie in its T
+      zc* K = c->cr_T + th * d * q;
+      right[q] = {slab(s2), lam(s2), lam(s2 + 1), chl, chr, d, K, K + fac, c->cr_theta[0] + th * q,
+                  c->cr_rho1 + (size_t)d2 * s2};
+      first[q] = {K, K + fac, right[q].theta, chl * d, d * chl, chr, chl * d, chr, chl * d, 1.0, 0};
+      max_ml = std::max(max_ml, chl * d);
+      max_r = std::max(max_r, (size_t)chl * d * chr);
+      max_l2 = std::max(max_l2, l2);
     }
+    for (int l1 = max_l2 - 1; l1 >= 0; --l1) {
+      Step st{left.size(), pairs.size(), gemms.size(), 0, 0, 0, 1, 1};
+      std::vector<GemmTask> adv;
+      for (int r = 0; r < nch; ++r) {
+        const int s1 = r * Lc + l1, ca = c->chi[s1], cb = c->chi[s1 + 1];
+        zc *A = c->cr_A + fac * r, *Gbar = c->cr_B + fac * r;
+        bool used = false;
+        for (int q = 0; q < ng; ++q) {
+          const auto [rq, l2] = all[g0 + q];
+          if (rq != r || l2 <= l1) continue;
+          used = true;
+          const int cur = (l2 - 1 - l1) & 1;  // steps taken so far
+          zc *Th = c->cr_theta[cur] + th * q, *Nx = c->cr_theta[1 - cur] + th * q, *T = c->cr_T + th * d * q;
+          const size_t pair = (size_t)l1 * Lc - (size_t)l1 * (l1 + 1) / 2 + (l2 - l1 - 1);
+          pairs.push_back({A, T, ca, cb, c->cr_rho2 + d4 * (np * r + pair)});
+          // T = Theta Gbar (ThetaNext's / TwoSiteRho's first contraction), then Theta' = sum_k A_k T_k
+          gemms.push_back({Th, Gbar, T, cb * d2, ca * d, cb, cb * d2, cb, cb * d2, 1.0, 0});
+          adv.push_back({A, T, Nx, ca, d2 * ca, cb, ca * d, cb, ca, 1.0, 0});
+        }
+        if (!used) continue;
+        left.push_back({slab(s1), lam(s1), ph, ca, cb, d, A, Gbar});
+        st.max_ca = std::max(st.max_ca, ca);
+        st.max_cb = std::max(st.max_cb, cb);
+      }
+      st.nleft = (int)(left.size() - st.left);
+      st.npair = (int)(pairs.size() - st.pair);
+      st.next = gemms.size();
+      if (l1 > 0)  // the leftmost site needs no environment beyond it
+        for (int k = 0; k < d; ++k)
+          for (const GemmTask& t : adv) {
+            GemmTask x = t;
+            x.A = t.A + (size_t)t.M * k;
+            x.B = t.B + (size_t)t.K * t.N * k;
+            x.accumulate = k > 0;
+            gemms.push_back(x);
+          }
+      steps.push_back(st);
+    }
+    // the group's descriptors in one copy
+    const size_t o1 = sizeof(CrRight) * right.size(), o2 = o1 + sizeof(GemmTask) * first.size(),
+                 o3 = o2 + sizeof(CrLeft) * left.size(), o4 = o3 + sizeof(CrPair) * pairs.size(),
+                 bytes = o4 + sizeof(GemmTask) * gemms.size();
+    if (bytes > c->cr_desc_bytes) {
+      HIPCHK(c, hipStreamSynchronize(c->st));
+      (void)hipFree(c->cr_desc);
+      (void)hipHostFree(c->cr_hdesc);
+      c->cr_desc = c->cr_hdesc = nullptr;
+      c->cr_desc_bytes = 0;
+      HIPCHK(c, hipMalloc(&c->cr_desc, bytes));
+      HIPCHK(c, hipHostMalloc(&c->cr_hdesc, bytes));
+      c->cr_desc_bytes = bytes;
+    }
+    auto put = [&](size_t off, const void* src, size_t n) { if (n) std::memcpy(c->cr_hdesc + off, src, n); };
+    put(0, right.data(), o1);
+    put(o1, first.data(), o2 - o1);
+    put(o2, left.data(), o3 - o2);
+    put(o3, pairs.data(), o4 - o3);
+    put(o4, gemms.data(), bytes - o4);
+    HIPCHK(c, hipMemcpyAsync(c->cr_desc, c->cr_hdesc, bytes, hipMemcpyHostToDevice, c->st));
+    const CrRight* dr = reinterpret_cast<CrRight*>(c->cr_desc);
+    const CrLeft* dl = reinterpret_cast<CrLeft*>(c->cr_desc + o2);
+    const CrPair* dp = reinterpret_cast<CrPair*>(c->cr_desc + o3);
+    const GemmTask* dg = reinterpret_cast<GemmTask*>(c->cr_desc + o4);
+    HIPCHK(c, launch_cr_kernal(dr, ng, max_r, c->st));
+    HIPCHK(c, tuned_zgemm(c, reinterpret_cast<GemmTask*>(c->cr_desc + o1), ng, max_ml, max_ml, false));
+    HIPCHK(c, launch_rho1_trace(dr, ng, d, c->st));
+    for (const Step& st : steps) {
+      HIPCHK(c, launch_cr_left(dl + st.left, st.nleft, (size_t)st.max_ca * d * st.max_cb, c->st));
+      HIPCHK(c, tuned_zgemm(c, dg + st.gemm, st.npair, st.max_cb * d2, st.max_ca * d, false));
+      HIPCHK(c, launch_rho_reduce(dp + st.pair, st.npair, d, c->st));
+      if (&st == &steps.back()) break;
+      for (int k = 0; k < d; ++k)
+        HIPCHK(c, tuned_zgemm(c, dg + st.next + (size_t)st.npair * k, st.npair, st.max_ca, st.max_ca * d2, false));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->st));  // the descriptors are rewritten by the next group
   }
   HIPCHK(c, hipStreamSynchronize(c->st));
   HIPCHK(c, hipMemcpy(rho2, c->cr_rho2, sizeof(zc) * d4 * np * c->nchain, hipMemcpyDeviceToHost));

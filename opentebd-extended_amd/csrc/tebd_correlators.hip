@@ -1,125 +1,159 @@
 // Kernels of the all-pairs two-site reduced density matrices (TwoSiteExpVal and
 // EvaluateMeasures, observables_module.f90:836-883,2286-2526, built from ThetaKernal,
-// ThetaNext and TwoSiteRho, :704-832).  The host (tebd_capi.cpp) carries, for a right
+// ThetaNext and TwoSiteRho, :704-832).  The host (tebd_capi.cpp) carries, for every right
 // site l2, the environment Theta(a, i, j, b) of l2 with the sites between absorbed, and
-// steps it one site l1 to the left with two GEMMs; these kernels do the parts that are
-// not GEMMs: the per-row scales lambda(a) phase(k) and the contraction of the left site
-// into the two-site density matrix.
+// steps all of them over one left site l1 at a time with batched GEMMs; these kernels do
+// the parts that are not GEMMs, for all right sites (k_cr_kernal, k_rho1_trace,
+// k_rho_reduce) or all chains (k_cr_left) in one launch.
+//
+// One right site at a time, a table was a sequence of ten short launches per pair of sites:
+// 27.8 ms for 276 pairs of a Fermi-Hubbard chain of 24 sites at chi = 64, whose products take
+// 1.5 ms at the GEMM's rate; stepped together, 3.8 ms (k_rho_reduce 47 us for 23 pairs).
 #include "tebd_device.h"
 #include "tebd_kernels.h"
 
 namespace {
 
-// s[a + chi k] = lambda[a] * phase[k] (phase null: 1), a < chi, k < d
-__global__ void k_scale_vec(const double* __restrict__ lambda, const double* __restrict__ phase, int chi, int d,
-                            double* __restrict__ s) {
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < chi * d; e += gridDim.x * blockDim.x) {
-    const int a = e % chi, k = e / chi;
-    s[e] = lambda[a] * (phase ? phase[k] : 1.0);
+// ThetaKernal's two factors (observables_module.f90:704-730) of a right site: the ket factor
+// K((a, i), e) = lambda_l(a) G(a, i, e) lambda_r(e), a (chi_l d) x chi_r matrix, and the bra factor
+// as a chi_r x (d chi_l) matrix with columns j + d b: B(e, j + d b) = conj(G(b, j, e)) lambda_l(b)
+// lambda_r(e); Theta = K B has Theta(a, i, j, b) at a + chi_l (i + d (j + d b)).
+__global__ void k_cr_kernal(const CrRight* __restrict__ sites) {
+  const CrRight t = sites[blockIdx.y];
+  const int m = t.chil * t.d;
+  const size_t n = (size_t)m * t.chir;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
+    const int row = (int)(e % m), eta = (int)(e / m);
+    const int a = row % t.chil, i = row / t.chil;
+    const zc g = t.G[e];
+    const double w = t.ll[a] * t.lr[eta];
+    t.K[e] = zmk(g.x * w, g.y * w);
+    t.B[eta + (size_t)t.chir * (i + (size_t)t.d * a)] = zmk(g.x * w, -g.y * w);
   }
 }
 
-// The bra factor of ThetaKernal (observables_module.f90:704-730) as a chi_r x (d chi_l) matrix
-// with columns j + d b: out[e + chi_r (j + d b)] = conj(G(b, j, e)) lambda1[b] lambda2[e], so
-// that Theta = K K^H-like product (ket factor) x out has Theta(a, i, j, b) at
-// a + chi_l (i + d (j + d b)).
-__global__ void k_bra_kernal(const zc* __restrict__ G, const double* __restrict__ lam1, const double* __restrict__ lam2,
-                             int chi_l, int d, int chi_r, zc* __restrict__ out) {
-  const size_t n = (size_t)chi_r * d * chi_l;
+// The factors of a left site: A((a, i), b) = lambda(a) phase(i) G(a, i, b) (phase null: 1) for the
+// ket, and the bra's conjugate transpose Gbar(b, a + chi_a l) = conj(G(a, l, b)) lambda(a).
+__global__ void k_cr_left(const CrLeft* __restrict__ sites) {
+  const CrLeft t = sites[blockIdx.y];
+  const int m = t.chia * t.d;
+  const size_t n = (size_t)m * t.chib;
   for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
-    const int eta = (int)(e % chi_r);
-    const size_t rest = e / chi_r;
-    const int j = (int)(rest % d), b = (int)(rest / d);
-    const zc g = G[b + (size_t)chi_l * (j + (size_t)d * eta)];
-    const double w = lam1[b] * lam2[eta];
-    out[e] = zmk(g.x * w, -g.y * w);
+    const int row = (int)(e % m), b = (int)(e / m);
+    const zc g = t.G[e];
+    const double w = t.lam[row % t.chia], p = t.phase ? w * t.phase[row / t.chia] : w;
+    t.A[e] = zmk(g.x * p, g.y * p);
+    t.Gbar[b + (size_t)t.chib * row] = zmk(g.x * w, -g.y * w);
   }
 }
 
 // TwoSiteRho's final contraction (observables_module.f90:815-826):
-//   rho[(i d + j) + d^2 (l d + k)] = sum_{a < chi_a, b < chi_b} s[a + chi_a i] G(a, i, b) T(b, j, k; a + chi_a l)
-// G: the left site's Gamma, element a + chi_a (i + d b); T: (chi_b d^2) x (chi_a d), element
-// b + chi_b (j + d k) + chi_b d^2 (a + chi_a l) (the environment with the left site's bra
-// Gamma absorbed).  One workgroup per entry of rho.
-__global__ __launch_bounds__(256) void k_rho_reduce(const zc* __restrict__ G, const double* __restrict__ s,
-                                                    const zc* __restrict__ T, int chi_a, int chi_b, int d,
-                                                    zc* __restrict__ rho) {
-  const int e = blockIdx.x;
-  const int d2 = d * d;
-  const int row = e % d2, col = e / d2;
-  const int i = row / d, j = row % d, l = col / d, k = col % d;
-  const size_t tcol0 = (size_t)chi_b * d2 * ((size_t)chi_a * l);
-  double re = 0.0, im = 0.0;
-  const int n = chi_a * chi_b;
-  for (int q = threadIdx.x; q < n; q += 256) {
-    const int a = q % chi_a, b = q / chi_a;
-    const zc g = G[a + (size_t)chi_a * (i + (size_t)d * b)];
-    const zc t = T[b + (size_t)chi_b * (j + (size_t)d * k) + tcol0 + (size_t)chi_b * d2 * a];
-    const double w = s[a + (size_t)chi_a * i];
-    re += w * (g.x * t.x - g.y * t.y);
-    im += w * (g.x * t.y + g.y * t.x);
-  }
-  __shared__ double sr[256], si[256];
-  sr[threadIdx.x] = re;
-  si[threadIdx.x] = im;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      sr[threadIdx.x] += sr[threadIdx.x + st];
-      si[threadIdx.x] += si[threadIdx.x + st];
+//   rho[(i d + j) + d^2 (l d + k)] = sum_{a < chi_a, b < chi_b} A(a, i, b) T(b, j, k; a + chi_a l)
+// A: the left site's scaled ket Gamma; T: (chi_b d^2) x (chi_a d), element b + chi_b (j + d k) +
+// chi_b d^2 (a + chi_a l) (the environment with the left site's bra Gamma absorbed).  One
+// workgroup per (j, k, l) and pair forms the d entries i from one pass over its part of T, the
+// bulk of the bytes: lanes run over b, where T is contiguous, and each wave takes a range of a.
+template <int D>
+__global__ __launch_bounds__(256) void k_rho_reduce(const CrPair* __restrict__ pairs) {
+  const CrPair t = pairs[blockIdx.y];
+  const int jk = blockIdx.x % (D * D), l = blockIdx.x / (D * D);
+  const int j = jk % D, k = jk / D;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int chi_a = t.chia, chi_b = t.chib;
+  const int part = (chi_a + 3) / 4, a0 = wave * part, a1 = min(chi_a, a0 + part);
+  const zc* T = t.T + (size_t)chi_b * jk + (size_t)chi_b * D * D * ((size_t)chi_a * l);
+  double re[D], im[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) re[i] = im[i] = 0.0;
+  for (int b = lane; b < chi_b; b += 64) {
+    const zc* A = t.A + (size_t)chi_a * D * b;
+    for (int a = a0; a < a1; ++a) {
+      const zc x = T[b + (size_t)chi_b * D * D * a];
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        const zc g = A[a + (size_t)chi_a * i];
+        re[i] += g.x * x.x - g.y * x.y;
+        im[i] += g.x * x.y + g.y * x.x;
+      }
     }
-    __syncthreads();
   }
-  if (threadIdx.x == 0) rho[e] = zmk(sr[0], si[0]);
+  __shared__ double red[4][2 * D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    const double sr = wave_sum(re[i]), si = wave_sum(im[i]);
+    if (lane == 0) {
+      red[wave][2 * i] = sr;
+      red[wave][2 * i + 1] = si;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const int i = threadIdx.x;
+    double sr = 0.0, si = 0.0;
+    for (int w = 0; w < 4; ++w) {
+      sr += red[w][2 * i];
+      si += red[w][2 * i + 1];
+    }
+    t.rho[(i * D + j) + D * D * (l * D + k)] = zmk(sr, si);
+  }
 }
 
 // The one-site density matrix as the trace of ThetaKernal over its bond index
 // (FormSingleSiteRho, observables_module.f90:95-117): rho[i + d j] = sum_a Theta(a, i, j, a),
 // Theta element a + chi (i + d (j + d b)).
-__global__ __launch_bounds__(256) void k_rho1_trace(const zc* __restrict__ Theta, int chi, int d, zc* __restrict__ rho) {
-  const int i = blockIdx.x % d, j = blockIdx.x / d;
+__global__ __launch_bounds__(256) void k_rho1_trace(const CrRight* __restrict__ sites) {
+  const CrRight t = sites[blockIdx.y];
+  const int d = t.d, chi = t.chil, i = blockIdx.x % d, j = blockIdx.x / d;
   double re = 0.0, im = 0.0;
   for (int a = threadIdx.x; a < chi; a += 256) {
-    const zc t = Theta[a + (size_t)chi * (i + (size_t)d * (j + (size_t)d * a))];
-    re += t.x;
-    im += t.y;
+    const zc x = t.theta[a + (size_t)chi * (i + (size_t)d * (j + (size_t)d * a))];
+    re += x.x;
+    im += x.y;
   }
-  __shared__ double sr[256], si[256];
-  sr[threadIdx.x] = re;
-  si[threadIdx.x] = im;
+  __shared__ double red[4][2];
+  re = wave_sum(re);
+  im = wave_sum(im);
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6][0] = re;
+    red[threadIdx.x >> 6][1] = im;
+  }
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      sr[threadIdx.x] += sr[threadIdx.x + st];
-      si[threadIdx.x] += si[threadIdx.x + st];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) rho[blockIdx.x] = zmk(sr[0], si[0]);
+  if (threadIdx.x == 0)
+    t.rho1[blockIdx.x] = zmk(red[0][0] + red[1][0] + red[2][0] + red[3][0], red[0][1] + red[1][1] + red[2][1] + red[3][1]);
+}
+
+int blocks_for(size_t n) {
+  const size_t b = (n + 255) / 256;
+  return (int)(b < 1 ? 1 : (b < 1024 ? b : 1024));
 }
 
 }  // namespace
 
-hipError_t launch_scale_vec(const double* lambda, const double* phase, int chi, int d, double* s, hipStream_t st) {
-  hipLaunchKernelGGL(k_scale_vec, dim3((chi * d + 255) / 256), dim3(256), 0, st, lambda, phase, chi, d, s);
+hipError_t launch_cr_kernal(const CrRight* d_sites, int n, size_t max_elems, hipStream_t st) {
+  hipLaunchKernelGGL(k_cr_kernal, dim3(blocks_for(max_elems), n), dim3(256), 0, st, d_sites);
   return hipGetLastError();
 }
 
-hipError_t launch_bra_kernal(const zc* G, const double* lam1, const double* lam2, int chi_l, int d, int chi_r, zc* out,
-                             hipStream_t st) {
-  const size_t n = (size_t)chi_r * d * chi_l;
-  const int blocks = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
-  hipLaunchKernelGGL(k_bra_kernal, dim3(blocks), dim3(256), 0, st, G, lam1, lam2, chi_l, d, chi_r, out);
+hipError_t launch_cr_left(const CrLeft* d_sites, int n, size_t max_elems, hipStream_t st) {
+  hipLaunchKernelGGL(k_cr_left, dim3(blocks_for(max_elems), n), dim3(256), 0, st, d_sites);
   return hipGetLastError();
 }
 
-hipError_t launch_rho_reduce(const zc* G, const double* s, const zc* T, int chi_a, int chi_b, int d, zc* rho,
-                             hipStream_t st) {
-  hipLaunchKernelGGL(k_rho_reduce, dim3(d * d * d * d), dim3(256), 0, st, G, s, T, chi_a, chi_b, d, rho);
+hipError_t launch_rho_reduce(const CrPair* d_pairs, int n, int d, hipStream_t st) {
+  const dim3 grid(d * d * d, n);
+  switch (d) {
+    case 2: hipLaunchKernelGGL(k_rho_reduce<2>, grid, dim3(256), 0, st, d_pairs); break;
+    case 3: hipLaunchKernelGGL(k_rho_reduce<3>, grid, dim3(256), 0, st, d_pairs); break;
+    case 4: hipLaunchKernelGGL(k_rho_reduce<4>, grid, dim3(256), 0, st, d_pairs); break;
+    case 5: hipLaunchKernelGGL(k_rho_reduce<5>, grid, dim3(256), 0, st, d_pairs); break;
+    case 6: hipLaunchKernelGGL(k_rho_reduce<6>, grid, dim3(256), 0, st, d_pairs); break;
+    case 8: hipLaunchKernelGGL(k_rho_reduce<8>, grid, dim3(256), 0, st, d_pairs); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_rho1_trace(const zc* Theta, int chi, int d, zc* rho, hipStream_t st) {
-  hipLaunchKernelGGL(k_rho1_trace, dim3(d * d), dim3(256), 0, st, Theta, chi, d, rho);
+hipError_t launch_rho1_trace(const CrRight* d_sites, int n, int d, hipStream_t st) {
+  hipLaunchKernelGGL(k_rho1_trace, dim3(d * d, n), dim3(256), 0, st, d_sites);
   return hipGetLastError();
 }

@@ -46,6 +46,26 @@ struct NcBlock {
   zc* V;             // trv x min(lgt, trv): right singular vectors
 };
 
+// All-pairs density matrices: a right site (its environment starts as Theta = K B), the left
+// site a chain's environments are stepped over, and one pair of the table.
+struct CrRight {
+  const zc* G;
+  const double *ll, *lr;
+  int chil, chir, d;
+  zc *K, *B, *theta, *rho1;
+};
+struct CrLeft {
+  const zc* G;
+  const double *lam, *phase;
+  int chia, chib, d;
+  zc *A, *Gbar;
+};
+struct CrPair {
+  const zc *A, *T;
+  int chia, chib;
+  zc* rho;
+};
+
 // Workspace of the split-operand theta (one slot per task of a batch): the int8 slices of
 // A = Gamma_l lambda_c (rows (a, k) -> a d + k) and of B = Gamma_r (columns (l, b) ->
 // b d + l), plane (2 s + part) of `rows` rows x `pitch` bytes each (pitch: the middle
