@@ -109,7 +109,12 @@ struct tebd_ctx {
   int wl_cap = 0;
   double* results = nullptr;
   double* results2 = nullptr;    // learned-rank path: per task ||theta||^2 and column norms of theta
-  zc* obs_ops = nullptr;         // (L-1) x d^4 operators of tebd_expval_two_site, allocated on first use
+  // tebd_expval_two_site, allocated on first use: the (L-1) x d^4 operators, the values, the
+  // descriptors and the partial sums of a batch of bonds
+  zc* obs_ops = nullptr;
+  zc *obs_out = nullptr, *obs_part = nullptr;
+  BondTask *d_obs = nullptr, *h_obs = nullptr;
+  int obs_batch = 0;
   // all-pairs reduced density matrices (tebd_two_point_rdms), allocated on first use:
   // environments of cr_envs right sites (two, chi^2 d^2, and T, chi^2 d^3, each), the left
   // factors of every chain (chi d chi), the phase, the device copies of the pair (d^4) and
@@ -120,7 +125,6 @@ struct tebd_ctx {
   int cr_envs = 0;
   unsigned char *cr_desc = nullptr, *cr_hdesc = nullptr;
   size_t cr_desc_bytes = 0;
-  zc* ident = nullptr;           // d^4 identity gate
   // rank model (learned-rank path) and the training record of the full path
   float* mlp = nullptr;          // TEBD_MLP_PARAMS on the device
   bool have_model = false;
@@ -2091,6 +2095,10 @@ void free_all(tebd_ctx* c) {
   (void)hipFree(c->results);
   (void)hipFree(c->results2);
   (void)hipFree(c->obs_ops);
+  (void)hipFree(c->obs_out);
+  (void)hipFree(c->obs_part);
+  (void)hipFree(c->d_obs);
+  (void)hipHostFree(c->h_obs);
   for (zc* p : {c->cr_theta[0], c->cr_theta[1], c->cr_T, c->cr_B, c->cr_A, c->cr_rho2, c->cr_rho1}) (void)hipFree(p);
   (void)hipFree(c->cr_desc);
   (void)hipHostFree(c->cr_hdesc);
@@ -2100,7 +2108,6 @@ void free_all(tebd_ctx* c) {
   (void)hipFree(c->d_pred);
   (void)hipHostFree(c->h_feat);
   (void)hipHostFree(c->h_pred);
-  (void)hipFree(c->ident);
   (void)hipFree(c->d_tasks);
   (void)hipFree(c->cf);
   (void)hipFree(c->cf_s);
@@ -2786,24 +2793,26 @@ int tebd_expval_two_site(tebd_ctx* c, const double* ops, double* out) {
   int e = ensure_state(c, false);
   if (e) return e;
   if (!ops || !out) return fail(c, TEBD_ERR_ARG, "expval_two_site: null operator or output");
-  const int L = c->L, d = c->d, nt = c->ntask_max, d2 = d * d;
-  if (!c->obs_ops) {
+  const int L = c->L, d = c->d;
+  if (!c->h_obs) {
+    // every bond at once, up to 64 MiB of partial sums
+    const double tiles = (double)expval_tiles(d, c->chi_max);
+    const int nb = (int)std::max(1.0, std::min({(double)(L - 1), 32768.0, std::floor(double(64 << 20) / (sizeof(zc) * tiles))}));
     HIPCHK(c, hipMalloc(&c->obs_ops, sizeof(zc) * c->d4() * (L - 1)));
-    HIPCHK(c, hipMalloc(&c->ident, sizeof(zc) * c->d4()));
-    std::vector<zc> id(c->d4());
-    for (int r = 0; r < d2; ++r)
-      for (int q = 0; q < d2; ++q) id[r + (size_t)d2 * q] = zc{r == q ? 1.0 : 0.0, 0.0};
-    HIPCHK(c, hipMemcpy(c->ident, id.data(), sizeof(zc) * c->d4(), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMalloc(&c->obs_out, sizeof(zc) * (L - 1)));
+    HIPCHK(c, hipMalloc(&c->obs_part, sizeof(zc) * (size_t)tiles * nb));
+    HIPCHK(c, hipMalloc(&c->d_obs, sizeof(BondTask) * nb));
+    HIPCHK(c, hipHostMalloc(&c->h_obs, sizeof(BondTask) * nb));
+    c->obs_batch = nb;
   }
   HIPCHK(c, hipMemcpyAsync(c->obs_ops, ops, sizeof(zc) * c->d4() * (L - 1), hipMemcpyHostToDevice, c->st));
-  BondTask *S0 = c->h_tasks, *S1 = S0 + nt;
-  BondTask *D0 = c->d_tasks, *D1 = D0 + nt;
-  for (int b0 = 0; b0 < L - 1; b0 += nt) {
-    const int nb = std::min(nt, L - 1 - b0);
+  for (int b0 = 0; b0 < L - 1; b0 += c->obs_batch) {
+    const int nb = std::min(c->obs_batch, L - 1 - b0);
+    if (b0 > 0) HIPCHK(c, hipStreamSynchronize(c->st));  // the descriptors are rewritten
     int max_chil = 1, max_chir = 1;
     for (int i = 0; i < nb; ++i) {
       const int link = b0 + i;
-      BondTask& t = S0[i];
+      BondTask& t = c->h_obs[i];
       std::memset(&t, 0, sizeof(t));
       t.chil = c->chi[link]; t.chic = c->chi[link + 1]; t.chir = c->chi[link + 2]; t.d = d;
       t.gl = c->gam + (size_t)link * c->gslab();
@@ -2811,24 +2820,15 @@ int tebd_expval_two_site(tebd_ctx* c, const double* ops, double* out) {
       t.ll = c->lam + (size_t)link * c->chi_max;
       t.lc = c->lam + (size_t)(link + 1) * c->chi_max;
       t.lr = c->lam + (size_t)(link + 2) * c->chi_max;
-      t.R = d * t.chil;
-      t.C = d * t.chir;
-      t.gate = c->ident;
-      t.W = c->W + (size_t)i * c->Rmax * c->Cpmax;
-      S1[i] = t;
-      S1[i].gate = c->obs_ops + (size_t)link * c->d4();
-      S1[i].W = c->V + (size_t)i * c->Cpmax * c->Cpmax;
+      t.gate = c->obs_ops + (size_t)link * c->d4();
       max_chil = std::max(max_chil, t.chil);
       max_chir = std::max(max_chir, t.chir);
     }
-    HIPCHK(c, hipMemcpyAsync(D0, S0, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(D1, S1, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, launch_theta_gate(D0, nb, d, max_chil, max_chir, c->st));
-    HIPCHK(c, launch_theta_gate(D1, nb, d, max_chil, max_chir, c->st));
-    HIPCHK(c, launch_zdotc(D0, D1, nb, c->results, c->st));
-    HIPCHK(c, hipMemcpyAsync(out + 2 * b0, c->results, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    HIPCHK(c, hipMemcpyAsync(c->d_obs, c->h_obs, sizeof(BondTask) * nb, hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, launch_expval(c->d_obs, nb, d, max_chil, max_chir, c->obs_part, c->obs_out + b0, c->st));
   }
+  HIPCHK(c, hipMemcpyAsync(out, c->obs_out, sizeof(zc) * (L - 1), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, hipStreamSynchronize(c->st));
   return TEBD_OK;
 }
 

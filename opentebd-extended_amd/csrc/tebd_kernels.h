@@ -1,10 +1,9 @@
 // Host-side launchers of the gfx950 kernels (tebd_kernels.hip, tebd_theta_mixed.hip, tebd_jacobi.hip, tebd_qrp.hip,
-// tebd_sketch.hip, tebd_canonical.hip, tebd_observables.hip, tebd_mlp.hip).
+// tebd_sketch.hip, tebd_canonical.hip, tebd_mlp.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include "tebd_device.h"
 
-hipError_t launch_theta_gate(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir, hipStream_t st);
 hipError_t launch_theta_gate_mfma(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir,
                                   hipStream_t st);
 hipError_t launch_theta_gate_mixed(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir,
@@ -33,7 +32,11 @@ hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int
 hipError_t launch_qrp_build_x(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_qrp_vectors(const BondTask* d_tasks, int ntasks, int max_k, int max_r, hipStream_t st);
 hipError_t launch_qrp_form_q(const BondTask* d_tasks, int ntasks, int max_r, hipStream_t st);
-hipError_t launch_zdotc(const BondTask* d_a, const BondTask* d_b, int ntasks, double* d_out, hipStream_t st);
+// <theta| O |theta> of every task (its gate the operator O): d_part holds expval_tiles(d, largest
+// bond dimension) entries per task.
+size_t expval_tiles(int d, int chi);
+hipError_t launch_expval(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir, zc* d_part, zc* d_out,
+                         hipStream_t st);
 hipError_t launch_finalize(const BondTask* d_tasks, int ntasks, int max_cpad, double cutoff, hipStream_t st);
 hipError_t launch_mlp_features(const BondTask* d_tasks, int ntasks, float* d_X, hipStream_t st);
 hipError_t launch_mlp_predict(const float* d_params, const float* d_X, int n, float* d_out, hipStream_t st);

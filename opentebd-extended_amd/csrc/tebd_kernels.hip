@@ -1,6 +1,6 @@
 // gfx950 kernels of the two-site update (FP64).
 //
-//   k_theta_gate   FormTheta + ThetaOperation_c (local_operations_module.f90:184-211,248-280)
+//   k_theta_gate_mfma  FormTheta + ThetaOperation_c (local_operations_module.f90:184-211,248-280)
 //                  fused: theta'(a,i,j,b) = ll(a) lr(b) sum_kl U(ij,kl) sum_g Gl(a,k,g) lc(g) Gr(g,l,b)
 //                  written straight into the SVD work matrix W (theta, or theta^dagger when
 //                  the bond has more columns than rows).
@@ -18,113 +18,9 @@ namespace {
 // ---------------------------------------------------------------------------
 // theta + gate
 // ---------------------------------------------------------------------------
-constexpr int KC = 16;  // gamma (contraction) chunk staged in LDS
-
-template <int D>
-struct ThetaCfg {
-  static constexpr int BA = (D <= 5) ? 16 : 8;  // alpha block == beta block
-  static constexpr int TR = BA * D;             // tile rows == tile cols: (k, alpha) pairs
-  static constexpr int MT = TR / 16;            // per-thread micro tile edge
-};
-
-template <int D>
-__global__ __launch_bounds__(256) void k_theta_gate(const BondTask* __restrict__ tasks) {
-  using Cfg = ThetaCfg<D>;
-  constexpr int BA = Cfg::BA, TR = Cfg::TR, MT = Cfg::MT, D2 = D * D;
-  const BondTask t = tasks[blockIdx.z];
-  const int a0 = blockIdx.x * BA, b0 = blockIdx.y * BA;
-  if (a0 >= t.chil || b0 >= t.chir) return;
-
-  constexpr int AB_ELEMS = 2 * KC * (TR + 1);
-  constexpr int T_ELEMS = TR * (TR + 1);
-  constexpr int SM_ELEMS = AB_ELEMS > T_ELEMS ? AB_ELEMS : T_ELEMS;
-  __shared__ zc sm[SM_ELEMS];
-  __shared__ zc sgate[D2 * D2];
-  zc* As = sm;                     // [KC][TR+1]  A(r, g) = Gl(a,k,g) lc(g), r = k*BA + a_local
-  zc* Bs = sm + KC * (TR + 1);     // [KC][TR+1]  B(g, c) = Gr(g,l,b),       c = l*BA + b_local
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-
-  for (int e = tid; e < D2 * D2; e += 256) sgate[e] = t.gate[e];
-
-  zc acc[MT][MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = zmk(0.0, 0.0);
-
-  const int chil = t.chil, chic = t.chic, chir = t.chir;
-  for (int g0 = 0; g0 < chic; g0 += KC) {
-    // A chunk: r fastest (contiguous alpha within one k)
-    for (int e = tid; e < KC * TR; e += 256) {
-      const int r = e % TR, g = e / TR;
-      const int k = r / BA, a = a0 + (r % BA), gg = g0 + g;
-      zc v = zmk(0.0, 0.0);
-      if (a < chil && gg < chic) v = zscale(t.gl[a + (size_t)chil * (k + (size_t)D * gg)], t.lc[gg]);
-      As[g * (TR + 1) + r] = v;
-    }
-    // B chunk: g fastest (contiguous gamma)
-    for (int e = tid; e < KC * TR; e += 256) {
-      const int g = e % KC, c = e / KC;
-      const int l = c / BA, b = b0 + (c % BA), gg = g0 + g;
-      zc v = zmk(0.0, 0.0);
-      if (b < chir && gg < chic) v = t.gr[gg + (size_t)chic * (l + (size_t)D * b)];
-      Bs[g * (TR + 1) + c] = v;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int g = 0; g < KC; ++g) {
-      zc av[MT], bv[MT];
-#pragma unroll
-      for (int i = 0; i < MT; ++i) av[i] = As[g * (TR + 1) + ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < MT; ++j) bv[j] = Bs[g * (TR + 1) + tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) zfma(acc[i][j], av[i], bv[j]);
-    }
-    __syncthreads();
-  }
-  // stage T(r, c) in LDS for the gate
-  zc* T = sm;
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) T[(ty + 16 * i) * (TR + 1) + tx + 16 * j] = acc[i][j];
-  __syncthreads();
-
-  // gate: one (alpha, beta) pair per thread
-  for (int pr = tid; pr < BA * BA; pr += 256) {
-    int al, bl;
-    if (!t.transposed) { al = pr % BA; bl = pr / BA; } else { bl = pr % BA; al = pr / BA; }
-    const int a = a0 + al, b = b0 + bl;
-    if (a >= chil || b >= chir) continue;
-    zc x[D2];
-#pragma unroll
-    for (int k = 0; k < D; ++k)
-#pragma unroll
-      for (int l = 0; l < D; ++l) x[k * D + l] = T[(k * BA + al) * (TR + 1) + l * BA + bl];
-    const double sc = t.ll[a] * t.lr[b];
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        zc o = zmk(0.0, 0.0);
-#pragma unroll
-        for (int kl = 0; kl < D2; ++kl) zfma(o, sgate[(i * D + j) + D2 * kl], x[kl]);
-        o = zscale(o, sc);
-        const size_t row = (size_t)i * chil + a;  // theta row (i, alpha)
-        const size_t col = (size_t)j * chir + b;  // theta col (j, beta)
-        if (!t.transposed) t.W[row + (size_t)t.R * col] = o;
-        else t.W[col + (size_t)t.R * row] = zconj(o);
-      }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// theta + gate on the FP64 matrix cores (v_mfma_f64_16x16x4f64).  Same tile as
-// k_theta_gate: BA alphas x BA betas, rows (k, alpha) and columns (l, beta) of the
+// theta + gate on the FP64 matrix cores (v_mfma_f64_16x16x4f64).  One workgroup per tile
+// of BA alphas x BA betas, rows (k, alpha) and columns (l, beta) of the
 // pre-gate theta, TR = BA d.  Stage 1 accumulates the (TR/16)^2 blocks of 16 x 16 over
 // the middle bond (4 waves, blocks dealt round-robin); stage 2 applies the gate to the
 // BA^2 (alpha, beta) pairs as one (d^2 x d^2) x (d^2 x BA^2) complex product.
@@ -164,8 +60,14 @@ struct MfmaThetaCfg {
   static_assert((KM * TR) % 256 == 0, "theta chunks are staged 256 elements at a time");
 };
 
-template <int D>
-__global__ __launch_bounds__(256) void k_theta_gate_mfma(const BondTask* __restrict__ tasks) {
+// With EXPVAL (TwoSiteRho / TotalEnergy, observables_module.f90:704-832,1432-1466) the gate is an
+// operator O and nothing but the tile's part of <theta| O |theta> = sum conj(theta) (O theta) is
+// kept: theta never leaves the chip.  Partial sums go to part[task][tile], summed in tile order
+// by k_expval_sum.  Writing theta and O theta out and reading both back took 19 ms for the 127
+// bonds of a Fermi-Hubbard chain at chi = 256, with the values summed by one workgroup per
+// bond; this form takes 8 ms.
+template <int D, bool EXPVAL>
+__global__ __launch_bounds__(256) void k_theta_gate_mfma(const BondTask* __restrict__ tasks, zc* __restrict__ part) {
   using C = MfmaThetaCfg<D>;
   constexpr int BA = C::BA, TR = C::TR, NB1 = C::NB1, NBW = C::NBW, D2 = C::D2;
   constexpr int MP = C::MP, KP = C::KP, NP = C::NP, LDT = C::LDT, KM = C::KM;
@@ -253,7 +155,8 @@ __global__ __launch_bounds__(256) void k_theta_gate_mfma(const BondTask* __restr
   }
   __syncthreads();
 
-  const bool tr = t.transposed != 0;
+  const bool tr = !EXPVAL && t.transposed != 0;
+  double sre = 0.0, sim = 0.0;
   for (int pb = wave; pb < NP / 16; pb += 4) {
     const int p = pb * 16 + lr;
     const int al = tr ? p / BA : p % BA;
@@ -270,7 +173,18 @@ __global__ __launch_bounds__(256) void k_theta_gate_mfma(const BondTask* __restr
         const zc x = kl < D2 ? T[((kl / D) * BA + al) * LDT + (kl % D) * BA + bl] : zmk(0.0, 0.0);
         zmfma(sU[(mb * 16 + lr) * KP + kl], x, ore, oim);
       }
-      if (in) {
+      if constexpr (EXPVAL) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int ij = mb * 16 + lk + 4 * g;
+          if (ij < D2) {
+            const zc x = T[((ij / D) * BA + al) * LDT + (ij % D) * BA + bl];
+            const double w = sc * sc;
+            sre += w * (x.x * ore[g] + x.y * oim[g]);
+            sim += w * (x.x * oim[g] - x.y * ore[g]);
+          }
+        }
+      } else if (in) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int ij = mb * 16 + lk + 4 * g;
@@ -285,6 +199,36 @@ __global__ __launch_bounds__(256) void k_theta_gate_mfma(const BondTask* __restr
       }
     }
   }
+  if constexpr (EXPVAL) {
+    sre = wave_sum(sre);
+    sim = wave_sum(sim);
+    __syncthreads();  // the tile is no longer read
+    if (lane == 0) sm[wave] = zmk(sre, sim);
+    __syncthreads();
+    if (tid == 0)
+      part[((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] =
+          zadd(zadd(sm[0], sm[1]), zadd(sm[2], sm[3]));
+  }
+}
+
+// out[task] = the sum of the task's tiles; one workgroup per task, gx x gy tiles of BA x BA.
+__global__ __launch_bounds__(256) void k_expval_sum(const BondTask* __restrict__ tasks, const zc* __restrict__ part,
+                                                    int gx, int gy, int ba, zc* __restrict__ out) {
+  const BondTask& t = tasks[blockIdx.x];
+  const int nx = (t.chil + ba - 1) / ba, ny = (t.chir + ba - 1) / ba;
+  const zc* p = part + (size_t)blockIdx.x * gx * gy;
+  double re = 0.0, im = 0.0;
+  for (int e = threadIdx.x; e < nx * ny; e += 256) {
+    const zc v = p[(size_t)(e / nx) * gx + e % nx];
+    re += v.x;
+    im += v.y;
+  }
+  __shared__ zc red[4];
+  re = wave_sum(re);
+  im = wave_sum(im);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = zmk(re, im);
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = zadd(zadd(red[0], red[1]), zadd(red[2], red[3]));
 }
 
 // ---------------------------------------------------------------------------
@@ -470,38 +414,48 @@ __global__ void k_write_gammas(const BondTask* __restrict__ tasks) {
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-hipError_t launch_theta_gate(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir,
-                             hipStream_t st) {
-  auto go = [&](auto kern, int BA) {
-    dim3 grid((max_chil + BA - 1) / BA, (max_chir + BA - 1) / BA, ntasks);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_tasks);
-    return hipGetLastError();
-  };
-  switch (d) {
-    case 2: return go(k_theta_gate<2>, ThetaCfg<2>::BA);
-    case 3: return go(k_theta_gate<3>, ThetaCfg<3>::BA);
-    case 4: return go(k_theta_gate<4>, ThetaCfg<4>::BA);
-    case 5: return go(k_theta_gate<5>, ThetaCfg<5>::BA);
-    case 6: return go(k_theta_gate<6>, ThetaCfg<6>::BA);
-    case 8: return go(k_theta_gate<8>, ThetaCfg<8>::BA);
-    default: return hipErrorInvalidValue;
-  }
-}
-
 hipError_t launch_theta_gate_mfma(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir,
                                   hipStream_t st) {
   auto go = [&](auto kern, int BA) {
     dim3 grid((max_chil + BA - 1) / BA, (max_chir + BA - 1) / BA, ntasks);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_tasks);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, d_tasks, (zc*)nullptr);
     return hipGetLastError();
   };
   switch (d) {
-    case 2: return go(k_theta_gate_mfma<2>, MfmaThetaCfg<2>::BA);
-    case 3: return go(k_theta_gate_mfma<3>, MfmaThetaCfg<3>::BA);
-    case 4: return go(k_theta_gate_mfma<4>, MfmaThetaCfg<4>::BA);
-    case 5: return go(k_theta_gate_mfma<5>, MfmaThetaCfg<5>::BA);
-    case 6: return go(k_theta_gate_mfma<6>, MfmaThetaCfg<6>::BA);
-    case 8: return go(k_theta_gate_mfma<8>, MfmaThetaCfg<8>::BA);
+    case 2: return go(k_theta_gate_mfma<2, false>, MfmaThetaCfg<2>::BA);
+    case 3: return go(k_theta_gate_mfma<3, false>, MfmaThetaCfg<3>::BA);
+    case 4: return go(k_theta_gate_mfma<4, false>, MfmaThetaCfg<4>::BA);
+    case 5: return go(k_theta_gate_mfma<5, false>, MfmaThetaCfg<5>::BA);
+    case 6: return go(k_theta_gate_mfma<6, false>, MfmaThetaCfg<6>::BA);
+    case 8: return go(k_theta_gate_mfma<8, false>, MfmaThetaCfg<8>::BA);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// Partial sums of one bond's expectation value with bond dimensions of up to chi.
+size_t expval_tiles(int d, int chi) {
+  const int ba = d <= 5 ? 16 : 8;
+  const size_t n = (chi + ba - 1) / ba;
+  return n * n;
+}
+
+hipError_t launch_expval(const BondTask* d_tasks, int ntasks, int d, int max_chil, int max_chir, zc* d_part, zc* d_out,
+                         hipStream_t st) {
+  auto go = [&](auto kern, int BA) {
+    const int gx = (max_chil + BA - 1) / BA, gy = (max_chir + BA - 1) / BA;
+    hipLaunchKernelGGL(kern, dim3(gx, gy, ntasks), dim3(256), 0, st, d_tasks, d_part);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_expval_sum, dim3(ntasks), dim3(256), 0, st, d_tasks, d_part, gx, gy, BA, d_out);
+    return hipGetLastError();
+  };
+  switch (d) {
+    case 2: return go(k_theta_gate_mfma<2, true>, MfmaThetaCfg<2>::BA);
+    case 3: return go(k_theta_gate_mfma<3, true>, MfmaThetaCfg<3>::BA);
+    case 4: return go(k_theta_gate_mfma<4, true>, MfmaThetaCfg<4>::BA);
+    case 5: return go(k_theta_gate_mfma<5, true>, MfmaThetaCfg<5>::BA);
+    case 6: return go(k_theta_gate_mfma<6, true>, MfmaThetaCfg<6>::BA);
+    case 8: return go(k_theta_gate_mfma<8, true>, MfmaThetaCfg<8>::BA);
     default: return hipErrorInvalidValue;
   }
 }
