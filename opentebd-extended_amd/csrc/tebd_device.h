@@ -146,8 +146,8 @@ __device__ __forceinline__ double zabs2(zc a) { return a.x * a.x + a.y * a.y; }
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
   const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xf, 0xf, true);
+  const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 template <int M>

@@ -22,7 +22,7 @@
 // A pair visit is bound by the latency of its rounds of rotations: three cyclic sweeps over
 // all index pairs per visit (93 rounds, two barriers each) took 59 us at 400 x 400
 // (Fermi-Hubbard, chi = 100) and 54 at 225 x 225 (Bose-Hubbard, chi = 45); one pass over the
-// cross pairs (16 rounds of one barrier) takes 17 and 15, for 6 to 7 outer sweeps instead of 5
+// cross pairs (16 rounds of one barrier) takes 16 and 14, for 6 to 7 outer sweeps instead of 5
 // to 6.
 //
 // Work that cannot change the result is skipped exactly:
@@ -255,12 +255,15 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
         }
       }
     }
+    unsigned entry = is_a ? T.entry[RW][tid] : 0u, next = tid < NN ? T.next[RW][tid] : 0u;
 #pragma unroll 1
     for (int r = 0; r < JB; ++r, buf ^= 1) {
       const RotBuf& R = rb[buf];
       if (is_a) {
-        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, T.entry[RW + r][tid], tid < NN ? T.next[RW + r][tid] : 0u, tr,
-                     tk, half, jrot);
+        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
+        const int ahead = RW + (r + 1 < JB ? r + 1 : 0);  // read now, used after the barrier
+        entry = T.entry[ahead][tid];
+        if (tid < NN) next = T.next[ahead][tid];
       } else if (is_q) {
         const double c = R.c[qt];
         const zc sw = R.sw[qt];
@@ -270,7 +273,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
           const zc xp = f[u], xq = s[u];
           f[u] = zsub(zscale(xp, c), zmul(zconj(sw), xq));
           const zc nq = zadd(zmul(sw, xp), zscale(xq, c));
-          s[u] = zdpp<kDppRotate>(nq, nq);
+          s[u] = zdpp<kDppRotate>(nq);
         }
       }
       __syncthreads();

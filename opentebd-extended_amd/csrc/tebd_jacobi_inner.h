@@ -6,7 +6,7 @@
 // What bounds a round: a wave64 instruction holds its SIMD for 4 cycles, so a round costs the
 // instructions of its longest wave plus one LDS round trip and one barrier.  With the index
 // arithmetic done in place, the rotations formed by all four waves and every entry read by
-// two threads, a round took 1650 cycles (0.69 us); hence
+// two threads, a round took 1650 cycles (0.69 us), now 1345; hence
 //   * one barrier per round: the thread that has updated the entry of one of the next round's
 //     pairs forms that rotation at once, from the value in its registers;
 //   * the threads that do so sit in one wave, the others skip the rotation's code;
@@ -14,7 +14,9 @@
 //     pair) comes from a table in LDS (read from global memory in every round it made each
 //     barrier wait for L2);
 //   * only the upper triangle of A is kept, each entry is read by one lane, and the two lanes
-//     of a 2x2 block exchange their rows.
+//     of a 2x2 block exchange their rows;
+//   * every LDS read of a round is issued before its first product, and the table's entries one
+//     round ahead, so a round waits for LDS once (1405 cycles without).
 #pragma once
 #include "tebd_device.h"
 
@@ -123,6 +125,11 @@ template <int CTRL>
 __device__ __forceinline__ zc zdpp(zc edge, zc v) {
   return zmk(dpp<CTRL>(edge.x, v.x), dpp<CTRL>(edge.y, v.y));
 }
+// The same where every lane has a source.
+template <int CTRL>
+__device__ __forceinline__ zc zdpp(zc v) {
+  return zmk(dpp_mov<CTRL>(v.x), dpp_mov<CTRL>(v.y));
+}
 // a or b, part by part (a conditional of the two structs would keep them in memory)
 __device__ __forceinline__ zc zsel(bool first, zc a, zc b) { return zmk(first ? a.x : b.x, first ? a.y : b.y); }
 // v with its sign flipped when the top bit of m is set
@@ -173,13 +180,15 @@ __device__ __forceinline__ void update_block(zc* A, double* dg, const RotBuf& R,
   zc own0 = *l0, own1 = *l1;
   double* const da = reinterpret_cast<double*>(reinterpret_cast<char*>(dg) + (next & 0xffu));
   double* const db = reinterpret_cast<double*>(reinterpret_cast<char*>(dg) + ((next >> 8) & 0xffu));
-  const double a = *da, b = *db;
+  double a = *da, b = *db;
+  // every LDS read of the round is under way before the first value is used
+  asm volatile("" : "+v"(a), "+v"(b), "+v"(own0.x), "+v"(own0.y), "+v"(own1.x), "+v"(own1.y));
   const bool rot = swr.x != 0.0 || swr.y != 0.0 || swk.x != 0.0 || swk.y != 0.0 || next != 0u;
   if (!__any(rot)) return;
   const unsigned s0 = entry << 1, s1 = entry;  // the conjugation bits at the top
   own0.y = flip(own0.y, s0);
   own1.y = flip(own1.y, s1);
-  const zc oth0 = zdpp<kDppSwap>(own0, own0), oth1 = zdpp<kDppSwap>(own1, own1);
+  const zc oth0 = zdpp<kDppSwap>(own0), oth1 = zdpp<kDppSwap>(own1);
   // this lane's row after the row rotation: A_p <- c A_p - s w A_q ; A_q <- s conj(w) A_p + c A_q;
   // then the column rotation: A_:p <- c A_:p - s conj(w) A_:q ; A_:q <- s w A_:p + c A_:q
   const double fx = half ? swr.x : -swr.x;

@@ -205,6 +205,7 @@ __device__ __forceinline__ void inner_solve(PairLds& L, const InnerRounds<kAllRo
       L.A[p][q] = make_rotation(L.rb[buf], L.dg[p], L.dg[q], &L.dg[p], &L.dg[q], &L.swept[isw & 1], pt, L.A[p][q], jrot);
     }
     __syncthreads();
+    unsigned entry = is_a ? T.entry[0][pt] : 0u, next = pt < 2 * kInnerPairs ? T.next[0][pt] : 0u;
 #pragma unroll 1
     for (int rd = 0; rd < kAllRounds; ++rd, buf ^= 1) {
       const RotBuf& R = L.rb[buf];
@@ -234,8 +235,10 @@ __device__ __forceinline__ void inner_solve(PairLds& L, const InnerRounds<kAllRo
           f[u] = zsel(qt != 0, nf, f[u]);
         }
       } else if (is_a) {
-        update_block(&L.A[0][0], L.dg, R, L.rb[buf ^ 1], &L.swept[isw & 1], T.entry[rd][pt],
-                     pt < 2 * kInnerPairs ? T.next[rd][pt] : 0u, tr, tk, half, jrot);
+        update_block(&L.A[0][0], L.dg, R, L.rb[buf ^ 1], &L.swept[isw & 1], entry, next, tr, tk, half, jrot);
+        const int ahead = rd + 1 < kAllRounds ? rd + 1 : 0;  // read now, used after the barrier
+        entry = T.entry[ahead][pt];
+        if (pt < 2 * kInnerPairs) next = T.next[ahead][pt];
       }
       __syncthreads();
     }
