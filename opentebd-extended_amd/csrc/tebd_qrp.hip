@@ -173,32 +173,44 @@ __device__ __forceinline__ void gram_reduce(const d4 (&dre)[NP][NQ], const d4 (&
 }
 
 // T (nbp x nbp, upper) of the compact WY form H_0 .. H_{nbp-1} = I - V T V^H from the
-// reflector scalars and G = V^H V:  T[q][q] = tau_q, T[0:q, q] = -tau_q T[0:q, 0:q] G[0:q, q].
-// Row p of T only involves row p's own earlier entries (T is upper triangular), so
-// thread p < QB forms row p in registers; written to the panel's slot Tp (column-major,
-// zero-padded to QB x QB).  Called by every thread of the workgroup.
-__device__ void form_t(const zc (*G)[QB + 1], const zc* stau, int nbp, zc* Tp) {
+// reflector scalars and G = V^H V:  T[q][q] = tau_q, and for two neighbouring diagonal blocks
+// T11, T22 of size h the block between them is -T11 G12 T22.  Wave 0 doubles h from 1 to 8, one
+// entry per lane (column by column, one thread per row, took 8.5 us, this 2); written to the
+// panel's slot Tp (column-major, zero-padded to QB x QB).  Called by every thread of the
+// workgroup; Tm and X are scratch.
+__device__ void form_t(const zc (*G)[QB + 1], const zc* stau, int nbp, zc* Tp, zc (*Tm)[QB + 1], zc (*X)[QB + 1]) {
   __syncthreads();  // G and stau are complete
-  if (threadIdx.x >= QB) return;
-  const int pp = threadIdx.x;
-  zc row[QB];
-#pragma unroll
-  for (int q = 0; q < QB; ++q) row[q] = zmk(0.0, 0.0);
-  if (pp < nbp) {
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      if (q == pp) row[q] = stau[q];
-      if (q > pp && q < nbp) {
-        zc acc = zmk(0.0, 0.0);
-#pragma unroll
-        for (int kk = 0; kk < QB; ++kk)
-          if (kk >= pp && kk < q) zfma(acc, row[kk], G[kk][q]);
-        row[q] = zmul(zmk(-stau[q].x, -stau[q].y), acc);
-      }
-    }
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int e = lane; e < QB * QB; e += 64) {
+    const int r = e % QB, c = e / QB;
+    Tm[r][c] = r == c && c < nbp ? stau[c] : zmk(0.0, 0.0);
   }
+  wave_sync();
 #pragma unroll
-  for (int q = 0; q < QB; ++q) Tp[pp + QB * q] = row[q];
+  for (int h = 1; h < QB; h *= 2) {
+    const int blk = lane / (h * h), i = 2 * h * blk + lane % h, j = 2 * h * blk + h + (lane / h) % h;
+    const bool mine = blk < QB / (2 * h) && j < nbp;
+    zc acc = zmk(0.0, 0.0);
+    if (mine)
+#pragma unroll
+      for (int k = 0; k < h; ++k)
+        if (2 * h * blk + h + k <= j) zfma(acc, G[i][2 * h * blk + h + k], Tm[2 * h * blk + h + k][j]);
+    if (mine) X[i][j] = acc;
+    wave_sync();
+    acc = zmk(0.0, 0.0);
+    if (mine)
+#pragma unroll
+      for (int k = 0; k < h; ++k) zfma(acc, Tm[i][2 * h * blk + k], X[2 * h * blk + k][j]);
+    wave_sync();
+    if (mine) Tm[i][j] = zmk(-acc.x, -acc.y);
+    wave_sync();
+  }
+  for (int e = lane; e < QB * QB; e += 64) Tp[e] = Tm[e % QB][e / QB];
 }
 
 // Householder scalars of the column (alpha; x) with |x|^2 = xn2 (xLARFG convention):
@@ -217,55 +229,54 @@ __device__ __forceinline__ bool householder(zc alpha, double xn2, zc& tau, doubl
   return true;
 }
 
+// The number of the n keys (LDS, n a multiple of 8) above `mine`.
+__device__ inline int count_above(const unsigned long long* key, int n, unsigned long long mine) {
+  int rank = 0;
+  for (int k = 0; k < n; k += 8) {
+    unsigned long long u[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) u[x] = key[k + x];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) rank += u[x] > mine ? 1 : 0;
+  }
+  return rank;
+}
+
 // Selection of panel j0 by the NT threads of a workgroup: sel[0..nbp) := the nbp
-// candidates (columns j0 + c, c < ncand, squared norms snrm[c] in LDS) of largest norm
-// in descending order, ties to the lowest index; NaN norms are never taken.  *sstop :=
-// 1 when even the largest is not above thr (the numerical rank is j0), 2 when fewer than
-// nbp candidates have a norm, else 0.  Up to NT candidates, every thread ranks one
-// candidate against all the others (one pass, broadcast LDS reads); beyond that, wave 0
-// takes nbp argmax passes (snrm entries taken are overwritten).  snrm has kMaxCols + 1
-// entries: the last receives the largest norm.  Ends with a barrier.
+// candidates (columns j0 + c, c < ncand) of largest norm in descending order; norms that
+// agree to 2^-39 count as equal, ties go to the lowest index; NaN norms are never taken.
+// *sstop := 1 when even the largest is not above thr (the numerical rank is j0), 2 when
+// fewer than nbp candidates have a norm, else 0.
+// key (kMaxCols) and top (kMaxCols / 64 * QB) are LDS.  A key is a squared norm's bits,
+// ordered as the number is, with the last 13 replaced by 8191 - c: one comparison orders two
+// candidates.  Every candidate is ranked among the 64 of its block, then the QB best of each
+// block among each other.  Ends with a barrier.
 template <int NT>
-__device__ void select_panel(double* snrm, int ncand, int nbp, double thr, int j0, int* sel, int* sstop, int tid) {
-  const int lane = tid & 63, wave = tid >> 6;
+__device__ void select_panel(const double* qnrm, unsigned long long* key, unsigned long long* top, int ncand, int nbp,
+                             double thr, int j0, int* sel, int* sstop, int tid) {
   if (tid < QB) sel[tid] = -1;
+  const int nblk = (ncand + 63) / 64;
+  for (int c = tid; c < 64 * nblk; c += NT) {
+    const double v = c < ncand ? qnrm[j0 + c] : -1.0;
+    key[c] = v >= 0.0 ? ((unsigned long long)__double_as_longlong(v) & ~8191ull) | (unsigned)(8191 - c) : 0ull;
+    if (c < nblk * QB) top[c] = 0ull;
+  }
   __syncthreads();
-  if (ncand <= NT) {
-    if (tid < ncand) {
-      const double v = snrm[tid];
-      if (v == v) {
-        int rank = 0;
-        for (int k = 0; k < ncand; ++k) {
-          const double u = snrm[k];
-          rank += (u > v || (u == v && k < tid)) ? 1 : 0;
-        }
-        if (rank < nbp) sel[rank] = j0 + tid;
-        if (rank == 0) snrm[kMaxCols] = v;
-      }
-    }
-  } else if (wave == 0) {
-    for (int q = 0; q < nbp; ++q) {
-      double bv = -1.0;
-      int bi = -1;
-      for (int k = lane; k < ncand; k += 64) {
-        const double v = snrm[k];
-        if (v > bv) { bv = v; bi = k; }
-      }
-      for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_xor(bv, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-      }
-      if (bi < 0) break;  // every lane holds the same winner
-      if (lane == 0) sel[q] = j0 + bi;
-      if (lane == 0 && q == 0) snrm[kMaxCols] = bv;
-      if (lane == (bi & 63)) snrm[bi] = -1.0;  // a lane only ever reads the entries it clears
-    }
+  for (int c = tid; c < 64 * nblk; c += NT) {
+    const unsigned long long mine = key[c];
+    const int rank = count_above(key + (c & ~63), 64, mine);
+    if (mine != 0ull && rank < QB) top[c / 64 * QB + rank] = mine;
+  }
+  __syncthreads();
+  for (int c = tid; c < nblk * QB; c += NT) {
+    const unsigned long long mine = top[c];
+    const int rank = count_above(top, nblk * QB, mine);
+    if (mine != 0ull && rank < nbp) sel[rank] = j0 + 8191 - (int)(mine & 8191ull);
   }
   __syncthreads();
   if (tid == 0) {
     int st = 0;
-    if (sel[0] < 0 || !(snrm[kMaxCols] > thr)) st = 1;
+    if (sel[0] < 0 || !(__longlong_as_double((long long)(key[sel[0] - j0] & ~8191ull)) > thr)) st = 1;
     for (int q = 1; q < nbp && !st; ++q)
       if (sel[q] < 0) st = 2;
     *sstop = st;
@@ -337,14 +348,14 @@ __device__ __forceinline__ void move_rows(zc* Wq, size_t ld, int i, int nmv, con
 
 // LDS of the register-resident panel.
 struct PanelLds {
-  double snrm[kMaxCols + 1];
+  unsigned long long key[kMaxCols], top[kMaxCols / 64 * QB];
   int sel[QB], mv_src[QB], mv_dst[QB];
   int snmv, sstop;
   double red[PW][32];
   double wsum[PW][32];
   double rnorm[PW];
   zc salpha;
-  zc G[QB][QB + 1];
+  zc G[QB][QB + 1], Tm[QB][QB + 1], X[QB][QB + 1];
   zc stau[QB];
 };
 
@@ -362,8 +373,10 @@ struct PanelLds {
 // it: per reflector a wave spends about 300 on the norm, the Householder scalars and the
 // 32-value reduction and 120 RPT on its rows, so few waves with two rows per thread beat
 // many with one; exchanging lanes by data-parallel moves and lane swaps instead of the LDS
-// crossbar, and one barrier less, shorten the rest.  With eight waves for every row count a
-// panel took 52 us at 128 rows, 65 at 225 and 73 at 400; now 32, 44 and 62.
+// crossbar, and one barrier less, shorten the rest.  With eight waves for every row count,
+// one wave's 16 passes over the norms for the selection and T column by column, a panel took
+// 52 us at 128 rows, 65 at 225 and 73 at 400; now 32, 34 and 41, of which the chain is 24, 26
+// and 30, the selection 3, 3 and 5 (5, 6 and 18 before) and T 2 (8.5).
 template <int RPT, int NW>
 __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S) {
   constexpr int NT = 64 * NW;
@@ -375,8 +388,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   const size_t ld = Rb;
 
   // 1. selection
-  for (int k = tid; k < ncand; k += NT) S.snrm[k] = t.qnrm[j0 + k];
-  select_panel<NT>(S.snrm, ncand, nbp, t.qstate[1], j0, S.sel, &S.sstop, tid);
+  select_panel<NT>(t.qnrm, S.key, S.top, ncand, nbp, t.qstate[1], j0, S.sel, &S.sstop, tid);
   if (S.sstop) {
     if (tid == 0) t.qstate[0] = S.sstop == 1 ? (double)j0 : 0.0;
     return;
@@ -516,7 +528,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
         if (c < nbp) t.Wq[i + ld * (j0 + c)] = a[s][c];
     }
   }
-  form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, S.Tm, S.X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
 
@@ -560,15 +572,14 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
   const int nbp = (kmax - j0) < QB ? (kmax - j0) : QB;
   const int ncand = t.Cb - j0;
   const size_t ld = t.Rb;
-  __shared__ double snrm[kMaxCols + 1];
+  __shared__ unsigned long long key[kMaxCols], top[kMaxCols / 64 * QB];
   __shared__ int sel[QB], mv_src[QB], mv_dst[QB];
   __shared__ int snmv, sstop;
   __shared__ double red[4];
-  __shared__ zc G[QB][QB + 1];
+  __shared__ zc G[QB][QB + 1], Tm[QB][QB + 1], X[QB][QB + 1];
   __shared__ zc stau[QB];
   __shared__ double gred[3][2][256];
-  for (int k = tid; k < ncand; k += 256) snrm[k] = t.qnrm[j0 + k];
-  select_panel<256>(snrm, ncand, nbp, t.qstate[1], j0, sel, &sstop, tid);
+  select_panel<256>(t.qnrm, key, top, ncand, nbp, t.qstate[1], j0, sel, &sstop, tid);
   if (sstop) {
     if (tid == 0) t.qstate[0] = sstop == 1 ? (double)j0 : 0.0;
     return;
@@ -636,7 +647,7 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
     gram_partial<1, 1>(vload, vload, K, wave, 4, lane, gre, gim);
     gram_reduce<1, 1>(gre, gim, gred, &G[0][0], QB + 1, wave, lane);
   }
-  form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, Tm, X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
 
