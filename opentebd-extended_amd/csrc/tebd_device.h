@@ -170,6 +170,12 @@ __device__ __forceinline__ double swap_sum(double a, double b) {
   const auto lo = sw((unsigned)x, (unsigned)y), hi = sw((unsigned)(x >> 32), (unsigned)(y >> 32));
   return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) + __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
 }
+// Lane 0's value, uniform over the wave.
+__device__ __forceinline__ double first_lane(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readfirstlane((int)x), hi = __builtin_amdgcn_readfirstlane((int)(x >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
 // Sum over the wave, in every lane (the order of a butterfly from distance 32 down to 1).
 __device__ __forceinline__ double wave_sum(double v) {
   v = swap_sum<32>(v, v);

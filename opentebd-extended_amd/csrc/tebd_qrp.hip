@@ -351,10 +351,9 @@ struct PanelLds {
   unsigned long long key[kMaxCols], top[kMaxCols / 64 * QB];
   int sel[QB], mv_src[QB], mv_dst[QB];
   int snmv, sstop;
-  double red[PW][32];
-  double wsum[PW][32];
-  double rnorm[PW];
-  zc salpha;
+  double red[2][PW][32];  // by reflector parity: one barrier per reflector
+  zc row[2][QB];
+  zc coef[PW][QB];
   zc G[QB][QB + 1], Tm[QB][QB + 1], X[QB][QB + 1];
   zc stau[QB];
 };
@@ -366,17 +365,21 @@ struct PanelLds {
 //     threshold the numerical rank is j0 and the factorisation ends;
 //  2. the picked columns are loaded into registers; the displaced ones are moved;
 //  3. unpivoted Householder QR of the panel rows j0.. (xLARFG convention).  For
-//     reflector q one fixed-order reduction yields w_k = v_q^H a_k (k > q, for the
-//     update) and G[p][q] = v_p^H v_q (p < q, for T);
+//     reflector q one fixed-order reduction over the rows below j, with the column not yet
+//     scaled, yields its norm, w_k = v_q^H a_k (k > q, for the update) and G[p][q] = v_p^H v_q
+//     (p < q, for T);
 //  4. the panel is stored back and T formed.
-// The 16 reflectors are one dependent chain, bound by the instructions each SIMD issues for
-// it: per reflector a wave spends about 300 on the norm, the Householder scalars and the
-// 32-value reduction and 120 RPT on its rows, so few waves with two rows per thread beat
-// many with one; exchanging lanes by data-parallel moves and lane swaps instead of the LDS
-// crossbar, and one barrier less, shorten the rest.  With eight waves for every row count,
-// one wave's 16 passes over the norms for the selection and T column by column, a panel took
-// 52 us at 128 rows, 65 at 225 and 73 at 400; now 32, 34 and 41, of which the chain is 24, 26
-// and 30, the selection 3, 3 and 5 (5, 6 and 18 before) and T 2 (8.5).
+// The 16 reflectors are one dependent chain of about 3000 cycles each, bound by the
+// instructions each SIMD issues for it (about 450 per reflector and wave with one row per
+// thread, 120 more with a second) and their latency: dot products 840 cycles, reduction of the 32
+// values over the wave 800, over the waves 190 (two) to 440 (four), Householder scalars 530,
+// coefficients 400, update 600.  So few waves with two rows per thread beat many with one, lanes
+// are exchanged by data-parallel moves and lane swaps instead of the LDS crossbar, and there is one
+// reduction and one barrier per reflector (a first one for the norm cost 3 us per panel).  With
+// eight waves for every row count, three barriers per reflector, one wave's 16 passes over the
+// norms for the selection and T column by column, a panel took 52 us at 128 rows, 65 at 225 and
+// 73 at 400; now 28, 31 and 37 (at 64: 27), of which the chain is 21, 23 and 26, the selection 3,
+// 3 and 5 and T 2.
 template <int RPT, int NW>
 __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S) {
   constexpr int NT = 64 * NW;
@@ -414,58 +417,38 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   // index is static: column q sits in a[.][q], first as data, then as reflector v_q
   // (rows > j0 + q) below R(:, q).
   static_for<QB>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
+    constexpr int q = decltype(qc)::value, buf = q & 1;
     if (q >= nbp) return;
     const int j = j0 + q;
-    double part = 0.0;
+    // the column below row j, zero elsewhere, so that the products need no row test
+    zc xq[RPT];
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
       const int i = tid + NT * s;
-      if (i > j && i < Rb) part += zabs2(a[s][q]);
-      if (i == j) S.salpha = a[s][q];
-    }
-    part = wave_sum(part);
-    if (lane == 0) S.rnorm[wave] = part;
-    __syncthreads();
-    double xn2 = 0.0;
+      xq[s] = i > j ? a[s][q] : zmk(0.0, 0.0);  // rows from Rb on are zero
+      if (i == j) {
 #pragma unroll
-    for (int w = 0; w < NW; ++w) xn2 += S.rnorm[w];
-    zc tau, scale = zmk(1.0, 0.0);
-    double beta = 0.0;
-    const bool refl = householder(S.salpha, xn2, tau, beta, scale);
-    // v_q (rows > j; v_j = 1 implicitly) and R(j, j)
-    if (refl) {
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        const int i = tid + NT * s;
-        if (i > j && i < Rb) a[s][q] = zmul(a[s][q], scale);
-        if (i == j) a[s][q] = zmk(beta, 0.0);
+        for (int c = 0; c < QB; ++c) S.row[buf][c] = a[s][c];
       }
     }
-    // slot m = 1 .. 15 - q: conj(v_q) a_(q+m) (the later columns, for the update);
-    // slot m > 15 - q: conj(v_p) v_q, p = m - 16 + q (the earlier reflectors, for T)
+    // slot 0: |x|^2; slot m = 1 .. 15 - q: conj(x) a_(q+m) (the later columns, for the update);
+    // slot m > 15 - q: conj(v_p) x, p = m - 16 + q (the earlier reflectors, for T)
     double x[2 * QB];
 #pragma unroll
     for (int e = 0; e < 2 * QB; ++e) x[e] = 0.0;
-    // v_q on this thread's rows: 1 at row j, zero outside rows j .. Rb - 1, so that the
-    // products and the update below need no row test
-    zc vq[RPT];
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
-      const int i = tid + NT * s;
-      vq[s] = (i == j) ? zmk(1.0, 0.0) : ((i > j && i < Rb) ? a[s][q] : zmk(0.0, 0.0));
-    }
-#pragma unroll
-    for (int s = 0; s < RPT; ++s)
+      x[0] = fma(xq[s].x, xq[s].x, fma(xq[s].y, xq[s].y, x[0]));
 #pragma unroll
       for (int m = 1; m < QB; ++m) {
-        const bool later = m <= QB - 1 - q;  // earlier reflectors: rows >= j > j0 + p
+        const bool later = m <= QB - 1 - q;  // earlier reflectors: rows > j > j0 + p
         const zc other = a[s][later ? q + m : m - QB + q];
-        const zc l = later ? vq[s] : other;
-        const zc r = later ? other : vq[s];
+        const zc l = later ? xq[s] : other;
+        const zc r = later ? other : xq[s];
         x[2 * m] = fma(l.x, r.x, fma(l.y, r.y, x[2 * m]));
         x[2 * m + 1] = fma(l.x, r.y, fma(-l.y, r.x, x[2 * m + 1]));
       }
+    }
     // reduce-scatter of the 32 values over the wave: lane l ends with value
     // 16 b5 + 8 b4 + 4 b3 + 2 b2 + b1 (b = bits of l), summed over all 64 lanes
     {
@@ -489,33 +472,46 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
       y1 += lane_xor<1>(y1);
       const int idx = 16 * ((lane >> 5) & 1) + 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) +
                       2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
-      if ((lane & 1) == 0) S.red[wave][idx] = y1;
+      if ((lane & 1) == 0) S.red[buf][wave][idx] = y1;
     }
     __syncthreads();
-    // every wave sums the waves' partials for itself, which saves a barrier
-    if (lane < 32) {
-      double sum = 0.0;
+    // Every wave sums the waves' partials for itself, which saves a barrier; lane m (mod 16)
+    // takes slot m.
+    const int m = lane & (QB - 1);
+    zc sum = zmk(0.0, 0.0);
 #pragma unroll
-      for (int w = 0; w < NW; ++w) sum += S.red[w][lane];
-      S.wsum[wave][lane] = sum;
+    for (int w = 0; w < NW; ++w) sum = zadd(sum, zmk(S.red[buf][w][2 * m], S.red[buf][w][2 * m + 1]));
+    const zc alpha = S.row[buf][q], other = S.row[buf][(q + m) & (QB - 1)];  // row j of slot m's column
+    const double xn2 = first_lane(sum.x);
+    zc tau, scale = zmk(1.0, 0.0);
+    double beta = 0.0;
+    const bool refl = householder(alpha, xn2, tau, beta, scale);
+    // v_q = (1; x scale): w_k = conj(scale) sum + a_jk, and v_p^H v_q = scale sum + conj(v_p,j)
+    if (m <= QB - 1 - q) {
+      S.coef[wave][m] = zmul(zmk(-tau.x, tau.y), zadd(zmul(zconj(scale), sum), other));
+    } else if (tid < QB) {
+      S.G[q + m - QB][q] = zadd(zmul(scale, sum), zconj(other));
     }
+    if (tid == 0) S.stau[q] = tau;  // to global memory after the chain: the next barrier would wait for it
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    const double* const wsum = S.wsum[wave];
-    if (tid == 0) {
-      for (int m = QB - q; m < QB; ++m) S.G[m - QB + q][q] = zmk(wsum[2 * m], wsum[2 * m + 1]);
-      S.stau[q] = tau;
-      t.tau[j] = tau;
-    }
     if (refl) {
-      const zc ctau = zconj(tau);
+      zc vq[RPT];
 #pragma unroll
-      for (int m = 1; m <= QB - 1 - q; ++m) {
-        const zc f = zmul(ctau, zmk(wsum[2 * m], wsum[2 * m + 1]));
+      for (int s = 0; s < RPT; ++s) {
+        const int i = tid + NT * s;
+        vq[s] = i == j ? zmk(1.0, 0.0) : zmul(xq[s], scale);
+        if (i > j) a[s][q] = vq[s];
+        if (i == j) a[s][q] = zmk(beta, 0.0);
+      }
 #pragma unroll
-        for (int s = 0; s < RPT; ++s) a[s][q + m] = zsub(a[s][q + m], zmul(f, vq[s]));
+      for (int k = 1; k <= QB - 1 - q; ++k) {
+        const zc f = S.coef[wave][k];  // minus the coefficient
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) zfma(a[s][q + k], f, vq[s]);
       }
     }
+    __builtin_amdgcn_wave_barrier();  // the coefficients are read before the next are written
   });
 
   // 4. store the panel (R above and on the diagonal, reflectors below) and T
@@ -528,6 +524,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
         if (c < nbp) t.Wq[i + ld * (j0 + c)] = a[s][c];
     }
   }
+  if (tid < nbp) t.tau[j0 + tid] = S.stau[tid];
   form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, S.Tm, S.X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
@@ -546,7 +543,9 @@ __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __
   }
   __shared__ PanelLds S;
   const int wave = threadIdx.x >> 6;
-  if (t.Rb <= 128) {
+  if (t.Rb <= 64 && t.Cb <= 64) {  // no barriers: 28 us instead of 31 at 64 x 64; more candidates need more threads
+    if (wave < 1) panel_reg<1, 1>(t, j0, S);
+  } else if (t.Rb <= 128) {
     if (wave < 2) panel_reg<1, 2>(t, j0, S);
   } else if (NWMAX >= 4 && t.Rb <= 256) {
     if (wave < 4) panel_reg<1, NWMAX < 4 ? NWMAX : 4>(t, j0, S);
