@@ -193,7 +193,8 @@ __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 // Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
 // sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
 // blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
-// includes the blocks' own couplings, the pairs within the blocks too, in two passes.
+// includes the blocks' own couplings, the pairs within the blocks too, in two passes (and in every
+// round of a batch that fills the GPU with long columns, where sweeps cost more than rounds).
 // Measured on Hubbard and Bose-Hubbard bonds (numpy restatement, 225 x 225 and 256 x 256):
 // 6 outer sweeps and 1300-1400 inner rounds in sequence per solve; three cyclic sweeps over
 // all 496 pairs per visit take 5 outer sweeps but 4400-4650 rounds in sequence.
@@ -227,13 +228,17 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
     __syncthreads();
     if (FULL) {
       int rd = 0;
+      unsigned entry = is_a ? T.entry[0][tid] : 0u, next = tid < NN ? T.next[0][tid] : 0u;
 #pragma unroll 1
       for (int h = 8; h >= 1; h >>= 1)
 #pragma unroll 1
         for (int r = 0; r < h; ++r, ++rd, buf ^= 1) {
           const RotBuf& R = rb[buf];
           if (is_a) {
-            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, T.entry[rd][tid], T.next[rd][tid], tr, tk, half, jrot);
+            const unsigned e1 = T.entry[rd + 1][tid], n1 = T.next[rd + 1][tid];
+            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
+            entry = e1;
+            next = n1;
           } else if (is_q) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -260,10 +265,19 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
     for (int r = 0; r < JB; ++r, buf ^= 1) {
       const RotBuf& R = rb[buf];
       if (is_a) {
-        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
         const int ahead = RW + (r + 1 < JB ? r + 1 : 0);  // read now, used after the barrier
-        entry = T.entry[ahead][tid];
-        if (tid < NN) next = T.next[ahead][tid];
+        unsigned e1, n1 = 0u;
+        if (FULL) {
+          e1 = T.entry[ahead][tid];
+          n1 = T.next[ahead][tid];
+        }
+        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
+        if (!FULL) {
+          e1 = T.entry[ahead][tid];
+          if (tid < NN) n1 = T.next[ahead][tid];
+        }
+        entry = e1;
+        next = n1;
       } else if (is_q) {
         const double c = R.c[qt];
         const zc sw = R.sw[qt];
@@ -289,7 +303,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
   }
 }
 
-template <bool FULL>
+template <bool FULL, bool WITHIN>
 __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* __restrict__ tasks, int sweep, int round,
                                                       double tol_rel, double tol_abs, int* __restrict__ wl_count,
                                                       int2* __restrict__ wl_items, int wl_cap) {
@@ -321,15 +335,18 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   };
   __shared__ Scratch sc;
   __shared__ RotBuf rb[2];
-  __shared__ typename std::conditional<FULL, decltype(FullTable::rounds), decltype(CrossTable::rounds)>::type table;
+  // The schedule of 16 rounds lies in LDS; that of 31 (60 KB, which would leave room for one workgroup
+  // on a CU instead of two) is read from L2 one round ahead.  With it in LDS the exact step of Hubbard
+  // L = 128, chi = 256 took 204 ms instead of 192 and the number-conserving one of L = 64, chi = 128
+  // 15.8 instead of 15.2.
+  __shared__ typename std::conditional<WITHIN, int, decltype(CrossTable::rounds)>::type table;
   __shared__ int s_flag;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const zc* Wi = t.W + (size_t)t.R * (bi * JB);
   const zc* Wj = t.W + (size_t)t.R * (bj * JB);
   if (tid == 0) s_flag = 0;
-  if constexpr (FULL) load_rounds(table, kFull.rounds, tid, kRoundThreads);
-  else load_rounds(table, kCross.rounds, tid, kRoundThreads);
+  if constexpr (!WITHIN) load_rounds(table, kCross.rounds, tid, kRoundThreads);
 
   // ---- Gram: A = [Wi Wj]^H [Wi Wj]
   {
@@ -396,7 +413,8 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
 
   // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
   zc (*Q)[JC + 1] = sc.Q;
-  inner_jacobi<FULL>(A, Q, dg, rb, table, tid);
+  if constexpr (WITHIN) inner_jacobi<true>(A, Q, dg, rb, kFull.rounds, tid);
+  else inner_jacobi<false>(A, Q, dg, rb, table, tid);
   zc* qg = t.Qg + (size_t)p * JC * JC;
   for (int e = tid; e < JC * JC; e += kRoundThreads) qg[e] = Q[e / JC][e % JC];  // qg[k JC + c] = Q[k][c]
   if (tid == 0) {
@@ -507,15 +525,12 @@ hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sw
   return hipGetLastError();
 }
 
-hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
+hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, bool within, int sweep, int round,
                                double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
                                int2* wl_items, int wl_cap, hipStream_t st) {
-  if (round == 0)
-    hipLaunchKernelGGL(k_jacobi_round<true>, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round,
-                       tol_rel, tol_abs, wl_count, wl_items, wl_cap);
-  else
-    hipLaunchKernelGGL(k_jacobi_round<false>, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round,
-                       tol_rel, tol_abs, wl_count, wl_items, wl_cap);
+  const auto k = round == 0 ? k_jacobi_round<true, true> : within ? k_jacobi_round<false, true> : k_jacobi_round<false, false>;
+  hipLaunchKernelGGL(k, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round, tol_rel, tol_abs,
+                     wl_count, wl_items, wl_cap);
   return hipGetLastError();
 }
 
