@@ -332,11 +332,11 @@ void clear_graphs(tebd_ctx* c) {
 // One Jacobi sweep (sweep start, then every round's Gram/eigenproblem kernel and its
 // rotation kernel) captured from the context's stream as an executable graph; null if
 // the capture fails.  The captured launches are the eager ones with the same arguments.
-hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, bool within, int cls, int rows_w, int rows_v) {
+hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int cls, int rows_w, int rows_v) {
   if (hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
   hipError_t e = launch_jacobi_sweep_begin(d_t, nb, cls, c->wl_count, c->st);
   for (int r = 0; r < 2 * Pmax - 1 && e == hipSuccess; ++r) {
-    e = launch_jacobi_round(d_t, nb, Pmax, within, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count, c->wl_items,
+    e = launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count, c->wl_items,
                             c->wl_cap, c->st);
     if (e == hipSuccess)
       e = launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st);
@@ -394,16 +394,13 @@ hipError_t fetch_counters(tebd_ctx* c, int nb) {
   return hipMemcpyAsync(c->h_counters, c->counters, sizeof(int) * kCounters * nb, hipMemcpyDeviceToHost, c->st);
 }
 
-constexpr int kWithinPairs = 256;  // pairs of a round, all tasks together (one per CU)
-constexpr int kWithinRows = 512;
-
 // Jacobi SVDs of the tasks of one stage (task i uses slot i): the small ones in one launch,
 // the others sweep by sweep until one rotates nothing.  When every task is small nothing is
 // waited for: *deferred is set, the counters' copy to the host is queued, and the caller
 // calls jacobi_account after its next wait.
 int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool* deferred) {
   HIPCHK(c, launch_jacobi_begin(d_t, nb, c->st));
-  int rows_w = 1, rows_v = 0, Pmax = 0, pairs = 0;
+  int rows_w = 1, rows_v = 0, Pmax = 0;
   bool one = false, two = false;
   for (int i = 0; i < nb; ++i) {
     if (small_solve(h_t[i])) {
@@ -411,7 +408,6 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
       continue;
     }
     Pmax = std::max(Pmax, h_t[i].P);
-    pairs += h_t[i].P;
     rows_w = std::max(rows_w, h_t[i].R);
     if (h_t[i].V) rows_v = std::max(rows_v, h_t[i].NV);
   }
@@ -426,14 +422,6 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
   // work and lets one captured graph serve every row count of a slab class.
   rows_w = round_up(rows_w, kGraphRowQuantum);
   rows_v = round_up(rows_v, kGraphRowQuantum);
-  // With few pairs in a round its latency counts, and with short columns the inner rounds: a visit
-  // then rotates the cross pairs alone.  With enough pairs to keep every CU busy and long columns
-  // the Grams and the rotations of W count, and rotating the pairs within the blocks too saves a
-  // sixth of the sweeps.  Hubbard, exact SVDs, ms per step without and with it: L = 128, chi = 256
-  // (21 bonds to a lane) 206 and 192; L = 32, chi = 256 (5 bonds) 121 and 123; L = 64, chi = 128 (10
-  // bonds of at most 512 rows) 47 and 51; the number-conserving blocks of L = 128, chi = 256 (hundreds
-  // of at most 256 rows) 77 and 84.
-  const bool within = pairs >= kWithinPairs && rows_w > kWithinRows;
   int sweeps = 0;
   bool converged = false;
   while (sweeps < kMaxSweeps && !converged) {
@@ -442,13 +430,13 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
     const int cls = sweeps == 0 ? 0 : ((sweeps & 1) ? 1 : 2);
     bool done = false;
     if (c->graphs && !c->profiling) {
-      const std::array<long long, 6> key = {(long long)(uintptr_t)d_t, nb, Pmax, rows_w, rows_v, 2 * cls + within};
+      const std::array<long long, 6> key = {(long long)(uintptr_t)d_t, nb, Pmax, rows_w, rows_v, cls};
       auto it = c->sweep_graphs.find(key);
       // A full cache is not emptied while the context runs: executable graphs are
       // destroyed only when the context (or its lane) is freed, after its stream has
       // drained.  Sweeps of shapes beyond the cap launch eagerly.
       if (it == c->sweep_graphs.end() && c->sweep_graphs.size() < kMaxSweepGraphs) {
-        hipGraphExec_t ge = capture_sweep(c, d_t, nb, Pmax, within, cls, rows_w, rows_v);
+        hipGraphExec_t ge = capture_sweep(c, d_t, nb, Pmax, cls, rows_w, rows_v);
         if (ge) it = c->sweep_graphs.emplace(key, ge).first;
         else c->graphs = false;  // capture unavailable: launch eagerly from now on
       }
@@ -462,7 +450,7 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
       for (int r = 0; r < 2 * Pmax - 1; ++r) {
         {
           ProfScope ps(c, 1);
-          HIPCHK(c, launch_jacobi_round(d_t, nb, Pmax, within, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count,
+          HIPCHK(c, launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count,
                                         c->wl_items, c->wl_cap, c->st));
         }
         ProfScope ps(c, 5);

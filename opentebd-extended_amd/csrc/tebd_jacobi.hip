@@ -165,6 +165,7 @@ __host__ __device__ constexpr int level_q(int h, int r, int t) {
 // The schedules: kCross the 16 rounds of level 16 (pair t's next entry lies in block (t, t + 1),
 // the last one's in block (0, 15)), kFull the 15 rounds of levels 8, 4, 2, 1 and then kCross.
 constexpr int kWithinRounds = JB - 1;
+constexpr int kWithinRows = 512;
 using CrossTable = InnerTable<JB, 2 * kInnerPairs>;
 using FullTable = InnerTable<kAllRounds, 2 * kOffBlocks>;
 template <class Table>
@@ -193,8 +194,12 @@ __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 // Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
 // sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
 // blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
-// includes the blocks' own couplings, the pairs within the blocks too, in two passes (and in every
-// round of a batch that fills the GPU with long columns, where sweeps cost more than rounds).
+// includes the blocks' own couplings, the pairs within the blocks too, in two passes.  So do all
+// rounds of a bond with more than kWithinRows rows: its Grams and rotations of W cost more than the
+// rounds, and a sixth fewer sweeps pays once the batch fills the GPU.  Hubbard, exact SVDs, ms per
+// step without and with it: L = 128, chi = 256 206 and 192; L = 32, chi = 256 121 and 127; L = 24, chi
+// = 200 86 and 94; below the bound L = 64, chi = 128 47 and 51, the number-conserving blocks of L =
+// 128, chi = 256 77 and 84.  The bound looks at the bond alone, so that no result depends on the batch.
 // Measured on Hubbard and Bose-Hubbard bonds (numpy restatement, 225 x 225 and 256 x 256):
 // 6 outer sweeps and 1300-1400 inner rounds in sequence per solve; three cyclic sweeps over
 // all 496 pairs per visit take 5 outer sweeps but 4400-4650 rounds in sequence.
@@ -303,7 +308,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
   }
 }
 
-template <bool FULL, bool WITHIN>
+template <bool FULL>
 __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* __restrict__ tasks, int sweep, int round,
                                                       double tol_rel, double tol_abs, int* __restrict__ wl_count,
                                                       int2* __restrict__ wl_items, int wl_cap) {
@@ -339,14 +344,16 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   // on a CU instead of two) is read from L2 one round ahead.  With it in LDS the exact step of Hubbard
   // L = 128, chi = 256 took 204 ms instead of 192 and the number-conserving one of L = 64, chi = 128
   // 15.8 instead of 15.2.
-  __shared__ typename std::conditional<WITHIN, int, decltype(CrossTable::rounds)>::type table;
+  __shared__ typename std::conditional<FULL, int, decltype(CrossTable::rounds)>::type table;
   __shared__ int s_flag;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const zc* Wi = t.W + (size_t)t.R * (bi * JB);
   const zc* Wj = t.W + (size_t)t.R * (bj * JB);
   if (tid == 0) s_flag = 0;
-  if constexpr (!WITHIN) load_rounds(table, kCross.rounds, tid, kRoundThreads);
+  const bool within = FULL || t.R > kWithinRows;
+  if constexpr (!FULL)
+    if (!within) load_rounds(table, kCross.rounds, tid, kRoundThreads);
 
   // ---- Gram: A = [Wi Wj]^H [Wi Wj]
   {
@@ -413,8 +420,9 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
 
   // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
   zc (*Q)[JC + 1] = sc.Q;
-  if constexpr (WITHIN) inner_jacobi<true>(A, Q, dg, rb, kFull.rounds, tid);
-  else inner_jacobi<false>(A, Q, dg, rb, table, tid);
+  if (within) inner_jacobi<true>(A, Q, dg, rb, kFull.rounds, tid);
+  if constexpr (!FULL)
+    if (!within) inner_jacobi<false>(A, Q, dg, rb, table, tid);
   zc* qg = t.Qg + (size_t)p * JC * JC;
   for (int e = tid; e < JC * JC; e += kRoundThreads) qg[e] = Q[e / JC][e % JC];  // qg[k JC + c] = Q[k][c]
   if (tid == 0) {
@@ -525,10 +533,10 @@ hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sw
   return hipGetLastError();
 }
 
-hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, bool within, int sweep, int round,
+hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
                                double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
                                int2* wl_items, int wl_cap, hipStream_t st) {
-  const auto k = round == 0 ? k_jacobi_round<true, true> : within ? k_jacobi_round<false, true> : k_jacobi_round<false, false>;
+  const auto k = round == 0 ? k_jacobi_round<true> : k_jacobi_round<false>;
   hipLaunchKernelGGL(k, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round, tol_rel, tol_abs,
                      wl_count, wl_items, wl_cap);
   return hipGetLastError();

@@ -16,8 +16,7 @@ hipError_t launch_prepare_svd(const BondTask* d_tasks, int ntasks, hipStream_t s
 hipError_t launch_frobenius(const BondTask* d_tasks, int ntasks, int max_cpad, hipStream_t st, int keep_sum);
 hipError_t launch_jacobi_begin(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sweep, int* wl_count, hipStream_t st);
-// within: every visit rotates the pairs within the two blocks too (round 0 always does).
-hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, bool within, int sweep, int round,
+hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
                                double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
                                int2* wl_items, int wl_cap, hipStream_t st);
 hipError_t launch_jacobi_rotate(const BondTask* d_tasks, int round, int max_rows_w, int max_rows_v, int* wl_count,

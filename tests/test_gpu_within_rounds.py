@@ -1,10 +1,9 @@
-"""A batch large enough that every Jacobi visit rotates the pairs within its two column blocks too.
+"""Bonds of more than 512 rows, whose Jacobi visits rotate the pairs within the column blocks too.
 
-One Trotter step of a saturated Hubbard chain (bond matrices of 800 x 800, 38 of them in a
-half-sweep on one lane: more than 256 column-block pairs) against the same step bond by bond,
-whose visits rotate the cross pairs alone.  The two states agree to the rounding of one update
-per bond and half-sweep; bound, fixed before the first run: 1e-9 on every lambda, local
-occupation and the truncation, as for all parity checks of evolved states.
+One Trotter step of a saturated Hubbard chain (bond matrices of 800 x 800) in one batch, whose
+tasks lie on both sides of that bound, against the same step bond by bond.  Bound, fixed before
+the first run: 1e-9 on every lambda and local occupation, as for all parity checks of evolved
+states.
 """
 import numpy as np
 import pytest
