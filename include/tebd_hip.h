@@ -229,8 +229,8 @@ int tebd_get_stats(tebd_ctx* ctx, double* stats, int n);
  * tebd_set_profiling(ctx, 1) clears and enables the counters;
  * tebd_get_profile fills out[4k .. 4k+3] = {launches, milliseconds, algorithmic
  * flops, algorithmic HBM bytes} of launch class k (n <= 28):
- *   0 theta + gate (k_theta_gate, or k_theta_gate_mixed in TEBD_MODE_MIXED)
- *   1 Jacobi round: pair Grams and 32x32 eigenproblems (k_jacobi_round)
+ *   0 theta + gate (k_theta_gate_mfma; k_theta_gate_mixed in TEBD_MODE_MIXED)
+ *   1 Jacobi round: pair Grams and 32x32 rotations (k_jacobi_round)
  *   2 truncation, Gamma rebuild, singular-vector and sketch formation
  *   3 pivoted-QR panel factorisation (k_qrp_panel_reg / k_qrp_panel)
  *   4 batched complex GEMMs of the learned-rank path (k_zgemm)
@@ -242,7 +242,7 @@ int tebd_set_profiling(tebd_ctx* ctx, int on);
 int tebd_get_profile(tebd_ctx* ctx, double* out, int n);
 
 /* hipGraph replay of the one-sided Jacobi sweeps (no counterpart in the reference):
- * with on = 1 (the default) each sweep's launches (sweep start, and the Gram /
+ * with on = 1 (the default) each sweep's launches of the large solves (sweep start, and the Gram /
  * eigenproblem and rotation kernels of its 2P-1 rounds) are captured once per launch
  * shape into an executable graph and replayed, instead of being launched one by one;
  * the convergence test between sweeps stays on the host.  Per-launch profiling
