@@ -196,7 +196,9 @@ int tebd_imag_time_prop(tebd_ctx* ctx, const double* H, int nh, double dtau, int
  * (l1, l2) (0-based within the chain) at index l1 Lc - l1(l1+1)/2 + (l2 - l1 - 1); row
  * i d + j, column l d + k for ket i, bra l on site l1 and ket j, bra k on site l2 (the
  * reference's rho2((i-1)d+j,(l-1)d+k)).  rho1 (host, or NULL): L matrices of d x d, element
- * i + d j (FormSingleSiteRho, :95-117).  Tr(O rho) gives any correlator or local value. */
+ * i + d j (FormSingleSiteRho, :95-117).  Tr(O rho) gives any correlator or local value.
+ * The environments of all right sites step together in a workspace of at most 4 GiB (or one
+ * site's, if that is more), allocated on the first call and freed with the context. */
 int tebd_two_point_rdms(tebd_ctx* ctx, const double* phase, double* rho2, double* rho1);
 
 /* Singular-value cutoff on the normalised weight s^2/||theta||^2.  Default
