@@ -336,8 +336,7 @@ hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int c
   if (hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
   hipError_t e = launch_jacobi_sweep_begin(d_t, nb, cls, c->wl_count, c->st);
   for (int r = 0; r < 2 * Pmax - 1 && e == hipSuccess; ++r) {
-    e = launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count, c->wl_items,
-                            c->wl_cap, c->st);
+    e = launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, c->wl_count, c->wl_items, c->wl_cap, c->st);
     if (e == hipSuccess)
       e = launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st);
   }
@@ -351,16 +350,12 @@ hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int c
   return ge;
 }
 
-// Tasks solved by k_jacobi_small: bond matrices of at most 2 pairs of column blocks that skip
-// the QR preconditioning.
-bool small_solve(const BondTask& t) { return !t.qr && t.P <= kSmallPairs; }
-
 // After the tasks' counters have reached h_counters: checks that the small solves converged
 // and adds every task's work to the statistics.  `sweeps`: sweeps of the large solves, which
 // have already entered their rotations per sweep.
 int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, int sweeps, bool converged) {
   for (int i = 0; i < nb; ++i) {
-    if (!small_solve(h_t[i])) continue;
+    if (!h_t[i].small) continue;
     const int* cnt = c->h_counters + kCounters * i;
     if (cnt[4] < 1) converged = false;
     sweeps = std::max(sweeps, cnt[4]);
@@ -374,8 +369,8 @@ int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, int sweeps, bool co
     const double rows = t.R + (t.V ? t.NV : 0);
     c->stats[8] += visits;
     c->stats[9] += rots;
-    c->stats[10] += (double)(small_solve(t) ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
-    if (c->profiling && !small_solve(t)) {
+    c->stats[10] += (double)(t.small ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
+    if (c->profiling && !t.small) {
       // k_jacobi_round, per formed Gram: the 16x16 cross block over R rows (8 flops per
       // complex MAC) reading the pair's JC columns once, and per rotated pair its JC x JC
       // rotation written; k_jacobi_rotate, per rotated pair: the JC columns of W and V
@@ -403,7 +398,7 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
   int rows_w = 1, rows_v = 0, Pmax = 0;
   bool one = false, two = false;
   for (int i = 0; i < nb; ++i) {
-    if (small_solve(h_t[i])) {
+    if (h_t[i].small) {
       (h_t[i].P == 1 ? one : two) = true;
       continue;
     }
@@ -450,8 +445,8 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
       for (int r = 0; r < 2 * Pmax - 1; ++r) {
         {
           ProfScope ps(c, 1);
-          HIPCHK(c, launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, rows_w, rows_v, c->wl_count,
-                                        c->wl_items, c->wl_cap, c->st));
+          HIPCHK(c, launch_jacobi_round(d_t, nb, Pmax, cls, r, kTolRel, kTolAbs, c->wl_count, c->wl_items, c->wl_cap,
+                                        c->st));
         }
         ProfScope ps(c, 5);
         HIPCHK(c, launch_jacobi_rotate(d_t, r, rows_w, rows_v, c->wl_count, c->wl_items, c->wl_cap, c->st));
@@ -502,7 +497,7 @@ int qrp_factor(tebd_ctx* c, BondTask* D, const BondTask* H, int nb, int max_cb, 
   for (int j0 = 0, panel = 0; !done; j0 += kQrPanel, ++panel) {
     {
       ProfScope ps(c, 3);
-      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, max_cb, j0, c->st));
+      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, max_cb, j0, H[0].cyclic != 0, c->st));
     }
     {
       ProfScope ps(c, 6);
@@ -557,7 +552,7 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
   // which other bonds share its batch.
   std::vector<int> qidx;
   for (int i = 0; i < nb; ++i)
-    if (force_qr || H[i].Rb >= kQrMinSide) qidx.push_back(i);
+    if (force_qr || (H[i].cyclic ? H[i].Cb : H[i].Rb) >= kQrMinSide) qidx.push_back(i);
   const int nq = (int)qidx.size();
   const bool use_qr = nq > 0;
   int max_rank = 1;
@@ -585,6 +580,7 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
       max_rank = std::max(max_rank, rank[j]);
       BondTask& t = H[i];
       t.qr = 1;
+      t.small = 0;
       t.W = c->X + (size_t)slot_of(c, t) * c->Cpmax * c->Cpmax;
       t.R = t.Cb;
       t.C = rank[j];
@@ -729,6 +725,7 @@ void make_full_task(tebd_ctx* c, BondTask& t, int link, const zc* gate, int slot
   t.C = std::min(m, n);
   t.Cpad = round_up(t.C, JC);
   t.P = t.Cpad / JC;
+  t.small = t.R < kQrMinSide;
   t.gl = c->gam + (size_t)link * c->gslab();
   t.gr = c->gam + (size_t)(link + 1) * c->gslab();
   t.ll = c->lam + (size_t)link * c->chi_max;
@@ -1182,6 +1179,7 @@ int device_svd_batch(tebd_ctx* c, const SvdJob* jobs, int nb) {
     BondTask& t = c->h_tasks[i];
     std::memset(&t, 0, sizeof(t));
     t.W = jobs[i].W; t.R = jobs[i].R; t.C = jobs[i].C; t.Cpad = round_up(t.C, JC); t.P = t.Cpad / JC;
+    t.small = t.P <= kSmallPairs;
     t.V = jobs[i].V; t.NV = t.Cpad; t.s = jobs[i].s; t.perm = jobs[i].perm;
     attach_jacobi(c, t, i);
     t.result = c->results + (size_t)RESULT_STRIDE * i;
@@ -1595,6 +1593,7 @@ int run_bonds_nc(tebd_ctx* c, const int* links, int nb, const zc* const* gate_pt
         BondTask& t = S[q];
         std::memset(&t, 0, sizeof(t));
         t.d = d;
+        t.cyclic = 1;
         t.link = links[blk_bond[live[q0 + q]]];
         t.R = b.R;
         t.C = std::min(b.lgt, b.trv);
@@ -1622,7 +1621,7 @@ int run_bonds_nc(tebd_ctx* c, const int* links, int nb, const zc* const* gate_pt
       HIPCHK(c, launch_nc_gather(c->d_nc_blk, n, c->d_nc_part, w->st));
       bool used_qr = false;
       int max_k = 1;
-      int ef = svd_factor(w, DS, S, err_links.data(), n, Cpm, true, &used_qr, &max_k);
+      int ef = svd_factor(w, DS, S, err_links.data(), n, Cpm, false, &used_qr, &max_k);
       if (!ef) {
         HIPCHK(c, launch_nc_vectors(c->d_nc_blk, DS, n, max_k, w->st));
         HIPCHK(c, hipMemcpyAsync(w->h_nc_s, w->s, sizeof(double) * w->Cpmax * n, hipMemcpyDeviceToHost, w->st));
@@ -3131,6 +3130,7 @@ int tebd_two_site_op_noalloc(int d, int chi_l, int chi_c, int chi_r, int chi_cap
   t.C = std::min(m, n);
   t.Cpad = round_up(t.C, JC);
   t.P = t.Cpad / JC;
+  t.small = t.R < kQrMinSide;
   t.gl = (const zc*)gamma_l;
   t.gr = (const zc*)gamma_r;
   t.ll = lambda_l;

@@ -231,6 +231,9 @@ struct BondTask {
   // column-pivoted QR preconditioning (qr = 1): Wq (Rb x Cb) holds the bond matrix and then its
   // Householder QR; the Jacobi (W, R, C above) runs on X = R(0:r, :)^dagger (Cb x r)
   int qr;
+  int cyclic;        // 1: every pair visit of the Jacobi runs whole cyclic sweeps (inner_solve) and a QR
+                     // panel reduces a column's norm by itself (reflectors_of_norm)
+  int small;         // 1: the whole Jacobi solve in one launch (tebd_jacobi_small.hip); P <= kSmallPairs
   int Rb, Cb;
   zc* Wq;
   double* qnrm;      // Cb remaining column norms^2
@@ -244,3 +247,5 @@ struct BondTask {
   const double* wtot;  // when set, the reference total weight (||theta||^2) for the truncation
   int rng_key;       // sketch stream of the bond: its position in its chain (not its batch slot)
 };
+
+constexpr int kSmallPairs = 2;  // most pairs of column blocks of a small solve

@@ -6,24 +6,28 @@
 // other (round-robin "circle" order, 2P-1 rounds per sweep).  A round is two kernels:
 //   k_jacobi_round   one workgroup per pair: the pair's Gram matrix on FP64 MFMA
 //                    (v_mfma_f64_16x16x4f64), the decision whether it needs a
-//                    rotation, and one pass of rotations over its index pairs in LDS
-//                    (tebd_jacobi_inner.h) -> Q (32x32, to global memory); rotated pairs are
+//                    rotation, and rotations over its index pairs in LDS -> Q (32x32, to
+//                    global memory): one pass (inner_jacobi) or the whole 32x32 problem by
+//                    cyclic sweeps (inner_solve, tebd_jacobi_inner.h); rotated pairs are
 //                    queued;
 //   k_jacobi_rotate  [W; V](:, pair) <- [W; V](:, pair) Q for every queued pair, on
 //                    MFMA, spread over 64-row slabs so a rotation costs one memory
 //                    round trip of the whole GPU instead of one workgroup's stream.
 // Only the first round of a sweep forms the full Gram of each pair and rotates the pairs
 // within the blocks too; the other rounds form the 16x16 cross block and the 32 column norms
-// (4x less Gram work), take the columns of a block as orthogonal and rotate the cross pairs
-// once.  With a strongly graded spectrum the rounding of rotations lets the small columns of
-// a block drift away from orthogonality, and the first round restores it (a cross-only
-// iteration does not converge there).
+// (4x less Gram work), take the columns of a block as orthogonal and, where a visit is one
+// pass, rotate the cross pairs once.  With a strongly graded spectrum the rounding of rotations
+// lets the small columns of a block drift away from orthogonality, and the first round restores
+// it (a cross-only iteration does not converge there).
 //
 // A pair visit is bound by the latency of its rounds of rotations: three cyclic sweeps over
 // all index pairs per visit (93 rounds, two barriers each) took 59 us at 400 x 400
 // (Fermi-Hubbard, chi = 100) and 54 at 225 x 225 (Bose-Hubbard, chi = 45); one pass over the
 // cross pairs (16 rounds of one barrier) takes 16 and 14, for 6 to 7 outer sweeps instead of 5
-// to 6.
+// to 6.  Whole cyclic sweeps per visit stay for tasks that say so (BondTask::cyclic).  The number
+// blocks' Schmidt values are cut at 1e-10, where another rounding keeps another state: with one pass a
+// Fermi-Hubbard chain of 64 sites, chi = 128, gave lambda up to 8e-9 from what cyclic sweeps give
+// (its step takes 14.5 ms so and 19.6 with them).
 //
 // Work that cannot change the result is skipped exactly:
 //   * a task whose previous sweep rotated nothing has converged: its workgroups exit;
@@ -41,116 +45,9 @@
 
 namespace {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-// D(16x16) += A(16x4) B(4x16).  Lane l supplies A[l%16][l/16] and B[l/16][l%16];
-// element g of the result in lane l is D[l/16 + 4g][l%16].
-__device__ __forceinline__ d4 mfma4(double a, double b, d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // k_jacobi_round runs 8 waves: all of them form the Gram matrix; in the inner solve
 // waves 0-3 update A and waves 4-7 the rotation accumulator Q.
-constexpr int kRoundThreads = 512;
-constexpr int kGramWaves = kRoundThreads / 64;
-
-// Round-robin ("circle") schedule over nb = 2P blocks: block 0 stays, the others
-// rotate; over nb-1 rounds every pair of blocks meets exactly once.
-__device__ __forceinline__ void rr_pair(int nb, int round, int p, int& bi, int& bj) {
-  auto pos = [&](int k) { return k == 0 ? 0 : 1 + (k - 1 + round) % (nb - 1); };
-  bi = pos(p);
-  bj = pos(nb - 1 - p);
-}
-
-// Hermitian 2x2 Jacobi rotation J = [[c, s w], [-s conj(w), c]], w = g/|g|, that
-// zeroes g in [[a, g], [conj(g), b]] via J^dagger H J, with the inner angle
-// (|theta| <= pi/4, Rutishauser's smaller root).  tan theta = t = 2|g| sign(b - a) /
-// (|b - a| + sqrt((b - a)^2 + 4|g|^2)); t w is formed without |g|.  The hardware
-// estimates of the square root and the quotient (about 2^-24, one Newton-Raphson step on
-// the quotient) suffice for t: an angle that is off by 1e-7 of itself leaves 1e-7 of
-// the coupling for the next sweep.  c = 1/sqrt(1 + t^2) is refined to full precision (two
-// steps) and s = c t, so the rotation is unitary to rounding whatever t's error.
-// a and b become the rotated diagonal a - t|g|, b + t|g|.
-__device__ __forceinline__ void jrot(double& a, double& b, zc g, double g2, double& c, zc& sw) {
-  const double dd = b - a;
-  const double e2 = fma(dd, dd, 4.0 * g2);
-  const double den = fma(e2, __builtin_amdgcn_rsq(e2), fabs(dd));
-  double inv = __builtin_amdgcn_rcp(den);
-  inv = inv * fma(-den, inv, 2.0);
-  const double f = dd < 0.0 ? -2.0 * inv : 2.0 * inv;
-  const double tx = f * g.x, ty = f * g.y;
-  const double h = fma(tx, tx, fma(ty, ty, 1.0));
-  double r = __builtin_amdgcn_rsq(h);
-  const double hh = 0.5 * h;
-  r = r * fma(-hh * r, r, 1.5);
-  r = r * fma(-hh * r, r, 1.5);
-  c = r;
-  sw = zmk(tx * r, ty * r);
-  a = fma(-f, g2, a);
-  b = fma(f, g2, b);
-}
-
-// Gram block D = X^H Y (16 x 16) of two 16-column blocks over rows [0, R), as
-// per-wave partial sums of kGramWaves waves: wave w takes rows 8 (w + kGramWaves m)
-// .. +7, m = 0, 1, ..., each in two MFMA k-steps of 4 rows, with the loads of two
-// consecutive m issued before their MFMAs (the pass is bound by memory latency).  Also
-// accumulates the lane's partial squared norms of X and Y.
-__device__ __forceinline__ void gram_block(const zc* __restrict__ X, const zc* __restrict__ Y, int R, int wave,
-                                           int lane, d4& gre, d4& gim, double& nx, double& ny) {
-  constexpr int U = 2;
-  const int lr = lane & 15, lk = lane >> 4;
-  gre = d4{0.0, 0.0, 0.0, 0.0};
-  gim = d4{0.0, 0.0, 0.0, 0.0};
-  nx = 0.0;
-  ny = 0.0;
-  const zc* xc = X + (size_t)R * lr;
-  const zc* yc = Y + (size_t)R * lr;
-  constexpr int PER = 8 * kGramWaves;  // rows per period: 8 of them for each wave
-  for (int r0 = 8 * wave; r0 < R; r0 += PER * U) {
-    zc a[2 * U], b[2 * U];
-#pragma unroll
-    for (int u = 0; u < 2 * U; ++u) {
-      const int r = r0 + PER * (u >> 1) + 4 * (u & 1) + lk;
-      a[u] = r < R ? xc[r] : zmk(0.0, 0.0);
-      b[u] = r < R ? yc[r] : zmk(0.0, 0.0);
-    }
-#pragma unroll
-    for (int u = 0; u < 2 * U; ++u) {
-      // A[p][k] = conj(X[k][p]), B[k][q] = Y[k][q]
-      gre = mfma4(a[u].x, b[u].x, gre);
-      gre = mfma4(a[u].y, b[u].y, gre);
-      gim = mfma4(a[u].x, b[u].y, gim);
-      gim = mfma4(-a[u].y, b[u].x, gim);
-      nx += zabs2(a[u]);
-      ny += zabs2(b[u]);
-    }
-  }
-}
-
-// Sums the Gram waves' partial 16x16 blocks in a fixed order (bitwise reproducible)
-// and stores rows [ro, ro+16) x cols [co, co+16) of the upper triangle of A (diagonal
-// blocks: the real diagonal goes to dg).  Every thread sums one real or imaginary part from
-// the scratch `red`, which shares its storage with the rotation accumulator.  Called by
-// every thread of the workgroup.
-__device__ __forceinline__ void reduce_block(zc (*A)[kInnerLd], double* dg, double (*red)[512], d4 gre, d4 gim, int wave,
-                                             int lane, int ro, int co, bool diag) {
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    red[wave][g * 64 + lane] = gre[g];
-    red[wave][256 + g * 64 + lane] = gim[g];
-  }
-  __syncthreads();
-  {
-    const int e = threadIdx.x, idx = e & 255, l = idx & 63, im = e >> 8;
-    double v = red[0][e];
-    for (int w = 1; w < kGramWaves; ++w) v += red[w][e];
-    const int p = (l >> 4) + 4 * (idx >> 6), q = l & 15;
-    if (!diag || p < q) reinterpret_cast<double*>(&A[ro + p][co + q])[im] = v;
-    else if (p == q && !im) dg[ro + p] = v;
-  }
-  __syncthreads();
-}
-
+constexpr int kRoundThreads = kPairThreads;
 static_assert(kRoundThreads == 512 && JB == kInnerPairs, "the inner solve's thread roles");
 
 // Index pair t (t < 16) of round r of level h (h = 1, 2, 4, 8 or 16): the 32 indices in
@@ -191,6 +88,32 @@ constexpr Table level_table(int first_level) {
 __device__ constexpr CrossTable kCross = level_table<CrossTable>(4);
 __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 
+// The rotation that zeroes g in [[a, g], [conj(g), b]], as jrot's: tan theta = t = 2|g| sign(b - a) /
+// (|b - a| + sqrt((b - a)^2 + 4|g|^2)); t w is formed without |g|.  The hardware
+// estimates of the square root and the quotient (about 2^-24, one Newton-Raphson step on
+// the quotient) suffice for t: an angle that is off by 1e-7 of itself leaves 1e-7 of
+// the coupling for the next sweep.  c = 1/sqrt(1 + t^2) is refined to full precision (two
+// steps) and s = c t, so the rotation is unitary to rounding whatever t's error.
+// a and b become the rotated diagonal a - t|g|, b + t|g|.
+__device__ __forceinline__ void pass_rotation(double& a, double& b, zc g, double g2, double& c, zc& sw) {
+  const double dd = b - a;
+  const double e2 = fma(dd, dd, 4.0 * g2);
+  const double den = fma(e2, __builtin_amdgcn_rsq(e2), fabs(dd));
+  double inv = __builtin_amdgcn_rcp(den);
+  inv = inv * fma(-den, inv, 2.0);
+  const double f = dd < 0.0 ? -2.0 * inv : 2.0 * inv;
+  const double tx = f * g.x, ty = f * g.y;
+  const double h = fma(tx, tx, fma(ty, ty, 1.0));
+  double r = __builtin_amdgcn_rsq(h);
+  const double hh = 0.5 * h;
+  r = r * fma(-hh * r, r, 1.5);
+  r = r * fma(-hh * r, r, 1.5);
+  c = r;
+  sw = zmk(tx * r, ty * r);
+  a = fma(-f, g2, a);
+  b = fma(f, g2, b);
+}
+
 // Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
 // sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
 // blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
@@ -198,8 +121,8 @@ __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 // rounds of a bond with more than kWithinRows rows: its Grams and rotations of W cost more than the
 // rounds, and a sixth fewer sweeps pays once the batch fills the GPU.  Hubbard, exact SVDs, ms per
 // step without and with it: L = 128, chi = 256 206 and 192; L = 32, chi = 256 121 and 127; L = 24, chi
-// = 200 86 and 94; below the bound L = 64, chi = 128 47 and 51, the number-conserving blocks of L =
-// 128, chi = 256 77 and 84.  The bound looks at the bond alone, so that no result depends on the batch.
+// = 200 86 and 94; below the bound L = 64, chi = 128 47 and 51.  The bound looks at the bond alone, so
+// that no result depends on the batch.
 // Measured on Hubbard and Bose-Hubbard bonds (numpy restatement, 225 x 225 and 256 x 256):
 // 6 outer sweeps and 1300-1400 inner rounds in sequence per solve; three cyclic sweeps over
 // all 496 pairs per visit take 5 outer sweeps but 4400-4650 rounds in sequence.
@@ -207,8 +130,11 @@ __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 // of a 16-lane row has two rows' entries at p_t, which stays, and q_t, which comes from the next
 // lane in every round), in the other levels in LDS.
 template <bool FULL, class Rounds>
-__device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1], double* dg, RotBuf* rb, const Rounds& T,
-                                             int tid) {
+__device__ __forceinline__ void inner_jacobi(PairLds& L, const Rounds& T, int tid) {
+  zc (*A)[kInnerLd] = L.A;
+  zc (*Q)[JC + 1] = L.Q;
+  double* dg = L.dg;
+  RotBuf* rb = L.rb;
   constexpr int NN = FULL ? 2 * kOffBlocks : 2 * kInnerPairs, RW = FULL ? kWithinRounds : 0;
   const bool is_a = tid < 2 * kOffBlocks, is_q = tid >= 256;
   const int tr = is_a ? kCross.tr[tid] : 0, tk = is_a ? kCross.tk[tid] : 0, half = tid & 1;
@@ -228,7 +154,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
   for (int pass = 0; pass < (FULL ? 2 : 1); ++pass) {
     if (tid < kInnerPairs) {
       const int p = level_p(FULL ? 8 : 16, tid), q = level_q(FULL ? 8 : 16, 0, tid);
-      A[p][q] = make_rotation(rb[buf], dg[p], dg[q], &dg[p], &dg[q], nullptr, tid, A[p][q], jrot);
+      A[p][q] = make_rotation(rb[buf], dg[p], dg[q], &dg[p], &dg[q], nullptr, tid, A[p][q], pass_rotation);
     }
     __syncthreads();
     if (FULL) {
@@ -241,7 +167,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
           const RotBuf& R = rb[buf];
           if (is_a) {
             const unsigned e1 = T.entry[rd + 1][tid], n1 = T.next[rd + 1][tid];
-            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
+            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, pass_rotation);
             entry = e1;
             next = n1;
           } else if (is_q) {
@@ -276,7 +202,7 @@ __device__ __forceinline__ void inner_jacobi(zc (*A)[kInnerLd], zc (*Q)[JC + 1],
           e1 = T.entry[ahead][tid];
           n1 = T.next[ahead][tid];
         }
-        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
+        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, pass_rotation);
         if (!FULL) {
           e1 = T.entry[ahead][tid];
           if (tid < NN) n1 = T.next[ahead][tid];
@@ -315,7 +241,7 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   const BondTask t = tasks[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= t.P || round >= 2 * t.P - 1) return;
-  if (!t.qr && t.P <= kSmallPairs) return;  // solved by k_jacobi_small
+  if (t.small) return;  // solved by k_jacobi_small
   int* cnt = t.counter;
   if (sweep > 0 && cnt[(sweep - 1) & 1] == 0) return;  // converged in the previous sweep
   const int nblk = 2 * t.P;
@@ -327,89 +253,74 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   unsigned long long* seen = t.pairseen + (size_t)lo * nblk + hi;
   if (!FULL && *seen == stamp) return;  // unchanged since it was verified orthogonal
 
-  __shared__ zc A[JC][kInnerLd];  // the pair's Gram matrix: its upper triangle; its diagonal is in dg
-  __shared__ double dg[JC];
-  // The rotation accumulator Q; until the inner solve starts, its storage holds the
-  // Gram's reduction scratch (red) and the column-norm partials (nred).
-  union Scratch {
-    zc Q[JC][JC + 1];
-    struct {
-      double red[kGramWaves][512];
-      double nred[kGramWaves][2][16];
-    } g;
-  };
-  __shared__ Scratch sc;
-  __shared__ RotBuf rb[2];
-  // The schedule of 16 rounds lies in LDS; that of 31 (60 KB, which would leave room for one workgroup
-  // on a CU instead of two) is read from L2 one round ahead.  With it in LDS the exact step of Hubbard
-  // L = 128, chi = 256 took 204 ms instead of 192 and the number-conserving one of L = 64, chi = 128
-  // 15.8 instead of 15.2.
+  // The schedule of 16 rounds lies in LDS; those of 31 (60 and 34 KB, which would leave room for one
+  // workgroup on a CU instead of two) are read from L2 one round ahead.  With the longer one in LDS the
+  // exact step of Hubbard L = 128, chi = 256 took 204 ms instead of 192.
+  __shared__ PairLds L;
   __shared__ typename std::conditional<FULL, int, decltype(CrossTable::rounds)>::type table;
-  __shared__ int s_flag;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const zc* Wi = t.W + (size_t)t.R * (bi * JB);
   const zc* Wj = t.W + (size_t)t.R * (bj * JB);
-  if (tid == 0) s_flag = 0;
-  const bool within = FULL || t.R > kWithinRows;
+  if (tid == 0) L.need = 0;
+  const bool cyclic = t.cyclic, within = FULL || t.R > kWithinRows;
   if constexpr (!FULL)
-    if (!within) load_rounds(table, kCross.rounds, tid, kRoundThreads);
+    if (!cyclic && !within) load_rounds(table, kCross.rounds, tid, kRoundThreads);
 
   // ---- Gram: A = [Wi Wj]^H [Wi Wj]
   {
     d4 gre, gim;
     double nx, ny;
-    auto gram = [&](const zc* X, const zc* Y) { gram_block(X, Y, t.R, wave, lane, gre, gim, nx, ny); };
-    gram(Wi, Wj);
+    gram_block(Wi, Wj, t.R, wave, lane, gre, gim, nx, ny);
     if (!FULL) {
       nx += __shfl_xor(nx, 16, 64);
       nx += __shfl_xor(nx, 32, 64);
       ny += __shfl_xor(ny, 16, 64);
       ny += __shfl_xor(ny, 32, 64);
       if (lane < 16) {
-        sc.g.nred[wave][0][lane] = nx;
-        sc.g.nred[wave][1][lane] = ny;
+        L.g.nred[wave][0][lane] = nx;
+        L.g.nred[wave][1][lane] = ny;
       }
       // within-block entries: zero (the blocks' columns are nearly orthogonal)
       {
         const int blk = tid / (JB * JB), r = (tid / JB) % JB, c = tid % JB;
-        A[blk * JB + r][blk * JB + c] = zmk(0.0, 0.0);
+        L.A[blk * JB + r][blk * JB + c] = zmk(0.0, 0.0);
       }
     }
-    reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, 0, JB, false);
+    reduce_block(L, true, gre, gim, tid, 0, JB, false);
     if (FULL) {
-      gram(Wi, Wi);
-      reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, 0, 0, true);
-      gram(Wj, Wj);
-      reduce_block(A, dg, sc.g.red, gre, gim, wave, lane, JB, JB, true);
+      gram_block(Wi, Wi, t.R, wave, lane, gre, gim, nx, ny);
+      reduce_block(L, true, gre, gim, tid, 0, 0, true);
+      gram_block(Wj, Wj, t.R, wave, lane, gre, gim, nx, ny);
+      reduce_block(L, true, gre, gim, tid, JB, JB, true);
     } else {
       if (tid < JC) {
         const int side = tid / JB, col = tid % JB;
         double v = 0.0;
-        for (int w = 0; w < kGramWaves; ++w) v += sc.g.nred[w][side][col];
-        dg[tid] = v;
+        for (int w = 0; w < kPairWaves; ++w) v += L.g.nred[w][side][col];
+        L.dg[tid] = v;
       }
       __syncthreads();
     }
   }
 
   // ---- does this pair need a rotation?  |A_pq| > tol_rel sqrt(A_pp A_qq) and
-  // |A_pq| > tol_abs max_c|w_c| (|w_p| + |w_q|).  The second bound is the rounding
-  // floor: rotations add errors of order eps * sigma_max to every column they touch.
+  // |A_pq| > tol_abs max_c|w_c| (|w_p| + |w_q|): the second bound is the
+  // rounding floor of the rotations in the |w_c|-sized columns of W
   {
-    const double fnorm = sqrt(t.result[2]);  // largest column norm
+    const double floor = tol_abs * sqrt(t.result[2]);  // of the largest column norm
     int need = 0;
     for (int e = tid; e < (FULL ? JC * JC : JB * JB); e += kRoundThreads) {
       const int pp = FULL ? e % JC : e % JB, qq = FULL ? e / JC : JB + e / JB;
       if (pp >= qq) continue;
-      const double g2 = zabs2(A[pp][qq]);
-      const double app = fmax(dg[pp], 0.0), aqq = fmax(dg[qq], 0.0);
-      const double fl = tol_abs * fnorm * (sqrt(app) + sqrt(aqq));
+      const double g2 = abs2(L.A[pp][qq]);
+      const double app = fmax(L.dg[pp], 0.0), aqq = fmax(L.dg[qq], 0.0);
+      const double fl = floor * (sqrt(app) + sqrt(aqq));
       if (g2 > tol_rel * tol_rel * app * aqq && g2 > fl * fl) need = 1;
     }
-    if (need) s_flag = 1;
+    if (need) L.need = 1;
     __syncthreads();
-    if (!s_flag) {
+    if (!L.need) {
       if (tid == 0) {
         *seen = stamp;
         atomicAdd(&cnt[2], 1);
@@ -419,10 +330,10 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   }
 
   // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
-  zc (*Q)[JC + 1] = sc.Q;
-  if (within) inner_jacobi<true>(A, Q, dg, rb, kFull.rounds, tid);
-  if constexpr (!FULL)
-    if (!within) inner_jacobi<false>(A, Q, dg, rb, table, tid);
+  if (cyclic) inner_solve<true>(L, kRing.rounds, tid, true);
+  else if (within) inner_jacobi<true>(L, kFull.rounds, tid);
+  else if constexpr (!FULL) inner_jacobi<false>(L, table, tid);
+  zc (*Q)[JC + 1] = L.Q;
   zc* qg = t.Qg + (size_t)p * JC * JC;
   for (int e = tid; e < JC * JC; e += kRoundThreads) qg[e] = Q[e / JC][e % JC];  // qg[k JC + c] = Q[k][c]
   if (tid == 0) {
@@ -534,8 +445,8 @@ hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sw
 }
 
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
-                               double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
-                               int2* wl_items, int wl_cap, hipStream_t st) {
+                               double tol_rel, double tol_abs, int* wl_count, int2* wl_items, int wl_cap,
+                               hipStream_t st) {
   const auto k = round == 0 ? k_jacobi_round<true> : k_jacobi_round<false>;
   hipLaunchKernelGGL(k, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round, tol_rel, tol_abs,
                      wl_count, wl_items, wl_cap);

@@ -17,18 +17,18 @@ hipError_t launch_frobenius(const BondTask* d_tasks, int ntasks, int max_cpad, h
 hipError_t launch_jacobi_begin(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sweep, int* wl_count, hipStream_t st);
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
-                               double tol_rel, double tol_abs, int max_rows_w, int max_rows_v, int* wl_count,
-                               int2* wl_items, int wl_cap, hipStream_t st);
+                               double tol_rel, double tol_abs, int* wl_count, int2* wl_items, int wl_cap,
+                               hipStream_t st);
 hipError_t launch_jacobi_rotate(const BondTask* d_tasks, int round, int max_rows_w, int max_rows_v, int* wl_count,
                                 int2* wl_items, int wl_cap, hipStream_t st);
-// The whole solve of every task without QR preconditioning and with at most two pairs
-// (BondTask::P <= 2), one launch per pair count present in the batch.
-constexpr int kSmallPairs = 2;
+// The whole solve of every task with BondTask::small, one launch per pair count present in the batch.
 hipError_t launch_jacobi_small(const BondTask* d_tasks, int ntasks, bool one_pair, bool two_pairs, double tol_rel,
                                double tol_abs, int max_sweeps, hipStream_t st);
 hipError_t launch_qrp_trailing(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, hipStream_t st);
 hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, double tol_rel, hipStream_t st);
-hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, hipStream_t st);
+// cyclic: BondTask::cyclic of every task of the batch.
+hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, bool cyclic,
+                            hipStream_t st);
 hipError_t launch_qrp_build_x(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_qrp_vectors(const BondTask* d_tasks, int ntasks, int max_k, int max_r, hipStream_t st);
 hipError_t launch_qrp_form_q(const BondTask* d_tasks, int ntasks, int max_r, hipStream_t st);

@@ -213,70 +213,109 @@ __device__ void form_t(const zc (*G)[QB + 1], const zc* stau, int nbp, zc* Tp, z
   for (int e = lane; e < QB * QB; e += 64) Tp[e] = Tm[e % QB][e / QB];
 }
 
+// The same T column by column: T[q][q] = tau_q, T[0:q, q] = -tau_q T[0:q, 0:q] G[0:q, q].  Thread
+// p < QB forms row p, which only involves row p's own earlier entries, in registers.
+__device__ void form_t_rows(const zc (*G)[QB + 1], const zc* stau, int nbp, zc* Tp) {
+  __syncthreads();  // G and stau are complete
+  if (threadIdx.x >= QB) return;
+  const int pp = threadIdx.x;
+  zc row[QB];
+#pragma unroll
+  for (int q = 0; q < QB; ++q) row[q] = zmk(0.0, 0.0);
+  if (pp < nbp) {
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+      if (q == pp) row[q] = stau[q];
+      if (q > pp && q < nbp) {
+        zc acc = zmk(0.0, 0.0);
+#pragma unroll
+        for (int kk = 0; kk < QB; ++kk)
+          if (kk >= pp && kk < q) zfma(acc, row[kk], G[kk][q]);
+        row[q] = zmul(zmk(-stau[q].x, -stau[q].y), acc);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < QB; ++q) Tp[pp + QB * q] = row[q];
+}
+
 // Householder scalars of the column (alpha; x) with |x|^2 = xn2 (xLARFG convention):
 // H^H (alpha; x) = (beta; 0) with H = I - tau v v^H, v = (1; x * scale).  Returns false
-// (tau = 0, H = I) when the column is already (real alpha; 0).
+// (tau = 0, H = I) when the column is already (real alpha; 0).  DIV: by quotients instead of the
+// reciprocals of beta and |alpha - beta|^2.
+template <bool DIV>
 __device__ __forceinline__ bool householder(zc alpha, double xn2, zc& tau, double& beta, zc& scale) {
   tau = zmk(0.0, 0.0);
   if (xn2 == 0.0 && alpha.y == 0.0) return false;
   const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
   beta = alpha.x >= 0.0 ? -nrm : nrm;
-  const double ib = 1.0 / beta;
-  tau = zmk((beta - alpha.x) * ib, -alpha.y * ib);
   const zc am = zmk(alpha.x - beta, alpha.y);
-  const double id = 1.0 / zabs2(am);
-  scale = zmk(am.x * id, -am.y * id);
+  if constexpr (DIV) {
+    tau = zmk((beta - alpha.x) / beta, -alpha.y / beta);
+    const double den = zabs2(am);
+    scale = zmk(am.x / den, -am.y / den);
+  } else {
+    const double ib = 1.0 / beta, id = 1.0 / zabs2(am);
+    tau = zmk((beta - alpha.x) * ib, -alpha.y * ib);
+    scale = zmk(am.x * id, -am.y * id);
+  }
   return true;
 }
 
-// The number of the n keys (LDS, n a multiple of 8) above `mine`.
-__device__ inline int count_above(const unsigned long long* key, int n, unsigned long long mine) {
+// The number of the n keys (LDS, n a multiple of 8) that come before key c = `mine`: the larger
+// ones, and the equal ones below c.
+__device__ inline int count_before(const unsigned long long* key, int n, unsigned long long mine, int c) {
   int rank = 0;
   for (int k = 0; k < n; k += 8) {
     unsigned long long u[8];
 #pragma unroll
     for (int x = 0; x < 8; ++x) u[x] = key[k + x];
 #pragma unroll
-    for (int x = 0; x < 8; ++x) rank += u[x] > mine ? 1 : 0;
+    for (int x = 0; x < 8; ++x) rank += u[x] > mine - (k + x < c ? 1ull : 0ull) ? 1 : 0;
   }
   return rank;
 }
 
 // Selection of panel j0 by the NT threads of a workgroup: sel[0..nbp) := the nbp
-// candidates (columns j0 + c, c < ncand) of largest norm in descending order; norms that
-// agree to 2^-39 count as equal, ties go to the lowest index; NaN norms are never taken.
-// *sstop := 1 when even the largest is not above thr (the numerical rank is j0), 2 when
-// fewer than nbp candidates have a norm, else 0.
-// key (kMaxCols) and top (kMaxCols / 64 * QB) are LDS.  A key is a squared norm's bits,
-// ordered as the number is, with the last 13 replaced by 8191 - c: one comparison orders two
-// candidates.  Every candidate is ranked among the 64 of its block, then the QB best of each
-// block among each other.  Ends with a barrier.
+// candidates (columns j0 + c, c < ncand) of largest norm in descending order, ties to the
+// lowest index; NaN norms are never taken.  *sstop := 1 when even the largest is not above thr
+// (the numerical rank is j0), 2 when fewer than nbp candidates have a norm, else 0.
+// key (kMaxCols), top and topc (kMaxCols / 64 * QB) are LDS.  A key is a squared norm's bits,
+// ordered as the number is, plus one; 0: no candidate.  Every candidate is ranked among the 64
+// of its block, then the QB best of each block (key in top, candidate in topc) among each
+// other: their order there is that of their indices wherever keys are equal.  Ends with a
+// barrier.
 template <int NT>
-__device__ void select_panel(const double* qnrm, unsigned long long* key, unsigned long long* top, int ncand, int nbp,
-                             double thr, int j0, int* sel, int* sstop, int tid) {
+__device__ void select_panel(const double* qnrm, unsigned long long* key, unsigned long long* top, int* topc, int ncand,
+                             int nbp, double thr, int j0, int* sel, int* sstop, int tid) {
   if (tid < QB) sel[tid] = -1;
   const int nblk = (ncand + 63) / 64;
   for (int c = tid; c < 64 * nblk; c += NT) {
     const double v = c < ncand ? qnrm[j0 + c] : -1.0;
-    key[c] = v >= 0.0 ? ((unsigned long long)__double_as_longlong(v) & ~8191ull) | (unsigned)(8191 - c) : 0ull;
+    key[c] = v >= 0.0 ? (unsigned long long)__double_as_longlong(v) + 1ull : 0ull;
     if (c < nblk * QB) top[c] = 0ull;
   }
   __syncthreads();
   for (int c = tid; c < 64 * nblk; c += NT) {
     const unsigned long long mine = key[c];
-    const int rank = count_above(key + (c & ~63), 64, mine);
-    if (mine != 0ull && rank < QB) top[c / 64 * QB + rank] = mine;
+    if (mine == 0ull) continue;
+    const int rank = count_before(key + (c & ~63), 64, mine, c & 63);
+    if (rank < QB) {
+      top[c / 64 * QB + rank] = mine;
+      topc[c / 64 * QB + rank] = c;
+    }
   }
   __syncthreads();
   for (int c = tid; c < nblk * QB; c += NT) {
     const unsigned long long mine = top[c];
-    const int rank = count_above(top, nblk * QB, mine);
-    if (mine != 0ull && rank < nbp) sel[rank] = j0 + 8191 - (int)(mine & 8191ull);
+    if (mine == 0ull) continue;
+    const int rank = count_before(top, nblk * QB, mine, c);
+    if (rank < nbp) sel[rank] = j0 + topc[c];
   }
   __syncthreads();
   if (tid == 0) {
     int st = 0;
-    if (sel[0] < 0 || !(__longlong_as_double((long long)(key[sel[0] - j0] & ~8191ull)) > thr)) st = 1;
+    if (sel[0] < 0 || !(qnrm[sel[0]] > thr)) st = 1;
     for (int q = 1; q < nbp && !st; ++q)
       if (sel[q] < 0) st = 2;
     *sstop = st;
@@ -346,9 +385,36 @@ __device__ __forceinline__ void move_rows(zc* Wq, size_t ld, int i, int nmv, con
   }
 }
 
+// Reduce-scatter of 32 values over the wave: lane l ends with value 16 b5 + 8 b4 + 4 b3 + 2 b2 + b1
+// (b = bits of l), summed over all 64 lanes, and the even lanes write them to out.
+__device__ __forceinline__ void reduce_scatter(const double (&x)[2 * QB], double* out, int lane) {
+  double y16[16], y8[8], y4[4], y2[2];
+  const bool h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
+#pragma unroll
+  for (int m = 0; m < 16; ++m) y16[m] = swap_sum<32>(x[m], x[m + 16]);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) y8[m] = swap_sum<16>(y16[m], y16[m + 8]);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const double lo = y8[m], hi = y8[m + 4];
+    y4[m] = (h3 ? hi : lo) + lane_xor<8>(h3 ? lo : hi);
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const double lo = y4[m], hi = y4[m + 2];
+    y2[m] = (h2 ? hi : lo) + lane_xor<4>(h2 ? lo : hi);
+  }
+  double y1 = (h1 ? y2[1] : y2[0]) + lane_xor<2>(h1 ? y2[0] : y2[1]);
+  y1 += lane_xor<1>(y1);
+  const int idx = 16 * ((lane >> 5) & 1) + 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) +
+                  ((lane >> 1) & 1);
+  if ((lane & 1) == 0) out[idx] = y1;
+}
+
 // LDS of the register-resident panel.
 struct PanelLds {
   unsigned long long key[kMaxCols], top[kMaxCols / 64 * QB];
+  int topc[kMaxCols / 64 * QB];
   int sel[QB], mv_src[QB], mv_dst[QB];
   int snmv, sstop;
   double red[2][PW][32];  // by reflector parity: one barrier per reflector
@@ -356,7 +422,94 @@ struct PanelLds {
   zc coef[PW][QB];
   zc G[QB][QB + 1], Tm[QB][QB + 1], X[QB][QB + 1];
   zc stau[QB];
+  double wsum[32], rnorm[PW];  // the separate norm's chain
 };
+
+// The panel's reflectors with the norm of a column reduced before the column is scaled and its
+// products are formed (two reductions per reflector).  Row t + 64 NW s is thread t's row s, and the
+// waves' sums are added in wave order, so a panel of more waves than its rows need gives the same
+// numbers.
+template <int RPT, int NW>
+__device__ __forceinline__ void reflectors_of_norm(zc (&a)[RPT][QB], PanelLds& S, int j0, int nbp, int Rb, int tid) {
+  constexpr int NT = 64 * NW;
+  const int lane = tid & 63, wave = tid >> 6;
+  static_for<QB>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    if (q >= nbp) return;
+    const int j = j0 + q;
+    double part = 0.0;
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) {
+      const int i = tid + NT * s;
+      if (i > j && i < Rb) part += fma(a[s][q].x, a[s][q].x, a[s][q].y * a[s][q].y);
+      if (i == j) S.row[0][0] = a[s][q];
+    }
+    part = wave_sum(part);
+    if (lane == 0) S.rnorm[wave] = part;
+    __syncthreads();
+    double xn2 = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) xn2 += S.rnorm[w];
+    zc tau, scale = zmk(1.0, 0.0);
+    double beta = 0.0;
+    const bool refl = householder<true>(S.row[0][0], xn2, tau, beta, scale);
+    // v_q (rows > j; v_j = 1 implicitly) and R(j, j)
+    if (refl) {
+#pragma unroll
+      for (int s = 0; s < RPT; ++s) {
+        const int i = tid + NT * s;
+        if (i > j && i < Rb) a[s][q] = zmul(a[s][q], scale);
+        if (i == j) a[s][q] = zmk(beta, 0.0);
+      }
+    }
+    // slot m = 1 .. 15 - q: conj(v_q) a_(q+m) (the later columns, for the update);
+    // slot m > 15 - q: conj(v_p) v_q, p = m - 16 + q (the earlier reflectors, for T)
+    double x[2 * QB];
+#pragma unroll
+    for (int e = 0; e < 2 * QB; ++e) x[e] = 0.0;
+    // v_q on this thread's rows: 1 at row j, zero outside rows j .. Rb - 1, so that the
+    // products and the update below need no row test
+    zc vq[RPT];
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) {
+      const int i = tid + NT * s;
+      vq[s] = (i == j) ? zmk(1.0, 0.0) : ((i > j && i < Rb) ? a[s][q] : zmk(0.0, 0.0));
+    }
+#pragma unroll
+    for (int s = 0; s < RPT; ++s)
+#pragma unroll
+      for (int m = 1; m < QB; ++m) {
+        const bool later = m <= QB - 1 - q;  // earlier reflectors: rows >= j > j0 + p
+        const zc other = a[s][later ? q + m : m - QB + q];
+        const zc l = later ? vq[s] : other;
+        const zc r = later ? other : vq[s];
+        x[2 * m] = fma(l.x, r.x, fma(l.y, r.y, x[2 * m]));
+        x[2 * m + 1] = fma(l.x, r.y, fma(-l.y, r.x, x[2 * m + 1]));
+      }
+    reduce_scatter(x, S.red[0][wave], lane);
+    __syncthreads();
+    if (tid < 32) {
+      double sum = 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sum += S.red[0][w][tid];
+      S.wsum[tid] = sum;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int m = QB - q; m < QB; ++m) S.G[m - QB + q][q] = zmk(S.wsum[2 * m], S.wsum[2 * m + 1]);
+      S.stau[q] = tau;
+    }
+    if (refl) {
+      const zc ctau = zconj(tau);
+#pragma unroll
+      for (int m = 1; m <= QB - 1 - q; ++m) {
+        const zc f = zmul(ctau, zmk(S.wsum[2 * m], S.wsum[2 * m + 1]));
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) a[s][q + m] = zsub(a[s][q + m], zmul(f, vq[s]));
+      }
+    }
+  });
+}
 
 // Panel j0 with the panel in registers (Rb <= RPT * 64 NW, NW waves; thread t owns rows
 // t + 64 NW s, s < RPT):
@@ -380,7 +533,9 @@ struct PanelLds {
 // norms for the selection and T column by column, a panel took 52 us at 128 rows, 65 at 225 and
 // 73 at 400; now 28, 31 and 37 (at 64: 27), of which the chain is 21, 23 and 26, the selection 3,
 // 3 and 5 and T 2.
-template <int RPT, int NW>
+// CYCLIC (BondTask::cyclic, the number blocks): the norms, products and T in the order of
+// reflectors_of_norm and form_t_rows, for the reason given in tebd_jacobi.hip.
+template <int RPT, int NW, bool CYCLIC>
 __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S) {
   constexpr int NT = 64 * NW;
   const int Rb = t.Rb, Cb = t.Cb;
@@ -391,7 +546,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   const size_t ld = Rb;
 
   // 1. selection
-  select_panel<NT>(t.qnrm, S.key, S.top, ncand, nbp, t.qstate[1], j0, S.sel, &S.sstop, tid);
+  select_panel<NT>(t.qnrm, S.key, S.top, S.topc, ncand, nbp, t.qstate[1], j0, S.sel, &S.sstop, tid);
   if (S.sstop) {
     if (tid == 0) t.qstate[0] = S.sstop == 1 ? (double)j0 : 0.0;
     return;
@@ -416,7 +571,8 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   // 3. Householder QR of the panel, the column loop unrolled so that every register
   // index is static: column q sits in a[.][q], first as data, then as reflector v_q
   // (rows > j0 + q) below R(:, q).
-  static_for<QB>([&](auto qc) {
+  if constexpr (CYCLIC) reflectors_of_norm<RPT, NW>(a, S, j0, nbp, Rb, tid);
+  else static_for<QB>([&](auto qc) {
     constexpr int q = decltype(qc)::value, buf = q & 1;
     if (q >= nbp) return;
     const int j = j0 + q;
@@ -449,31 +605,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
         x[2 * m + 1] = fma(l.x, r.y, fma(-l.y, r.x, x[2 * m + 1]));
       }
     }
-    // reduce-scatter of the 32 values over the wave: lane l ends with value
-    // 16 b5 + 8 b4 + 4 b3 + 2 b2 + b1 (b = bits of l), summed over all 64 lanes
-    {
-      double y16[16], y8[8], y4[4], y2[2];
-      const bool h3 = lane & 8, h2 = lane & 4, h1 = lane & 2;
-#pragma unroll
-      for (int m = 0; m < 16; ++m) y16[m] = swap_sum<32>(x[m], x[m + 16]);
-#pragma unroll
-      for (int m = 0; m < 8; ++m) y8[m] = swap_sum<16>(y16[m], y16[m + 8]);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const double lo = y8[m], hi = y8[m + 4];
-        y4[m] = (h3 ? hi : lo) + lane_xor<8>(h3 ? lo : hi);
-      }
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        const double lo = y4[m], hi = y4[m + 2];
-        y2[m] = (h2 ? hi : lo) + lane_xor<4>(h2 ? lo : hi);
-      }
-      double y1 = (h1 ? y2[1] : y2[0]) + lane_xor<2>(h1 ? y2[0] : y2[1]);
-      y1 += lane_xor<1>(y1);
-      const int idx = 16 * ((lane >> 5) & 1) + 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) +
-                      2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
-      if ((lane & 1) == 0) S.red[buf][wave][idx] = y1;
-    }
+    reduce_scatter(x, S.red[buf][wave], lane);
     __syncthreads();
     // Every wave sums the waves' partials for itself, which saves a barrier; lane m (mod 16)
     // takes slot m.
@@ -485,7 +617,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
     const double xn2 = first_lane(sum.x);
     zc tau, scale = zmk(1.0, 0.0);
     double beta = 0.0;
-    const bool refl = householder(alpha, xn2, tau, beta, scale);
+    const bool refl = householder<false>(alpha, xn2, tau, beta, scale);
     // v_q = (1; x scale): w_k = conj(scale) sum + a_jk, and v_p^H v_q = scale sum + conj(v_p,j)
     if (m <= QB - 1 - q) {
       S.coef[wave][m] = zmul(zmk(-tau.x, tau.y), zadd(zmul(zconj(scale), sum), other));
@@ -525,14 +657,15 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
     }
   }
   if (tid < nbp) t.tau[j0 + tid] = S.stau[tid];
-  form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, S.Tm, S.X);
+  if constexpr (CYCLIC) form_t_rows(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  else form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, S.Tm, S.X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
 
 // One workgroup per task; the shape of its panel depends on the task's own row count, so a
 // task is factorised the same way whatever batch it is in.  Waves that a task does not need
 // leave at once.
-template <int NWMAX>
+template <int NWMAX, bool CYCLIC>
 __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
   if (t.qstate[0] >= 0.0) return;
@@ -543,22 +676,25 @@ __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __
   }
   __shared__ PanelLds S;
   const int wave = threadIdx.x >> 6;
-  if (t.Rb <= 64 && t.Cb <= 64) {  // no barriers: 28 us instead of 31 at 64 x 64; more candidates need more threads
-    if (wave < 1) panel_reg<1, 1>(t, j0, S);
+  constexpr int N4 = NWMAX < 4 ? NWMAX : 4;
+  if (!CYCLIC && t.Rb <= 64 && t.Cb <= 64) {  // no barriers: 28 us instead of 31 at 64 x 64; more candidates need more threads
+    if (wave < 1) panel_reg<1, 1, CYCLIC>(t, j0, S);
   } else if (t.Rb <= 128) {
-    if (wave < 2) panel_reg<1, 2>(t, j0, S);
+    if (wave < 2) panel_reg<1, 2, CYCLIC>(t, j0, S);
   } else if (NWMAX >= 4 && t.Rb <= 256) {
-    if (wave < 4) panel_reg<1, NWMAX < 4 ? NWMAX : 4>(t, j0, S);
+    if (wave < 4) panel_reg<1, N4, CYCLIC>(t, j0, S);
   } else if (NWMAX >= 8 && t.Rb <= 512) {
-    if (wave < 4) panel_reg<2, NWMAX < 4 ? NWMAX : 4>(t, j0, S);
+    if constexpr (CYCLIC) panel_reg<1, NWMAX, CYCLIC>(t, j0, S);
+    else if (wave < 4) panel_reg<2, N4, CYCLIC>(t, j0, S);
   } else if (NWMAX >= 8) {
-    panel_reg<2, NWMAX>(t, j0, S);
+    panel_reg<2, NWMAX, CYCLIC>(t, j0, S);
   }
 }
 
 // Panel j0 through global memory (any Rb; one workgroup of 256 threads per task): the
 // same selection, column moves, factorisation and T as k_qrp_panel_reg, with the
 // reflector applied column by column (one wave per column).
+template <bool CYCLIC>
 __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
   if (t.qstate[0] >= 0.0) return;
@@ -572,13 +708,14 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
   const int ncand = t.Cb - j0;
   const size_t ld = t.Rb;
   __shared__ unsigned long long key[kMaxCols], top[kMaxCols / 64 * QB];
+  __shared__ int topc[kMaxCols / 64 * QB];
   __shared__ int sel[QB], mv_src[QB], mv_dst[QB];
   __shared__ int snmv, sstop;
   __shared__ double red[4];
   __shared__ zc G[QB][QB + 1], Tm[QB][QB + 1], X[QB][QB + 1];
   __shared__ zc stau[QB];
   __shared__ double gred[3][2][256];
-  select_panel<256>(t.qnrm, key, top, ncand, nbp, t.qstate[1], j0, sel, &sstop, tid);
+  select_panel<256>(t.qnrm, key, top, topc, ncand, nbp, t.qstate[1], j0, sel, &sstop, tid);
   if (sstop) {
     if (tid == 0) t.qstate[0] = sstop == 1 ? (double)j0 : 0.0;
     return;
@@ -609,7 +746,7 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
     const zc alpha = cj[j];
     zc tau, scale = zmk(1.0, 0.0);
     double beta = 0.0;
-    const bool refl = householder(alpha, xn2, tau, beta, scale);
+    const bool refl = householder<CYCLIC>(alpha, xn2, tau, beta, scale);
     __syncthreads();  // every thread has read alpha
     if (refl) {
       for (int i = j + 1 + tid; i < t.Rb; i += 256) cj[i] = zmul(cj[i], scale);
@@ -646,7 +783,8 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
     gram_partial<1, 1>(vload, vload, K, wave, 4, lane, gre, gim);
     gram_reduce<1, 1>(gre, gim, gred, &G[0][0], QB + 1, wave, lane);
   }
-  form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, Tm, X);
+  if constexpr (CYCLIC) form_t_rows(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  else form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, Tm, X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
 
@@ -1095,12 +1233,19 @@ hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, dou
   return hipGetLastError();
 }
 
-hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, hipStream_t st) {
+hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, bool cyclic,
+                            hipStream_t st) {
   if (max_cb > kMaxCols) return hipErrorInvalidValue;
-  if (max_rb <= 128) hipLaunchKernelGGL(k_qrp_panel_reg<2>, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
-  else if (max_rb <= 256) hipLaunchKernelGGL(k_qrp_panel_reg<4>, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
-  else if (max_rb <= 1024) hipLaunchKernelGGL(k_qrp_panel_reg<8>, dim3(ntasks), dim3(512), 0, st, d_tasks, j0);
-  else hipLaunchKernelGGL(k_qrp_panel, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+  const auto k2 = cyclic ? k_qrp_panel_reg<2, true> : k_qrp_panel_reg<2, false>;
+  const auto k4 = cyclic ? k_qrp_panel_reg<4, true> : k_qrp_panel_reg<4, false>;
+  const auto k8 = cyclic ? k_qrp_panel_reg<8, true> : k_qrp_panel_reg<8, false>;
+  if (max_rb <= 128) hipLaunchKernelGGL(k2, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
+  else if (max_rb <= 256) hipLaunchKernelGGL(k4, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+  else if (max_rb <= 1024) hipLaunchKernelGGL(k8, dim3(ntasks), dim3(512), 0, st, d_tasks, j0);
+  else {
+    const auto k = cyclic ? k_qrp_panel<true> : k_qrp_panel<false>;
+    hipLaunchKernelGGL(k, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+  }
   return hipGetLastError();
 }
 
