@@ -41,6 +41,11 @@ constexpr int kQrCheck = 8;       // panels between checks whether every task ha
 // launch (tebd_jacobi_small.hip).  A chain's edge bonds (4 x 256, say) are preconditioned with the
 // bulk's: on their own they held up the half-sweep by 160-320 us.
 constexpr int kQrMinSide = 64;
+// CanonicalForm's SVDs of at most 32 columns and this many rows are solved in one launch too; more
+// rows or columns are more work than one workgroup should have.  Canonical form of 8 sites of d = 4,
+// chi = 60 (240 x 60): all sweep by sweep 22 ms, all in one launch 30; of 10 sites of d = 2, chi =
+// 32 (64 x 32): 11.5 and 9.
+constexpr int kSmallFormRows = 64;
 constexpr int kMaxSweeps = 40;
 constexpr double kTolRel = 1e-13;   // relative orthogonality of converged column pairs
 constexpr double kTolAbs = 1e-13;   // rounding floor: |A_pq| <= kTolAbs ||theta|| (|w_p| + |w_q|)
@@ -1178,8 +1183,9 @@ int device_svd_batch(tebd_ctx* c, const SvdJob* jobs, int nb) {
   for (int i = 0; i < nb; ++i) {
     BondTask& t = c->h_tasks[i];
     std::memset(&t, 0, sizeof(t));
+    t.cyclic = 1;
     t.W = jobs[i].W; t.R = jobs[i].R; t.C = jobs[i].C; t.Cpad = round_up(t.C, JC); t.P = t.Cpad / JC;
-    t.small = t.P <= kSmallPairs;
+    t.small = t.P == 1 && t.R <= kSmallFormRows;
     t.V = jobs[i].V; t.NV = t.Cpad; t.s = jobs[i].s; t.perm = jobs[i].perm;
     attach_jacobi(c, t, i);
     t.result = c->results + (size_t)RESULT_STRIDE * i;

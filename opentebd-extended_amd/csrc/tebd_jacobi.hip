@@ -24,10 +24,13 @@
 // all index pairs per visit (93 rounds, two barriers each) took 59 us at 400 x 400
 // (Fermi-Hubbard, chi = 100) and 54 at 225 x 225 (Bose-Hubbard, chi = 45); one pass over the
 // cross pairs (16 rounds of one barrier) takes 16 and 14, for 6 to 7 outer sweeps instead of 5
-// to 6.  Whole cyclic sweeps per visit stay for tasks that say so (BondTask::cyclic).  The number
-// blocks' Schmidt values are cut at 1e-10, where another rounding keeps another state: with one pass a
-// Fermi-Hubbard chain of 64 sites, chi = 128, gave lambda up to 8e-9 from what cyclic sweeps give
-// (its step takes 14.5 ms so and 19.6 with them).
+// to 6.  Whole cyclic sweeps per visit stay for tasks that say so (BondTask::cyclic):
+//   * CanonicalForm's matrices are not preconditioned: with a generic basis and singular values
+//     over 13 decades one pass per visit does not converge within 40 sweeps at 192 columns
+//     (cyclic: 36).
+//   * the number blocks' Schmidt values are cut at 1e-10, where another rounding keeps another
+//     state: with one pass a Fermi-Hubbard chain of 64 sites, chi = 128, gave lambda up to 8e-9 from
+//     what cyclic sweeps give (its step takes 14.5 ms so and 19.6 with them).
 //
 // Work that cannot change the result is skipped exactly:
 //   * a task whose previous sweep rotated nothing has converged: its workgroups exit;
