@@ -91,32 +91,6 @@ constexpr Table level_table(int first_level) {
 __device__ constexpr CrossTable kCross = level_table<CrossTable>(4);
 __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 
-// The rotation that zeroes g in [[a, g], [conj(g), b]], as jrot's: tan theta = t = 2|g| sign(b - a) /
-// (|b - a| + sqrt((b - a)^2 + 4|g|^2)); t w is formed without |g|.  The hardware
-// estimates of the square root and the quotient (about 2^-24, one Newton-Raphson step on
-// the quotient) suffice for t: an angle that is off by 1e-7 of itself leaves 1e-7 of
-// the coupling for the next sweep.  c = 1/sqrt(1 + t^2) is refined to full precision (two
-// steps) and s = c t, so the rotation is unitary to rounding whatever t's error.
-// a and b become the rotated diagonal a - t|g|, b + t|g|.
-__device__ __forceinline__ void pass_rotation(double& a, double& b, zc g, double g2, double& c, zc& sw) {
-  const double dd = b - a;
-  const double e2 = fma(dd, dd, 4.0 * g2);
-  const double den = fma(e2, __builtin_amdgcn_rsq(e2), fabs(dd));
-  double inv = __builtin_amdgcn_rcp(den);
-  inv = inv * fma(-den, inv, 2.0);
-  const double f = dd < 0.0 ? -2.0 * inv : 2.0 * inv;
-  const double tx = f * g.x, ty = f * g.y;
-  const double h = fma(tx, tx, fma(ty, ty, 1.0));
-  double r = __builtin_amdgcn_rsq(h);
-  const double hh = 0.5 * h;
-  r = r * fma(-hh * r, r, 1.5);
-  r = r * fma(-hh * r, r, 1.5);
-  c = r;
-  sw = zmk(tx * r, ty * r);
-  a = fma(-f, g2, a);
-  b = fma(f, g2, b);
-}
-
 // Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
 // sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
 // blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
@@ -157,7 +131,7 @@ __device__ __forceinline__ void inner_jacobi(PairLds& L, const Rounds& T, int ti
   for (int pass = 0; pass < (FULL ? 2 : 1); ++pass) {
     if (tid < kInnerPairs) {
       const int p = level_p(FULL ? 8 : 16, tid), q = level_q(FULL ? 8 : 16, 0, tid);
-      A[p][q] = make_rotation(rb[buf], dg[p], dg[q], &dg[p], &dg[q], nullptr, tid, A[p][q], pass_rotation);
+      A[p][q] = make_rotation(rb[buf], dg[p], dg[q], &dg[p], &dg[q], nullptr, tid, A[p][q], jrot);
     }
     __syncthreads();
     if (FULL) {
@@ -170,7 +144,7 @@ __device__ __forceinline__ void inner_jacobi(PairLds& L, const Rounds& T, int ti
           const RotBuf& R = rb[buf];
           if (is_a) {
             const unsigned e1 = T.entry[rd + 1][tid], n1 = T.next[rd + 1][tid];
-            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, pass_rotation);
+            update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
             entry = e1;
             next = n1;
           } else if (is_q) {
@@ -205,7 +179,7 @@ __device__ __forceinline__ void inner_jacobi(PairLds& L, const Rounds& T, int ti
           e1 = T.entry[ahead][tid];
           n1 = T.next[ahead][tid];
         }
-        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, pass_rotation);
+        update_block(&A[0][0], dg, R, rb[buf ^ 1], nullptr, entry, next, tr, tk, half, jrot);
         if (!FULL) {
           e1 = T.entry[ahead][tid];
           if (tid < NN) n1 = T.next[ahead][tid];
@@ -239,8 +213,8 @@ __device__ __forceinline__ void inner_jacobi(PairLds& L, const Rounds& T, int ti
 
 template <bool FULL>
 __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* __restrict__ tasks, int sweep, int round,
-                                                      double tol_rel, double tol_abs, int* __restrict__ wl_count,
-                                                      int2* __restrict__ wl_items, int wl_cap) {
+                                                      double tol_rel, double tol_abs, double tol_pass,
+                                                      int* __restrict__ wl_count, int2* __restrict__ wl_items, int wl_cap) {
   const BondTask t = tasks[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= t.P || round >= 2 * t.P - 1) return;
@@ -308,10 +282,10 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   }
 
   // ---- does this pair need a rotation?  |A_pq| > tol_rel sqrt(A_pp A_qq) and
-  // |A_pq| > tol_abs max_c|w_c| (|w_p| + |w_q|): the second bound is the
-  // rounding floor of the rotations in the |w_c|-sized columns of W
+  // |A_pq| > tol max_c|w_c| (|w_p| + |w_q|), tol = tol_abs (cyclic) or tol_pass: the second bound
+  // is the rounding floor of the rotations in the |w_c|-sized columns of W
   {
-    const double floor = tol_abs * sqrt(t.result[2]);  // of the largest column norm
+    const double floor = (cyclic ? tol_abs : tol_pass) * sqrt(t.result[2]);  // of the largest column norm
     int need = 0;
     for (int e = tid; e < (FULL ? JC * JC : JB * JB); e += kRoundThreads) {
       const int pp = FULL ? e % JC : e % JB, qq = FULL ? e / JC : JB + e / JB;
@@ -448,11 +422,11 @@ hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sw
 }
 
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
-                               double tol_rel, double tol_abs, int* wl_count, int2* wl_items, int wl_cap,
-                               hipStream_t st) {
+                               double tol_rel, double tol_abs, double tol_pass, int* wl_count, int2* wl_items,
+                               int wl_cap, hipStream_t st) {
   const auto k = round == 0 ? k_jacobi_round<true> : k_jacobi_round<false>;
   hipLaunchKernelGGL(k, dim3(max_pairs, ntasks), dim3(kRoundThreads), 0, st, d_tasks, sweep, round, tol_rel, tol_abs,
-                     wl_count, wl_items, wl_cap);
+                     tol_pass, wl_count, wl_items, wl_cap);
   return hipGetLastError();
 }
 

@@ -17,8 +17,8 @@ hipError_t launch_frobenius(const BondTask* d_tasks, int ntasks, int max_cpad, h
 hipError_t launch_jacobi_begin(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_jacobi_sweep_begin(const BondTask* d_tasks, int ntasks, int sweep, int* wl_count, hipStream_t st);
 hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pairs, int sweep, int round,
-                               double tol_rel, double tol_abs, int* wl_count, int2* wl_items, int wl_cap,
-                               hipStream_t st);
+                               double tol_rel, double tol_abs, double tol_pass, int* wl_count, int2* wl_items,
+                               int wl_cap, hipStream_t st);
 hipError_t launch_jacobi_rotate(const BondTask* d_tasks, int round, int max_rows_w, int max_rows_v, int* wl_count,
                                 int2* wl_items, int wl_cap, hipStream_t st);
 // The whole solve of every task with BondTask::small, one launch per pair count present in the batch.
