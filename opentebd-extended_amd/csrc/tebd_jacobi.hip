@@ -31,6 +31,7 @@
 //   * the number blocks' Schmidt values are cut at 1e-10, where another rounding keeps another
 //     state: with one pass a Fermi-Hubbard chain of 64 sites, chi = 128, gave lambda up to 8e-9 from
 //     what cyclic sweeps give (its step takes 14.5 ms so and 19.6 with them).
+// They also stay for bonds of more than kCyclicRows rows, see there.
 //
 // Work that cannot change the result is skipped exactly:
 //   * a task whose previous sweep rotated nothing has converged: its workgroups exit;
@@ -40,8 +41,6 @@
 // sweep parity), counter[2] pairs whose Gram was formed and counter[3] rotated pairs
 // over the whole SVD; blkver[b] counts rotations of block b and pairseen[lo*2P+hi]
 // holds (blkver[lo], blkver[hi]) from the last time that pair was verified.
-#include <type_traits>
-
 #include "tebd_device.h"
 #include "tebd_jacobi_inner.h"
 #include "tebd_kernels.h"
@@ -62,10 +61,18 @@ __host__ __device__ constexpr int level_q(int h, int r, int t) {
   return level_p(h, t) - (t & (h - 1)) + h + (((t & (h - 1)) + r) & (h - 1));
 }
 
+// Bonds of more rows solve each visited pair by cyclic sweeps: their Grams and rotations of W cost
+// more than the rounds, which run side by side once a batch fills the GPU, so fewer outer sweeps
+// pay.  Hubbard, exact SVDs, ms per step with one pass per visit and with cyclic sweeps, chains of
+// 24 and of 96 sites: 560 rows 51 and 56, 111 and 98; 720 rows 75 and 84, 211 and 176; 800 rows 77
+// and 82, 264 and 211; 912 rows 124 and 130, 452 and 341; 1024 rows 163 and 165, 673 and 537; 128
+// sites, 1024 rows 235 and 186.  Below the bound, 64 sites of 512 rows 55 and 59, 24 sites of 400
+// rows 26 and 32.  The bound looks at the bond alone, so that no result depends on the batch.
+constexpr int kCyclicRows = 512;
+
 // The schedules: kCross the 16 rounds of level 16 (pair t's next entry lies in block (t, t + 1),
 // the last one's in block (0, 15)), kFull the 15 rounds of levels 8, 4, 2, 1 and then kCross.
 constexpr int kWithinRounds = JB - 1;
-constexpr int kWithinRows = 512;
 using CrossTable = InnerTable<JB, 2 * kInnerPairs>;
 using FullTable = InnerTable<kAllRounds, 2 * kOffBlocks>;
 template <class Table>
@@ -94,12 +101,7 @@ __device__ constexpr FullTable kFull = level_table<FullTable>(0);
 // Eigenvector rotations of a pair's Gram matrix A into Q.  A pair is visited once per outer
 // sweep, so its eigenproblem need not be finished: the 256 index pairs across the two
 // blocks are rotated once (16 rounds); in the first round of a sweep (FULL), whose Gram
-// includes the blocks' own couplings, the pairs within the blocks too, in two passes.  So do all
-// rounds of a bond with more than kWithinRows rows: its Grams and rotations of W cost more than the
-// rounds, and a sixth fewer sweeps pays once the batch fills the GPU.  Hubbard, exact SVDs, ms per
-// step without and with it: L = 128, chi = 256 206 and 192; L = 32, chi = 256 121 and 127; L = 24, chi
-// = 200 86 and 94; below the bound L = 64, chi = 128 47 and 51.  The bound looks at the bond alone, so
-// that no result depends on the batch.
+// includes the blocks' own couplings, the pairs within the blocks too, in two passes.
 // Measured on Hubbard and Bose-Hubbard bonds (numpy restatement, 225 x 225 and 256 x 256):
 // 6 outer sweeps and 1300-1400 inner rounds in sequence per solve; three cyclic sweeps over
 // all 496 pairs per visit take 5 outer sweeps but 4400-4650 rounds in sequence.
@@ -230,19 +232,15 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   unsigned long long* seen = t.pairseen + (size_t)lo * nblk + hi;
   if (!FULL && *seen == stamp) return;  // unchanged since it was verified orthogonal
 
-  // The schedule of 16 rounds lies in LDS; those of 31 (60 and 34 KB, which would leave room for one
-  // workgroup on a CU instead of two) are read from L2 one round ahead.  With the longer one in LDS the
-  // exact step of Hubbard L = 128, chi = 256 took 204 ms instead of 192.
+  // The schedules are read from L2 one round ahead: that of 16 rounds in LDS gave no time and its 17
+  // KB kept the other lanes' kernels off the CU (96 sites, 1024 rows: 559 ms a step with it, 537).
   __shared__ PairLds L;
-  __shared__ typename std::conditional<FULL, int, decltype(CrossTable::rounds)>::type table;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const zc* Wi = t.W + (size_t)t.R * (bi * JB);
   const zc* Wj = t.W + (size_t)t.R * (bj * JB);
   if (tid == 0) L.need = 0;
-  const bool cyclic = t.cyclic, within = FULL || t.R > kWithinRows;
-  if constexpr (!FULL)
-    if (!cyclic && !within) load_rounds(table, kCross.rounds, tid, kRoundThreads);
+  const bool cyclic = t.cyclic || t.R > kCyclicRows;
 
   // ---- Gram: A = [Wi Wj]^H [Wi Wj]
   {
@@ -308,8 +306,8 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
 
   // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
   if (cyclic) inner_solve<true>(L, kRing.rounds, tid, true);
-  else if (within) inner_jacobi<true>(L, kFull.rounds, tid);
-  else if constexpr (!FULL) inner_jacobi<false>(L, table, tid);
+  else if constexpr (FULL) inner_jacobi<true>(L, kFull.rounds, tid);
+  else inner_jacobi<false>(L, kCross.rounds, tid);
   zc (*Q)[JC + 1] = L.Q;
   zc* qg = t.Qg + (size_t)p * JC * JC;
   for (int e = tid; e < JC * JC; e += kRoundThreads) qg[e] = Q[e / JC][e % JC];  // qg[k JC + c] = Q[k][c]
