@@ -129,12 +129,12 @@ struct tebd_ctx {
   int obs_batch = 0;
   // all-pairs reduced density matrices (tebd_two_point_rdms), allocated on first use:
   // environments of cr_envs right sites (two, chi^2 d^2, and T, chi^2 d^3, each), the left
-  // factors of every chain (chi d chi), the phase, the device copies of the pair (d^4) and
+  // factors of cr_chains chains (chi d chi), the phase, the device copies of the pair (d^4) and
   // site (d^2) matrices, and the descriptors of a group of right sites (device and pinned)
   zc* cr_theta[2] = {nullptr, nullptr};
   zc *cr_T = nullptr, *cr_B = nullptr, *cr_A = nullptr, *cr_rho2 = nullptr, *cr_rho1 = nullptr;
   double* cr_phase = nullptr;
-  int cr_envs = 0;
+  int cr_envs = 0, cr_chains = 0;
   unsigned char *cr_desc = nullptr, *cr_hdesc = nullptr;
   size_t cr_desc_bytes = 0;
   // rank model (learned-rank path) and the training record of the full path
@@ -3213,14 +3213,16 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
   const size_t np = (size_t)Lc * (Lc - 1) / 2, d4 = (size_t)d2 * d2;
   const size_t th = (size_t)chi * chi * d2, fac = (size_t)chi * d * chi;
   if (!c->cr_rho1) {
-    // every right site at once, up to the budget of environments
+    // every right site at once, up to the budget of environments and what a grid's second and
+    // third dimensions hold
     const double per = sizeof(zc) * (double)th * (2 + d);
-    c->cr_envs = (int)std::max(1.0, std::min((double)c->L, std::floor(kCrBudget / per)));
+    c->cr_envs = (int)std::max(1.0, std::min({(double)c->L, 32768.0, std::floor(kCrBudget / per)}));
+    c->cr_chains = std::max(1, std::min(nch, c->cr_envs / Lc));
     HIPCHK(c, hipMalloc(&c->cr_theta[0], sizeof(zc) * th * c->cr_envs));
     HIPCHK(c, hipMalloc(&c->cr_theta[1], sizeof(zc) * th * c->cr_envs));
     HIPCHK(c, hipMalloc(&c->cr_T, sizeof(zc) * th * d * c->cr_envs));
-    HIPCHK(c, hipMalloc(&c->cr_B, sizeof(zc) * fac * nch));
-    HIPCHK(c, hipMalloc(&c->cr_A, sizeof(zc) * fac * nch));
+    HIPCHK(c, hipMalloc(&c->cr_B, sizeof(zc) * fac * c->cr_chains));
+    HIPCHK(c, hipMalloc(&c->cr_A, sizeof(zc) * fac * c->cr_chains));
     HIPCHK(c, hipMalloc(&c->cr_phase, sizeof(double) * d));
     HIPCHK(c, hipMalloc(&c->cr_rho2, sizeof(zc) * d4 * np * nch));
     HIPCHK(c, hipMalloc(&c->cr_rho1, sizeof(zc) * d2 * c->L));
@@ -3232,24 +3234,30 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
   }
   auto slab = [&](int s) { return c->gam + (size_t)s * c->gslab(); };
   auto lam = [&](int b) { return c->lam + (size_t)b * chi; };
-  // right sites (chain r, site l2), the rightmost first, in groups of cr_envs environments; a
-  // group's environments are stepped together over the left sites l1 of their chains
-  std::vector<std::pair<int, int>> all;
-  for (int l2 = Lc - 1; l2 >= 0; --l2)
-    for (int r = 0; r < nch; ++r) all.push_back({r, l2});
+  // right sites (chain r, site l2) in groups of at most cr_envs environments: those of cr_chains
+  // chains together where all of a chain's fit, else a part of one chain's; the rightmost first.  A
+  // group's environments are stepped together over the left sites l1 of their chains.
+  struct Group { int r0, nr, l2_hi, l2_lo; };  // chains r0 .. r0 + nr - 1, sites l2_hi down to l2_lo
+  std::vector<Group> groups;
+  for (int r0 = 0; r0 < nch; r0 += c->cr_chains) {
+    const int nr = std::min(c->cr_chains, nch - r0), part = std::max(1, c->cr_envs / nr);
+    for (int hi = Lc - 1; hi >= 0; hi -= part) groups.push_back({r0, nr, hi, std::max(0, hi - part + 1)});
+  }
   struct Step { size_t left, pair, gemm, next; int nleft, npair, max_ca, max_cb; };
-  for (size_t g0 = 0; g0 < all.size(); g0 += c->cr_envs) {
-    const int ng = (int)std::min(all.size() - g0, (size_t)c->cr_envs);
+  for (const Group& g : groups) {
+    const int nsites = g.l2_hi - g.l2_lo + 1, ng = g.nr * nsites;
+    // environment (l2_hi - l2) nr + (r - r0) is that of chain r and site l2
+    auto env = [&](int r, int l2) { return (g.l2_hi - l2) * g.nr + (r - g.r0); };
     std::vector<CrRight> right(ng);
     std::vector<GemmTask> first(ng);
     std::vector<CrLeft> left;
     std::vector<CrPair> pairs;
     std::vector<GemmTask> gemms;  // per step: T = Theta Gbar of every pair, then A_k T_k of every pair, k < d
     std::vector<Step> steps;
-    int max_ml = 1, max_l2 = 0;
+    int max_ml = 1;
     size_t max_r = 1;
     for (int q = 0; q < ng; ++q) {
-      const auto [r, l2] = all[g0 + q];
+      const int r = g.r0 + q % g.nr, l2 = g.l2_hi - q / g.nr;
       const int s2 = r * Lc + l2, chl = c->chi[s2], chr = c->chi[s2 + 1];
       // K and B, which only start the environment, lie in its T
       zc* K = c->cr_T + th * d * q;
@@ -3258,19 +3266,15 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
       first[q] = {K, K + fac, right[q].theta, chl * d, d * chl, chr, chl * d, chr, chl * d, 1.0, 0};
       max_ml = std::max(max_ml, chl * d);
       max_r = std::max(max_r, (size_t)chl * d * chr);
-      max_l2 = std::max(max_l2, l2);
     }
-    for (int l1 = max_l2 - 1; l1 >= 0; --l1) {
+    for (int l1 = g.l2_hi - 1; l1 >= 0; --l1) {
       Step st{left.size(), pairs.size(), gemms.size(), 0, 0, 0, 1, 1};
       std::vector<GemmTask> adv;
-      for (int r = 0; r < nch; ++r) {
+      for (int r = g.r0; r < g.r0 + g.nr; ++r) {
         const int s1 = r * Lc + l1, ca = c->chi[s1], cb = c->chi[s1 + 1];
-        zc *A = c->cr_A + fac * r, *Gbar = c->cr_B + fac * r;
-        bool used = false;
-        for (int q = 0; q < ng; ++q) {
-          const auto [rq, l2] = all[g0 + q];
-          if (rq != r || l2 <= l1) continue;
-          used = true;
+        zc *A = c->cr_A + fac * (r - g.r0), *Gbar = c->cr_B + fac * (r - g.r0);
+        for (int l2 = g.l2_hi; l2 >= g.l2_lo && l2 > l1; --l2) {
+          const int q = env(r, l2);
           const int cur = (l2 - 1 - l1) & 1;  // steps taken so far
           zc *Th = c->cr_theta[cur] + th * q, *Nx = c->cr_theta[1 - cur] + th * q, *T = c->cr_T + th * d * q;
           const size_t pair = (size_t)l1 * Lc - (size_t)l1 * (l1 + 1) / 2 + (l2 - l1 - 1);
@@ -3279,7 +3283,6 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
           gemms.push_back({Th, Gbar, T, cb * d2, ca * d, cb, cb * d2, cb, cb * d2, 1.0, 0});
           adv.push_back({A, T, Nx, ca, d2 * ca, cb, ca * d, cb, ca, 1.0, 0});
         }
-        if (!used) continue;
         left.push_back({slab(s1), lam(s1), ph, ca, cb, d, A, Gbar});
         st.max_ca = std::max(st.max_ca, ca);
         st.max_cb = std::max(st.max_cb, cb);
