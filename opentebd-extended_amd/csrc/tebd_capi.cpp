@@ -672,6 +672,97 @@ void account_gemm(tebd_ctx* c, const GemmTask* g, int n) {
   }
 }
 
+// The workspaces of the measurements are allocated on first use; a call that cannot have the largest
+// one tries half as much until its smallest does not fit either.  A failed allocation leaves nothing
+// behind, neither memory nor HIP's last error.
+template <class T>
+hipError_t alloc_n(T** p, size_t n) {
+  const hipError_t e = hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * n);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+  }
+  return e;
+}
+
+template <class T>
+hipError_t alloc_pinned(T** p, size_t n) {
+  const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(p), sizeof(T) * n);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+  }
+  return e;
+}
+
+void free_expval(tebd_ctx* c) {
+  (void)hipFree(c->obs_ops);
+  (void)hipFree(c->obs_out);
+  (void)hipFree(c->obs_part);
+  (void)hipFree(c->d_obs);
+  (void)hipHostFree(c->h_obs);
+  c->obs_ops = c->obs_out = c->obs_part = nullptr;
+  c->d_obs = c->h_obs = nullptr;
+  c->obs_batch = 0;
+}
+
+hipError_t alloc_expval(tebd_ctx* c) {
+  // every bond at once, up to 64 MiB of partial sums
+  const int L = c->L;
+  const size_t tiles = expval_tiles(c->d, c->chi_max);
+  int nb = (int)std::max(1.0, std::min({(double)(L - 1), 32768.0, std::floor(double(64 << 20) / (sizeof(zc) * (double)tiles))}));
+  for (;; nb = (nb + 1) / 2) {
+    hipError_t e = alloc_n(&c->obs_ops, c->d4() * (L - 1));
+    if (e == hipSuccess) e = alloc_n(&c->obs_out, L - 1);
+    if (e == hipSuccess) e = alloc_n(&c->obs_part, tiles * nb);
+    if (e == hipSuccess) e = alloc_n(&c->d_obs, nb);
+    if (e == hipSuccess) e = alloc_pinned(&c->h_obs, nb);
+    if (e == hipSuccess) {
+      c->obs_batch = nb;
+      return e;
+    }
+    free_expval(c);
+    if (e != hipErrorOutOfMemory || nb == 1) return e;
+  }
+}
+
+void free_rdms(tebd_ctx* c) {
+  for (zc** p : {&c->cr_theta[0], &c->cr_theta[1], &c->cr_T, &c->cr_B, &c->cr_A, &c->cr_rho2, &c->cr_rho1}) {
+    (void)hipFree(*p);
+    *p = nullptr;
+  }
+  (void)hipFree(c->cr_phase);
+  c->cr_phase = nullptr;
+  c->cr_envs = c->cr_chains = 0;
+}
+
+hipError_t alloc_rdms(tebd_ctx* c) {
+  const size_t d = c->d, d2 = d * d, chi = c->chi_max, Lc = c->chain_len, nch = c->nchain;
+  const size_t np = Lc * (Lc - 1) / 2, th = chi * chi * d2, fac = chi * d * chi;
+  // every right site at once, up to the budget of environments and what a grid's second and
+  // third dimensions hold
+  const double per = sizeof(zc) * (double)th * (2 + d);
+  int envs = (int)std::max(1.0, std::min({(double)c->L, 32768.0, std::floor(kCrBudget / per)}));
+  for (;; envs = (envs + 1) / 2) {
+    const int chains = std::max(1, std::min((int)nch, envs / (int)Lc));
+    hipError_t e = alloc_n(&c->cr_rho2, d2 * d2 * np * nch);
+    if (e == hipSuccess) e = alloc_n(&c->cr_rho1, d2 * c->L);
+    if (e == hipSuccess) e = alloc_n(&c->cr_phase, d);
+    if (e == hipSuccess) e = alloc_n(&c->cr_B, fac * chains);
+    if (e == hipSuccess) e = alloc_n(&c->cr_A, fac * chains);
+    if (e == hipSuccess) e = alloc_n(&c->cr_theta[0], th * envs);
+    if (e == hipSuccess) e = alloc_n(&c->cr_theta[1], th * envs);
+    if (e == hipSuccess) e = alloc_n(&c->cr_T, th * d * envs);
+    if (e == hipSuccess) {
+      c->cr_envs = envs;
+      c->cr_chains = chains;
+      return e;
+    }
+    free_rdms(c);
+    if (e != hipErrorOutOfMemory || envs == 1) return e;
+  }
+}
+
 // Shape class of a batched GEMM launch: conj flag, M and N rounded up to 64, the batch
 // size rounded up to a power of two.
 uint64_t gemm_key(int max_m, int max_n, int ntasks, bool conj) {
@@ -1790,6 +1881,7 @@ tebd_ctx* make_lane(tebd_ctx* c, int lane, int slot0, int nslots) {
   l->cf_sets = 0;
   l->cr_theta[0] = l->cr_theta[1] = l->cr_T = l->cr_B = l->cr_A = l->cr_rho2 = l->cr_rho1 = nullptr;
   l->cr_phase = nullptr;
+  l->cr_envs = l->cr_chains = 0;
   l->cr_desc = l->cr_hdesc = nullptr;
   l->nc_theta = l->nc_vec = nullptr;   // the number-conserving update runs on the context only
   l->nc_small = nullptr;
@@ -2107,15 +2199,10 @@ void free_all(tebd_ctx* c) {
   (void)hipFree(c->wl_items);
   (void)hipFree(c->results);
   (void)hipFree(c->results2);
-  (void)hipFree(c->obs_ops);
-  (void)hipFree(c->obs_out);
-  (void)hipFree(c->obs_part);
-  (void)hipFree(c->d_obs);
-  (void)hipHostFree(c->h_obs);
-  for (zc* p : {c->cr_theta[0], c->cr_theta[1], c->cr_T, c->cr_B, c->cr_A, c->cr_rho2, c->cr_rho1}) (void)hipFree(p);
+  free_expval(c);
+  free_rdms(c);
   (void)hipFree(c->cr_desc);
   (void)hipHostFree(c->cr_hdesc);
-  (void)hipFree(c->cr_phase);
   (void)hipFree(c->mlp);
   (void)hipFree(c->d_feat);
   (void)hipFree(c->d_pred);
@@ -2807,17 +2894,7 @@ int tebd_expval_two_site(tebd_ctx* c, const double* ops, double* out) {
   if (e) return e;
   if (!ops || !out) return fail(c, TEBD_ERR_ARG, "expval_two_site: null operator or output");
   const int L = c->L, d = c->d;
-  if (!c->h_obs) {
-    // every bond at once, up to 64 MiB of partial sums
-    const double tiles = (double)expval_tiles(d, c->chi_max);
-    const int nb = (int)std::max(1.0, std::min({(double)(L - 1), 32768.0, std::floor(double(64 << 20) / (sizeof(zc) * tiles))}));
-    HIPCHK(c, hipMalloc(&c->obs_ops, sizeof(zc) * c->d4() * (L - 1)));
-    HIPCHK(c, hipMalloc(&c->obs_out, sizeof(zc) * (L - 1)));
-    HIPCHK(c, hipMalloc(&c->obs_part, sizeof(zc) * (size_t)tiles * nb));
-    HIPCHK(c, hipMalloc(&c->d_obs, sizeof(BondTask) * nb));
-    HIPCHK(c, hipHostMalloc(&c->h_obs, sizeof(BondTask) * nb));
-    c->obs_batch = nb;
-  }
+  if (!c->obs_batch) HIPCHK(c, alloc_expval(c));
   HIPCHK(c, hipMemcpyAsync(c->obs_ops, ops, sizeof(zc) * c->d4() * (L - 1), hipMemcpyHostToDevice, c->st));
   for (int b0 = 0; b0 < L - 1; b0 += c->obs_batch) {
     const int nb = std::min(c->obs_batch, L - 1 - b0);
@@ -3212,21 +3289,7 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
   const int d = c->d, Lc = c->chain_len, chi = c->chi_max, d2 = d * d, nch = c->nchain;
   const size_t np = (size_t)Lc * (Lc - 1) / 2, d4 = (size_t)d2 * d2;
   const size_t th = (size_t)chi * chi * d2, fac = (size_t)chi * d * chi;
-  if (!c->cr_rho1) {
-    // every right site at once, up to the budget of environments and what a grid's second and
-    // third dimensions hold
-    const double per = sizeof(zc) * (double)th * (2 + d);
-    c->cr_envs = (int)std::max(1.0, std::min({(double)c->L, 32768.0, std::floor(kCrBudget / per)}));
-    c->cr_chains = std::max(1, std::min(nch, c->cr_envs / Lc));
-    HIPCHK(c, hipMalloc(&c->cr_theta[0], sizeof(zc) * th * c->cr_envs));
-    HIPCHK(c, hipMalloc(&c->cr_theta[1], sizeof(zc) * th * c->cr_envs));
-    HIPCHK(c, hipMalloc(&c->cr_T, sizeof(zc) * th * d * c->cr_envs));
-    HIPCHK(c, hipMalloc(&c->cr_B, sizeof(zc) * fac * c->cr_chains));
-    HIPCHK(c, hipMalloc(&c->cr_A, sizeof(zc) * fac * c->cr_chains));
-    HIPCHK(c, hipMalloc(&c->cr_phase, sizeof(double) * d));
-    HIPCHK(c, hipMalloc(&c->cr_rho2, sizeof(zc) * d4 * np * nch));
-    HIPCHK(c, hipMalloc(&c->cr_rho1, sizeof(zc) * d2 * c->L));
-  }
+  if (!c->cr_envs) HIPCHK(c, alloc_rdms(c));
   const double* ph = nullptr;
   if (phase) {
     HIPCHK(c, hipMemcpy(c->cr_phase, phase, sizeof(double) * d, hipMemcpyHostToDevice));
@@ -3311,8 +3374,8 @@ int tebd_two_point_rdms(tebd_ctx* c, const double* phase, double* rho2, double* 
       (void)hipHostFree(c->cr_hdesc);
       c->cr_desc = c->cr_hdesc = nullptr;
       c->cr_desc_bytes = 0;
-      HIPCHK(c, hipMalloc(&c->cr_desc, bytes));
-      HIPCHK(c, hipHostMalloc(&c->cr_hdesc, bytes));
+      HIPCHK(c, alloc_n(&c->cr_desc, bytes));
+      HIPCHK(c, alloc_pinned(&c->cr_hdesc, bytes));
       c->cr_desc_bytes = bytes;
     }
     auto put = [&](size_t off, const void* src, size_t n) { if (n) std::memcpy(c->cr_hdesc + off, src, n); };

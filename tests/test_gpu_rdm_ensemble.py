@@ -1,7 +1,9 @@
-"""All-pairs density matrices of an ensemble with more sites than a grid's second dimension holds.
+"""All-pairs density matrices of an ensemble with more sites than a grid's second dimension is
+specified to hold.
 
-8200 chains of 8 spins: 65600 environments, while a launch takes 65535 rows of workgroups.  On
-product states every matrix is the product of the two sites' own, which is exact: 1e-13.
+8200 chains of 8 spins: 65600 environments, while HIP gives 65536 as the most workgroups of a launch's
+second and third dimensions.  On product states every matrix is the product of the two sites' own,
+which is exact: 1e-13.
 """
 import numpy as np
 import pytest
