@@ -501,8 +501,12 @@ int slot_of(const tebd_ctx* c, const BondTask& t) { return (int)((t.qstate - c->
 // Column-pivoted Householder QR of every task's bond matrix, stopped at the
 // numerical rank.  Returns the ranks in rank[].
 int qrp_factor(tebd_ctx* c, BondTask* D, const BondTask* H, int nb, int max_cb, std::vector<int>& rank) {
-  int max_rb = 1;
-  for (int i = 0; i < nb; ++i) max_rb = std::max(max_rb, H[i].Rb);
+  int max_rb = 0;
+  bool large = false;
+  for (int i = 0; i < nb; ++i) {
+    if (H[i].Rb > kQrRegRows) large = true;
+    else max_rb = std::max(max_rb, H[i].Rb);
+  }
   HIPCHK(c, launch_qrp_begin(D, nb, max_cb, kQrTol, c->st));
   // every task's last panel (j0 + width >= min(Rb, Cb)) records its rank, so after the
   // panel with j0 + kQrPanel >= max_cb all tasks have finished
@@ -510,11 +514,11 @@ int qrp_factor(tebd_ctx* c, BondTask* D, const BondTask* H, int nb, int max_cb, 
   for (int j0 = 0, panel = 0; !done; j0 += kQrPanel, ++panel) {
     {
       ProfScope ps(c, 3);
-      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, max_cb, j0, H[0].cyclic != 0, c->st));
+      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, large, max_cb, j0, H[0].cyclic != 0, c->st));
     }
     {
       ProfScope ps(c, 6);
-      HIPCHK(c, launch_qrp_trailing(D, nb, max_rb, max_cb, j0, c->st));
+      HIPCHK(c, launch_qrp_trailing(D, nb, max_rb, large, max_cb, j0, c->st));
     }
     const bool last = j0 + kQrPanel >= max_cb;
     if ((panel + 1) % kQrCheck == 0 || last) {

@@ -662,13 +662,13 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
 
-// One workgroup per task; the shape of its panel depends on the task's own row count, so a
-// task is factorised the same way whatever batch it is in.  Waves that a task does not need
-// leave at once.
+// One workgroup per task; the shape of its panel, and whether it is this kernel or k_qrp_panel,
+// depend on the task's own row count, so a task is factorised the same way whatever batch it is
+// in.  Waves that a task does not need leave at once.
 template <int NWMAX, bool CYCLIC>
 __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
-  if (t.qstate[0] >= 0.0) return;
+  if (t.Rb > kQrRegRows || t.qstate[0] >= 0.0) return;
   const int kmax = t.Rb < t.Cb ? t.Rb : t.Cb;
   if (j0 >= kmax) {
     if (threadIdx.x == 0) t.qstate[0] = (double)kmax;
@@ -691,13 +691,13 @@ __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __
   }
 }
 
-// Panel j0 through global memory (any Rb; one workgroup of 256 threads per task): the
+// Panel j0 through global memory (Rb > kQrRegRows; one workgroup of 256 threads per task): the
 // same selection, column moves, factorisation and T as k_qrp_panel_reg, with the
 // reflector applied column by column (one wave per column).
 template <bool CYCLIC>
 __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
-  if (t.qstate[0] >= 0.0) return;
+  if (t.Rb <= kQrRegRows || t.qstate[0] >= 0.0) return;
   const int kmax = t.Rb < t.Cb ? t.Rb : t.Cb;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (j0 >= kmax) {
@@ -789,7 +789,7 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
 }
 
 // Block reflector of one panel on 32 columns per workgroup (FP64 MFMA):
-//   MODE 0  trailing update of panel j0 = arg: A2 <- Q_p^H A2 = A2 - V (T^H (V^H A2)) on the
+//   MODE 0  (tasks of more than kQrRegRows rows) trailing update of panel j0 = arg: A2 <- Q_p^H A2 = A2 - V (T^H (V^H A2)) on the
 //           columns right of the panel, and the exact remaining norms |A2(j0+nbp:, c)|^2
 //           into qnrm;
 //   MODE 1  panel p = arg of the factor applied to the Rb-side vectors Yr (k columns):
@@ -809,6 +809,7 @@ __global__ __launch_bounds__(kReflThreads) void k_qrp_reflect(const BondTask* __
   const size_t ld = t.Rb;
   zc* A2;
   if (MODE == 0) {
+    if (t.Rb <= kQrRegRows) return;
     j0 = arg;
     const double rank = t.qstate[0];
     if (rank >= 0.0 && rank <= (double)j0) return;
@@ -942,6 +943,7 @@ __global__ __launch_bounds__(kReflThreads) void k_qrp_reflect(const BondTask* __
 template <int RB>
 __global__ __launch_bounds__(kReflThreads) void k_qrp_trailing_reg(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.y];
+  if (t.Rb > kQrRegRows) return;
   const double rank = t.qstate[0];
   if (rank >= 0.0 && rank <= (double)j0) return;
   const int kmax = t.Rb < t.Cb ? t.Rb : t.Cb;
@@ -1233,31 +1235,38 @@ hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, dou
   return hipGetLastError();
 }
 
-hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, bool cyclic,
+hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0, bool cyclic,
                             hipStream_t st) {
   if (max_cb > kMaxCols) return hipErrorInvalidValue;
   const auto k2 = cyclic ? k_qrp_panel_reg<2, true> : k_qrp_panel_reg<2, false>;
   const auto k4 = cyclic ? k_qrp_panel_reg<4, true> : k_qrp_panel_reg<4, false>;
   const auto k8 = cyclic ? k_qrp_panel_reg<8, true> : k_qrp_panel_reg<8, false>;
-  if (max_rb <= 128) hipLaunchKernelGGL(k2, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
-  else if (max_rb <= 256) hipLaunchKernelGGL(k4, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
-  else if (max_rb <= 1024) hipLaunchKernelGGL(k8, dim3(ntasks), dim3(512), 0, st, d_tasks, j0);
-  else {
-    const auto k = cyclic ? k_qrp_panel<true> : k_qrp_panel<false>;
-    hipLaunchKernelGGL(k, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+  if (max_rb > 0) {
+    if (max_rb <= 128) hipLaunchKernelGGL(k2, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
+    else if (max_rb <= 256) hipLaunchKernelGGL(k4, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
+    else hipLaunchKernelGGL(k8, dim3(ntasks), dim3(512), 0, st, d_tasks, j0);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
+  if (!large) return hipSuccess;
+  const auto k = cyclic ? k_qrp_panel<true> : k_qrp_panel<false>;
+  hipLaunchKernelGGL(k, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
   return hipGetLastError();
 }
 
-hipError_t launch_qrp_trailing(const BondTask* d_tasks, int ntasks, int max_rb, int max_cb, int j0, hipStream_t st) {
+hipError_t launch_qrp_trailing(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0,
+                               hipStream_t st) {
   if (j0 + QB >= max_cb) return hipSuccess;
-  const dim3 g16((max_cb - j0 - 1) / 16 + 1, ntasks);
-  if (max_rb <= 256) hipLaunchKernelGGL(k_qrp_trailing_reg<2>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
-  else if (max_rb <= 512) hipLaunchKernelGGL(k_qrp_trailing_reg<4>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
-  else if (max_rb <= 1024) hipLaunchKernelGGL(k_qrp_trailing_reg<8>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
-  else
-    hipLaunchKernelGGL(k_qrp_reflect<0>, dim3((max_cb - j0 - 1) / 32 + 1, ntasks), dim3(kReflThreads), 0, st,
-                       d_tasks, j0);
+  if (max_rb > 0) {
+    const dim3 g16((max_cb - j0 - 1) / 16 + 1, ntasks);
+    if (max_rb <= 256) hipLaunchKernelGGL(k_qrp_trailing_reg<2>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
+    else if (max_rb <= 512) hipLaunchKernelGGL(k_qrp_trailing_reg<4>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
+    else hipLaunchKernelGGL(k_qrp_trailing_reg<8>, g16, dim3(kReflThreads), 0, st, d_tasks, j0);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!large) return hipSuccess;
+  hipLaunchKernelGGL(k_qrp_reflect<0>, dim3((max_cb - j0 - 1) / 32 + 1, ntasks), dim3(kReflThreads), 0, st, d_tasks, j0);
   return hipGetLastError();
 }
 
