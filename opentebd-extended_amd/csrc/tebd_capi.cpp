@@ -37,12 +37,13 @@ constexpr int kNumProf = 28;
 constexpr double kQrTol = 1e-17;  // QR stops when every remaining column norm is <= kQrTol ||theta||_F
 constexpr int kQrPanel = 16;      // panel width of the blocked pivoted QR (tebd_qrp.hip)
 constexpr int kQrCheck = 8;       // panels between checks whether every task has stopped
-// Bond matrices with no side of at least kQrMinSide go straight to the Jacobi, solved in one
-// launch (tebd_jacobi_small.hip).  A chain's edge bonds (4 x 256, say) are preconditioned with the
-// bulk's: on their own they held up the half-sweep by 160-320 us.
+// Bond matrices with no side of at least kQrMinSide go straight to the Jacobi, with whole cyclic sweeps
+// per pair visit: bonds this small keep their smallest Schmidt vectors, which the Vidal form divides by
+// lambda ~ 1e-14, as accurate as they were.  A chain's edge bonds (4 x 256, say) are preconditioned with
+// the bulk's: on their own they held up the half-sweep by 160-320 us.
 constexpr int kQrMinSide = 64;
-// CanonicalForm's SVDs of at most 32 columns and this many rows are solved in one launch too; more
-// rows or columns are more work than one workgroup should have.  Canonical form of 8 sites of d = 4,
+// CanonicalForm's SVDs of one pair of column blocks and this many rows may be one launch too; more rows
+// are more work than one workgroup should have.  Canonical form of 8 sites of d = 4,
 // chi = 60 (240 x 60): all sweep by sweep 22 ms, all in one launch 30; of 10 sites of d = 2, chi =
 // 32 (64 x 32): 11.5 and 9.
 constexpr int kSmallFormRows = 64;
@@ -363,12 +364,11 @@ hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int c
   return ge;
 }
 
-// After the tasks' counters have reached h_counters: checks that the small solves converged
-// and adds every task's work to the statistics.  `sweeps`: sweeps of the large solves, which
-// have already entered their rotations per sweep.
-int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, int sweeps, bool converged) {
-  for (int i = 0; i < nb; ++i) {
-    if (!h_t[i].small) continue;
+// After the tasks' counters have reached h_counters: adds every task's work to the statistics and
+// reports a solve that has not converged.  One-launch solves bring their own sweeps; `sweeps` and
+// `converged` are those of the others, which have already entered their rotations per sweep.
+int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, bool one_launch, int sweeps, bool converged) {
+  for (int i = 0; i < nb && one_launch; ++i) {
     const int* cnt = c->h_counters + kCounters * i;
     if (cnt[4] < 1) converged = false;
     sweeps = std::max(sweeps, cnt[4]);
@@ -382,8 +382,8 @@ int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, int sweeps, bool co
     const double rows = t.R + (t.V ? t.NV : 0);
     c->stats[8] += visits;
     c->stats[9] += rots;
-    c->stats[10] += (double)(t.small ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
-    if (c->profiling && !t.small) {
+    c->stats[10] += (double)(one_launch ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
+    if (c->profiling && !one_launch) {
       // k_jacobi_round, per formed Gram: the 16x16 cross block over R rows (8 flops per
       // complex MAC) reading the pair's JC columns once, and per rotated pair its JC x JC
       // rotation written; k_jacobi_rotate, per rotated pair: the JC columns of W and V
@@ -402,26 +402,22 @@ hipError_t fetch_counters(tebd_ctx* c, int nb) {
   return hipMemcpyAsync(c->h_counters, c->counters, sizeof(int) * kCounters * nb, hipMemcpyDeviceToHost, c->st);
 }
 
-// Jacobi SVDs of the tasks of one stage (task i uses slot i): the small ones in one launch,
-// the others sweep by sweep until one rotates nothing.  When every task is small nothing is
-// waited for: *deferred is set, the counters' copy to the host is queued, and the caller
-// calls jacobi_account after its next wait.
+// Jacobi SVDs of the tasks of one stage (task i uses slot i): in one launch when every task may be
+// (BondTask::small), else sweep by sweep until one rotates nothing.  After one launch nothing is
+// waited for: *deferred is set, the counters' copy to the host is queued, and the caller calls
+// jacobi_account after its next wait.
 int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool* deferred) {
   HIPCHK(c, launch_jacobi_begin(d_t, nb, c->st));
-  int rows_w = 1, rows_v = 0, Pmax = 0;
-  bool one = false, two = false;
+  int rows_w = 1, rows_v = 0, Pmax = 1;
+  *deferred = true;
   for (int i = 0; i < nb; ++i) {
-    if (h_t[i].small) {
-      (h_t[i].P == 1 ? one : two) = true;
-      continue;
-    }
+    *deferred = *deferred && h_t[i].small;
     Pmax = std::max(Pmax, h_t[i].P);
     rows_w = std::max(rows_w, h_t[i].R);
     if (h_t[i].V) rows_v = std::max(rows_v, h_t[i].NV);
   }
-  if (one || two) HIPCHK(c, launch_jacobi_small(d_t, nb, one, two, kTolRel, kTolAbs, kMaxSweeps, c->st));
-  *deferred = Pmax == 0;
   if (*deferred) {
+    HIPCHK(c, launch_jacobi_small(d_t, nb, kTolRel, kTolAbs, kMaxSweeps, c->st));
     HIPCHK(c, fetch_counters(c, nb));
     return TEBD_OK;
   }
@@ -473,7 +469,7 @@ int jacobi_sweeps(tebd_ctx* c, BondTask* d_t, const BondTask* h_t, int nb, bool*
     c->stats[14 + std::min(sweeps, kSweepHist - 1)] += rot;
     ++sweeps;
   }
-  return jacobi_account(c, h_t, nb, sweeps, converged);
+  return jacobi_account(c, h_t, nb, false, sweeps, converged);
 }
 
 // Compact-WY factors kept per slot: one kQrPanel^2 block per panel, min(Rb, Cb) <= Cpmax.
@@ -514,7 +510,7 @@ int qrp_factor(tebd_ctx* c, BondTask* D, const BondTask* H, int nb, int max_cb, 
   for (int j0 = 0, panel = 0; !done; j0 += kQrPanel, ++panel) {
     {
       ProfScope ps(c, 3);
-      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, large, max_cb, j0, H[0].cyclic != 0, c->st));
+      HIPCHK(c, launch_qrp_panel(D, nb, max_rb, large, max_cb, j0, H[0].normed != 0, c->st));
     }
     {
       ProfScope ps(c, 6);
@@ -569,7 +565,7 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
   // which other bonds share its batch.
   std::vector<int> qidx;
   for (int i = 0; i < nb; ++i)
-    if (force_qr || (H[i].cyclic ? H[i].Cb : H[i].Rb) >= kQrMinSide) qidx.push_back(i);
+    if (force_qr || (H[i].normed ? H[i].Cb : H[i].Rb) >= kQrMinSide) qidx.push_back(i);
   const int nq = (int)qidx.size();
   const bool use_qr = nq > 0;
   int max_rank = 1;
@@ -597,6 +593,7 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
       max_rank = std::max(max_rank, rank[j]);
       BondTask& t = H[i];
       t.qr = 1;
+      t.cyclic = t.normed;
       t.small = 0;
       t.W = c->X + (size_t)slot_of(c, t) * c->Cpmax * c->Cpmax;
       t.R = t.Cb;
@@ -624,7 +621,7 @@ int svd_factor(tebd_ctx* c, BondTask* D, BondTask* H, const int* links, int nb, 
   HIPCHK(c, hipMemcpyAsync(c->h_results, c->results, sizeof(double) * RESULT_STRIDE * nb, hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   if (deferred) {
-    int e = jacobi_account(c, H, nb, 0, true);
+    int e = jacobi_account(c, H, nb, true, 0, true);
     if (e) return e;
   }
   *max_k = 1;
@@ -833,7 +830,8 @@ void make_full_task(tebd_ctx* c, BondTask& t, int link, const zc* gate, int slot
   t.C = std::min(m, n);
   t.Cpad = round_up(t.C, JC);
   t.P = t.Cpad / JC;
-  t.small = t.R < kQrMinSide;
+  t.cyclic = t.R < kQrMinSide;
+  t.small = t.cyclic && t.P == 1;
   t.gl = c->gam + (size_t)link * c->gslab();
   t.gr = c->gam + (size_t)(link + 1) * c->gslab();
   t.ll = c->lam + (size_t)link * c->chi_max;
@@ -1304,7 +1302,7 @@ int device_svd_batch(tebd_ctx* c, const SvdJob* jobs, int nb) {
   if (e) return e;
   if (deferred) {  // the task descriptors are rewritten by the next batch: wait here as after a sweep
     HIPCHK(c, hipStreamSynchronize(c->st));
-    if ((e = jacobi_account(c, c->h_tasks, nb, 0, true))) return e;
+    if ((e = jacobi_account(c, c->h_tasks, nb, true, 0, true))) return e;
   }
   HIPCHK(c, launch_col_norms(c->d_tasks, nb, Cpmax, c->st));
   HIPCHK(c, launch_truncate(c->d_tasks, nb, 0.0, c->st));
@@ -1702,7 +1700,7 @@ int run_bonds_nc(tebd_ctx* c, const int* links, int nb, const zc* const* gate_pt
         BondTask& t = S[q];
         std::memset(&t, 0, sizeof(t));
         t.d = d;
-        t.cyclic = 1;
+        t.cyclic = t.normed = 1;
         t.link = links[blk_bond[live[q0 + q]]];
         t.R = b.R;
         t.C = std::min(b.lgt, b.trv);
@@ -3225,7 +3223,8 @@ int tebd_two_site_op_noalloc(int d, int chi_l, int chi_c, int chi_r, int chi_cap
   t.C = std::min(m, n);
   t.Cpad = round_up(t.C, JC);
   t.P = t.Cpad / JC;
-  t.small = t.R < kQrMinSide;
+  t.cyclic = t.R < kQrMinSide;
+  t.small = t.cyclic && t.P == 1;
   t.gl = (const zc*)gamma_l;
   t.gr = (const zc*)gamma_r;
   t.ll = lambda_l;

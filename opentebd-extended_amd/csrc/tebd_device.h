@@ -191,8 +191,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 constexpr int JB = 16;
 constexpr int JC = 2 * JB;
 // Ints per task of BondTask::counter: [0..1] rotated pairs per sweep parity, [2] Gram visits,
-// [3] rotations; of a small solve (tebd_jacobi_small.hip) [4] sweeps run (0: not converged)
-// and [8 + s] pairs rotated in sweep s (the last bin: that sweep and later ones).
+// [3] rotations; of a one-launch solve (tebd_jacobi_small.hip) [4] sweeps run (0: not converged; 1
+// for the other solves) and [8 + s] pairs rotated in sweep s (the last bin: that sweep and later ones).
 constexpr int kSweepBins = 16;
 constexpr int kCounters = 8 + kSweepBins;
 
@@ -231,9 +231,9 @@ struct BondTask {
   // column-pivoted QR preconditioning (qr = 1): Wq (Rb x Cb) holds the bond matrix and then its
   // Householder QR; the Jacobi (W, R, C above) runs on X = R(0:r, :)^dagger (Cb x r)
   int qr;
-  int cyclic;        // 1: every pair visit of the Jacobi runs whole cyclic sweeps (inner_solve) and a QR
-                     // panel reduces a column's norm by itself (reflectors_of_norm)
-  int small;         // 1: the whole Jacobi solve in one launch (tebd_jacobi_small.hip); P <= kSmallPairs
+  int cyclic;        // 1: every pair visit of the Jacobi runs whole cyclic sweeps (inner_solve)
+  int small;         // 1: P = 1 and cyclic: the Jacobi may be one launch (tebd_jacobi_small.hip)
+  int normed;        // 1: a QR panel reduces a column's norm by itself (reflectors_of_norm)
   int Rb, Cb;
   zc* Wq;
   double* qnrm;      // Cb remaining column norms^2
@@ -247,5 +247,3 @@ struct BondTask {
   const double* wtot;  // when set, the reference total weight (||theta||^2) for the truncation
   int rng_key;       // sketch stream of the bond: its position in its chain (not its batch slot)
 };
-
-constexpr int kSmallPairs = 2;  // most pairs of column blocks of a small solve

@@ -220,7 +220,6 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   const BondTask t = tasks[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= t.P || round >= 2 * t.P - 1) return;
-  if (t.small) return;  // solved by k_jacobi_small
   int* cnt = t.counter;
   if (sweep > 0 && cnt[(sweep - 1) & 1] == 0) return;  // converged in the previous sweep
   const int nblk = 2 * t.P;
@@ -262,12 +261,12 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
         L.A[blk * JB + r][blk * JB + c] = zmk(0.0, 0.0);
       }
     }
-    reduce_block(L, true, gre, gim, tid, 0, JB, false);
+    reduce_block(L, gre, gim, tid, 0, JB, false);
     if (FULL) {
       gram_block(Wi, Wi, t.R, wave, lane, gre, gim, nx, ny);
-      reduce_block(L, true, gre, gim, tid, 0, 0, true);
+      reduce_block(L, gre, gim, tid, 0, 0, true);
       gram_block(Wj, Wj, t.R, wave, lane, gre, gim, nx, ny);
-      reduce_block(L, true, gre, gim, tid, JB, JB, true);
+      reduce_block(L, gre, gim, tid, JB, JB, true);
     } else {
       if (tid < JC) {
         const int side = tid / JB, col = tid % JB;
@@ -305,7 +304,7 @@ __global__ __launch_bounds__(kRoundThreads) void k_jacobi_round(const BondTask* 
   }
 
   // ---- rotations of A -> Q, to the pair's slot; queue the pair for rotation
-  if (cyclic) inner_solve<true>(L, kRing.rounds, tid, true);
+  if (cyclic) inner_solve(L, kRing.rounds, tid);
   else if constexpr (FULL) inner_jacobi<true>(L, kFull.rounds, tid);
   else inner_jacobi<false>(L, kCross.rounds, tid);
   zc (*Q)[JC + 1] = L.Q;
@@ -393,7 +392,7 @@ __global__ __launch_bounds__(256) void k_jacobi_rotate(const BondTask* __restric
 __global__ void k_jacobi_begin(const BondTask* __restrict__ tasks) {
   const BondTask t = tasks[blockIdx.x];
   const int nblk = 2 * t.P;
-  if (threadIdx.x < kCounters) t.counter[threadIdx.x] = 0;
+  if (threadIdx.x < kCounters) t.counter[threadIdx.x] = threadIdx.x == 4 ? 1 : 0;
   for (int e = threadIdx.x; e < nblk; e += blockDim.x) t.blkver[e] = 0u;
   for (int e = threadIdx.x; e < nblk * nblk; e += blockDim.x) t.pairseen[e] = ~0ull;
 }

@@ -1,7 +1,7 @@
 // A Jacobi pair: its 32 x 32 Hermitian Gram matrix in LDS and rounds of 16 disjoint rotations on
-// it.  Shared by the large solve (tebd_jacobi.hip) and the small one (tebd_jacobi_small.hip): the
-// small one, and the large one where the task asks for it, solve a pair's problem by whole cyclic
-// sweeps (inner_solve); the large one has schedules of its own for a single pass.
+// it.  Shared by the sweep-by-sweep solve (tebd_jacobi.hip) and the one-launch solve
+// (tebd_jacobi_small.hip): the latter, and the former where the task asks for it, solve a pair's
+// problem by whole cyclic sweeps (inner_solve); the former has schedules of its own for a single pass.
 //
 // What bounds a round: a wave64 instruction holds its SIMD for 4 cycles, so a round costs the
 // instructions of its longest wave plus one LDS round trip and one barrier.  With the index
@@ -347,19 +347,17 @@ __device__ __forceinline__ void gram_block(const zc* X, const zc* Y, int R, int 
 
 // Sums the waves' partial blocks in wave order and stores the upper triangle's part of rows
 // [ro, ro+16) x cols [co, co+16) of A (diagonal blocks: the real diagonal goes to dg).  Called
-// by every thread; `on` is uniform per pair.
-__device__ __forceinline__ void reduce_block(PairLds& L, bool on, d4 gre, d4 gim, int pt, int ro, int co, bool diag) {
+// by every thread.
+__device__ __forceinline__ void reduce_block(PairLds& L, d4 gre, d4 gim, int pt, int ro, int co, bool diag) {
 #pragma clang fp contract(off)
   const int wave = pt >> 6, lane = pt & 63;
-  if (on) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      L.g.red[wave][g * 64 + lane] = gre[g];
-      L.g.red[wave][256 + g * 64 + lane] = gim[g];
-    }
+  for (int g = 0; g < 4; ++g) {
+    L.g.red[wave][g * 64 + lane] = gre[g];
+    L.g.red[wave][256 + g * 64 + lane] = gim[g];
   }
   __syncthreads();
-  if (on) {
+  {
     const int idx = pt & 255, l = idx & 63, im = pt >> 8;
     double v = L.g.red[0][pt];
     for (int w = 1; w < kPairWaves; ++w) v += L.g.red[w][pt];
@@ -370,15 +368,13 @@ __device__ __forceinline__ void reduce_block(PairLds& L, bool on, d4 gre, d4 gim
   __syncthreads();
 }
 
-// The 32 x 32 eigenproblems of the workgroup's pairs, by cyclic Jacobi: at most
-// kInnerSweepCap sweeps, ended when a sweep rotates nothing or the next one would.  Waves 0..3 of
-// a pair update A; waves 4..7 apply the round's rotations to Q, held in registers: lane t of a
-// 16-lane row has two rows' entries of Q at ring positions t and 31 - t, and the ring's move by
-// one position per round is a move between neighbouring lanes.  All threads take part in every
-// barrier; pairs that need no rotation, or have finished, only wait (ONE_PAIR: the workgroup has no
-// other pair to wait for and ends the solve).
-template <bool ONE_PAIR, class Rounds>
-__device__ __forceinline__ void inner_solve(PairLds& L, const Rounds& T, int pt, bool on) {
+// The pair's 32 x 32 eigenproblem by cyclic Jacobi: at most kInnerSweepCap sweeps, ended when a sweep
+// rotates nothing or the next one would not.  Waves 0..3 update A; waves 4..7 apply the round's
+// rotations to Q, held in registers: lane t of a 16-lane row has two rows' entries of Q at ring
+// positions t and 31 - t, and the ring's move by one position per round is a move between
+// neighbouring lanes.
+template <class Rounds>
+__device__ __forceinline__ void inner_solve(PairLds& L, const Rounds& T, int pt) {
 #pragma clang fp contract(off)
   const bool is_q = pt >= 256, is_a = pt < 2 * kOffBlocks;
   const int tr = is_a ? kRing.tr[pt] : 0, tk = is_a ? kRing.tk[pt] : 0, half = pt & 1;
@@ -391,12 +387,11 @@ __device__ __forceinline__ void inner_solve(PairLds& L, const Rounds& T, int pt,
     s[u] = zmk(qk + 16 * u == ring(0, JC - 1 - qt) ? 1.0 : 0.0, 0.0);
   }
   int buf = 0;
-  bool live = on;
 #pragma unroll 1
   for (int isw = 0; isw < kInnerSweepCap; ++isw) {
     if (pt == 0) L.swept[isw & 1] = 0;
     __syncthreads();
-    if (live && pt < JC / 2) {
+    if (pt < JC / 2) {
       const int p = kRing.p[0][pt], q = kRing.q[0][pt];
       L.A[p][q] = make_rotation(L.rb[buf], L.dg[p], L.dg[q], &L.dg[p], &L.dg[q], &L.swept[isw & 1], pt, L.A[p][q], jrot);
     }
@@ -405,8 +400,7 @@ __device__ __forceinline__ void inner_solve(PairLds& L, const Rounds& T, int pt,
 #pragma unroll 1
     for (int rd = 0; rd < kAllRounds; ++rd, buf ^= 1) {
       const RotBuf& R = L.rb[buf];
-      if (!live) {
-      } else if (is_q) {
+      if (is_q) {
         // with p the lower of the pair's indices: Q_:p <- c Q_:p - s conj(w) Q_:q ; Q_:q <- s w Q_:p
         // + c Q_:q.  f and s take the two roles as fp says; the signs go into x, and only the
         // imaginary parts' products change their order of rounding with the roles.
@@ -442,17 +436,16 @@ __device__ __forceinline__ void inner_solve(PairLds& L, const Rounds& T, int pt,
     // would the next sweep rotate anything?
     if (pt == 0) L.more = 0;
     __syncthreads();
-    if (live && L.swept[isw & 1])
+    if (L.swept[isw & 1])
       for (int e = pt; e < JC * JC; e += kPairThreads) {
         const int pp = e % JC, qq = e / JC;
         if (pp < qq && needs_rotation(abs2(L.A[pp][qq]), L.dg[pp], L.dg[qq])) L.more = 1;
       }
     __syncthreads();
-    if (live && !L.more) live = false;
-    if (ONE_PAIR && !live) break;
+    if (!L.more) break;
   }
   // after whole sweeps the ring is back at its start
-  if (on && is_q) {
+  if (is_q) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       L.Q[qk + 16 * u][ring(0, qt)] = f[u];

@@ -21,17 +21,17 @@ hipError_t launch_jacobi_round(const BondTask* d_tasks, int ntasks, int max_pair
                                int wl_cap, hipStream_t st);
 hipError_t launch_jacobi_rotate(const BondTask* d_tasks, int round, int max_rows_w, int max_rows_v, int* wl_count,
                                 int2* wl_items, int wl_cap, hipStream_t st);
-// The whole solve of every task with BondTask::small, one launch per pair count present in the batch.
-hipError_t launch_jacobi_small(const BondTask* d_tasks, int ntasks, bool one_pair, bool two_pairs, double tol_rel,
-                               double tol_abs, int max_sweeps, hipStream_t st);
+// The whole solve of every task in one launch; every task has BondTask::small.
+hipError_t launch_jacobi_small(const BondTask* d_tasks, int ntasks, double tol_rel, double tol_abs, int max_sweeps,
+                               hipStream_t st);
 hipError_t launch_qrp_trailing(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0,
                                hipStream_t st);
 hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, double tol_rel, hipStream_t st);
 // Tasks of up to kQrRegRows rows are factorised in registers, the others through global memory.
-// max_rb: the most rows among the former (0: none), large: there are others; cyclic:
-// BondTask::cyclic of every task of the batch.
+// max_rb: the most rows among the former (0: none), large: there are others; normed:
+// BondTask::normed of every task of the batch.
 constexpr int kQrRegRows = 1024;
-hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0, bool cyclic,
+hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0, bool normed,
                             hipStream_t st);
 hipError_t launch_qrp_build_x(const BondTask* d_tasks, int ntasks, hipStream_t st);
 hipError_t launch_qrp_vectors(const BondTask* d_tasks, int ntasks, int max_k, int max_r, hipStream_t st);

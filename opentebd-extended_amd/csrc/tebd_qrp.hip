@@ -533,9 +533,9 @@ __device__ __forceinline__ void reflectors_of_norm(zc (&a)[RPT][QB], PanelLds& S
 // norms for the selection and T column by column, a panel took 52 us at 128 rows, 65 at 225 and
 // 73 at 400; now 28, 31 and 37 (at 64: 27), of which the chain is 21, 23 and 26, the selection 3,
 // 3 and 5 and T 2.
-// CYCLIC (BondTask::cyclic, the number blocks): the norms, products and T in the order of
+// NORMED (BondTask::normed, the number blocks): the norms, products and T in the order of
 // reflectors_of_norm and form_t_rows, for the reason given in tebd_jacobi.hip.
-template <int RPT, int NW, bool CYCLIC>
+template <int RPT, int NW, bool NORMED>
 __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S) {
   constexpr int NT = 64 * NW;
   const int Rb = t.Rb, Cb = t.Cb;
@@ -571,7 +571,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
   // 3. Householder QR of the panel, the column loop unrolled so that every register
   // index is static: column q sits in a[.][q], first as data, then as reflector v_q
   // (rows > j0 + q) below R(:, q).
-  if constexpr (CYCLIC) reflectors_of_norm<RPT, NW>(a, S, j0, nbp, Rb, tid);
+  if constexpr (NORMED) reflectors_of_norm<RPT, NW>(a, S, j0, nbp, Rb, tid);
   else static_for<QB>([&](auto qc) {
     constexpr int q = decltype(qc)::value, buf = q & 1;
     if (q >= nbp) return;
@@ -657,7 +657,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
     }
   }
   if (tid < nbp) t.tau[j0 + tid] = S.stau[tid];
-  if constexpr (CYCLIC) form_t_rows(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  if constexpr (NORMED) form_t_rows(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
   else form_t(S.G, S.stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, S.Tm, S.X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
@@ -665,7 +665,7 @@ __device__ __forceinline__ void panel_reg(const BondTask& t, int j0, PanelLds& S
 // One workgroup per task; the shape of its panel, and whether it is this kernel or k_qrp_panel,
 // depend on the task's own row count, so a task is factorised the same way whatever batch it is
 // in.  Waves that a task does not need leave at once.
-template <int NWMAX, bool CYCLIC>
+template <int NWMAX, bool NORMED>
 __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
   if (t.Rb > kQrRegRows || t.qstate[0] >= 0.0) return;
@@ -677,24 +677,24 @@ __global__ __launch_bounds__(64 * NWMAX) void k_qrp_panel_reg(const BondTask* __
   __shared__ PanelLds S;
   const int wave = threadIdx.x >> 6;
   constexpr int N4 = NWMAX < 4 ? NWMAX : 4;
-  if (!CYCLIC && t.Rb <= 64 && t.Cb <= 64) {  // no barriers: 28 us instead of 31 at 64 x 64; more candidates need more threads
-    if (wave < 1) panel_reg<1, 1, CYCLIC>(t, j0, S);
+  if (!NORMED && t.Rb <= 64 && t.Cb <= 64) {  // no barriers: 28 us instead of 31 at 64 x 64; more candidates need more threads
+    if (wave < 1) panel_reg<1, 1, NORMED>(t, j0, S);
   } else if (t.Rb <= 128) {
-    if (wave < 2) panel_reg<1, 2, CYCLIC>(t, j0, S);
+    if (wave < 2) panel_reg<1, 2, NORMED>(t, j0, S);
   } else if (NWMAX >= 4 && t.Rb <= 256) {
-    if (wave < 4) panel_reg<1, N4, CYCLIC>(t, j0, S);
+    if (wave < 4) panel_reg<1, N4, NORMED>(t, j0, S);
   } else if (NWMAX >= 8 && t.Rb <= 512) {
-    if constexpr (CYCLIC) panel_reg<1, NWMAX, CYCLIC>(t, j0, S);
-    else if (wave < 4) panel_reg<2, N4, CYCLIC>(t, j0, S);
+    if constexpr (NORMED) panel_reg<1, NWMAX, NORMED>(t, j0, S);
+    else if (wave < 4) panel_reg<2, N4, NORMED>(t, j0, S);
   } else if (NWMAX >= 8) {
-    panel_reg<2, NWMAX, CYCLIC>(t, j0, S);
+    panel_reg<2, NWMAX, NORMED>(t, j0, S);
   }
 }
 
 // Panel j0 through global memory (Rb > kQrRegRows; one workgroup of 256 threads per task): the
 // same selection, column moves, factorisation and T as k_qrp_panel_reg, with the
 // reflector applied column by column (one wave per column).
-template <bool CYCLIC>
+template <bool NORMED>
 __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ tasks, int j0) {
   const BondTask t = tasks[blockIdx.x];
   if (t.Rb <= kQrRegRows || t.qstate[0] >= 0.0) return;
@@ -746,7 +746,7 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
     const zc alpha = cj[j];
     zc tau, scale = zmk(1.0, 0.0);
     double beta = 0.0;
-    const bool refl = householder<CYCLIC>(alpha, xn2, tau, beta, scale);
+    const bool refl = householder<NORMED>(alpha, xn2, tau, beta, scale);
     __syncthreads();  // every thread has read alpha
     if (refl) {
       for (int i = j + 1 + tid; i < t.Rb; i += 256) cj[i] = zmul(cj[i], scale);
@@ -783,7 +783,7 @@ __global__ __launch_bounds__(256) void k_qrp_panel(const BondTask* __restrict__ 
     gram_partial<1, 1>(vload, vload, K, wave, 4, lane, gre, gim);
     gram_reduce<1, 1>(gre, gim, gred, &G[0][0], QB + 1, wave, lane);
   }
-  if constexpr (CYCLIC) form_t_rows(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
+  if constexpr (NORMED) form_t_rows(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB);
   else form_t(G, stau, nbp, t.Tq + (size_t)(j0 / QB) * QB * QB, Tm, X);
   if (tid == 0 && j0 + nbp >= kmax) t.qstate[0] = (double)kmax;
 }
@@ -1235,12 +1235,12 @@ hipError_t launch_qrp_begin(const BondTask* d_tasks, int ntasks, int max_cb, dou
   return hipGetLastError();
 }
 
-hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0, bool cyclic,
+hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, bool large, int max_cb, int j0, bool normed,
                             hipStream_t st) {
   if (max_cb > kMaxCols) return hipErrorInvalidValue;
-  const auto k2 = cyclic ? k_qrp_panel_reg<2, true> : k_qrp_panel_reg<2, false>;
-  const auto k4 = cyclic ? k_qrp_panel_reg<4, true> : k_qrp_panel_reg<4, false>;
-  const auto k8 = cyclic ? k_qrp_panel_reg<8, true> : k_qrp_panel_reg<8, false>;
+  const auto k2 = normed ? k_qrp_panel_reg<2, true> : k_qrp_panel_reg<2, false>;
+  const auto k4 = normed ? k_qrp_panel_reg<4, true> : k_qrp_panel_reg<4, false>;
+  const auto k8 = normed ? k_qrp_panel_reg<8, true> : k_qrp_panel_reg<8, false>;
   if (max_rb > 0) {
     if (max_rb <= 128) hipLaunchKernelGGL(k2, dim3(ntasks), dim3(128), 0, st, d_tasks, j0);
     else if (max_rb <= 256) hipLaunchKernelGGL(k4, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
@@ -1249,7 +1249,7 @@ hipError_t launch_qrp_panel(const BondTask* d_tasks, int ntasks, int max_rb, boo
     if (e != hipSuccess) return e;
   }
   if (!large) return hipSuccess;
-  const auto k = cyclic ? k_qrp_panel<true> : k_qrp_panel<false>;
+  const auto k = normed ? k_qrp_panel<true> : k_qrp_panel<false>;
   hipLaunchKernelGGL(k, dim3(ntasks), dim3(256), 0, st, d_tasks, j0);
   return hipGetLastError();
 }
