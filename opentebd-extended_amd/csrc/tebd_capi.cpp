@@ -31,7 +31,7 @@ constexpr int kGemmRegions = 8;  // GEMM descriptor arrays per batch (learned pa
 // 1/kProbeSafety of the true value with probability
 // P(Gamma(16, 1) < 1.6) = P(Poisson(1.6) >= 16) < 2e-11.
 constexpr double kProbeSafety = 10.0;
-constexpr int kSweepHist = kSweepBins;              // sweeps tallied one by one in the histograms
+constexpr int kSweepHist = 16;                      // sweeps tallied one by one in the histograms
 constexpr int kNumStats = 14 + 2 * kSweepHist;
 constexpr int kNumProf = 28;
 constexpr double kQrTol = 1e-17;  // QR stops when every remaining column norm is <= kQrTol ||theta||_F
@@ -369,10 +369,10 @@ hipGraphExec_t capture_sweep(tebd_ctx* c, BondTask* d_t, int nb, int Pmax, int c
 // `converged` are those of the others, which have already entered their rotations per sweep.
 int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, bool one_launch, int sweeps, bool converged) {
   for (int i = 0; i < nb && one_launch; ++i) {
-    const int* cnt = c->h_counters + kCounters * i;
-    if (cnt[4] < 1) converged = false;
-    sweeps = std::max(sweeps, cnt[4]);
-    for (int s = 0; s < kSweepHist; ++s) c->stats[14 + s] += cnt[8 + s];
+    const int* cnt = c->h_counters + kCounters * i;  // one pair: a Gram per sweep
+    if (cnt[3] == cnt[2]) converged = false;
+    sweeps = std::max(sweeps, cnt[2]);
+    for (int s = 0; s < cnt[3]; ++s) c->stats[14 + std::min(s, kSweepHist - 1)] += 1;
   }
   c->stats[1] += sweeps;
   if (sweeps > 0) c->stats[14 + kSweepHist + std::min(sweeps, kSweepHist) - 1] += 1;
@@ -382,7 +382,7 @@ int jacobi_account(tebd_ctx* c, const BondTask* h_t, int nb, bool one_launch, in
     const double rows = t.R + (t.V ? t.NV : 0);
     c->stats[8] += visits;
     c->stats[9] += rots;
-    c->stats[10] += (double)(one_launch ? c->h_counters[kCounters * i + 4] : sweeps) * t.P * (2 * t.P - 1);
+    c->stats[10] += (one_launch ? visits : (double)sweeps) * t.P * (2 * t.P - 1);
     if (c->profiling && !one_launch) {
       // k_jacobi_round, per formed Gram: the 16x16 cross block over R rows (8 flops per
       // complex MAC) reading the pair's JC columns once, and per rotated pair its JC x JC
@@ -2462,7 +2462,7 @@ constexpr size_t kNoAllocBytes =
     5 * na_up(sizeof(zc) * kNoAllocSide * kNoAllocSide) +                      // W, V, X, Yr, Zc
     2 * na_up(sizeof(double) * kNoAllocSide) + 2 * na_up(sizeof(int) * kNoAllocSide) +  // s, qnrm, perm, qpiv
     na_up(sizeof(zc) * kNoAllocSide) + na_up(sizeof(double) * 2) +              // tau, qstate
-    na_up(sizeof(zc) * kNoAllocTq) + na_up(sizeof(int) * kCounters) +                   // Tq, counters
+    na_up(sizeof(zc) * kNoAllocTq) + na_up(sizeof(int) * kCounters) +           // Tq, counters
     na_up(sizeof(unsigned) * kNoAllocNblk) + na_up(sizeof(unsigned long long) * kNoAllocNblk * kNoAllocNblk) +
     na_up(sizeof(zc) * (kNoAllocNblk / 2) * JC * JC) + na_up(sizeof(int) * 2) +  // Qg, wl_count
     na_up(sizeof(int2) * 2 * (kNoAllocNblk / 2)) + 2 * na_up(sizeof(double) * RESULT_STRIDE) +

@@ -191,10 +191,9 @@ __device__ __forceinline__ double wave_sum(double v) {
 constexpr int JB = 16;
 constexpr int JC = 2 * JB;
 // Ints per task of BondTask::counter: [0..1] rotated pairs per sweep parity, [2] Gram visits,
-// [3] rotations; of a one-launch solve (tebd_jacobi_small.hip) [4] sweeps run (0: not converged; 1
-// for the other solves) and [8 + s] pairs rotated in sweep s (the last bin: that sweep and later ones).
-constexpr int kSweepBins = 16;
-constexpr int kCounters = 8 + kSweepBins;
+// [3] rotations.  A one-launch solve (tebd_jacobi_small.hip: one pair, a Gram per sweep) whose every
+// visit ended in a rotation has not converged; otherwise the last visit of a solve finds nothing.
+constexpr int kCounters = 4;
 
 // One bond update ("task") as the kernels see it.
 struct BondTask {

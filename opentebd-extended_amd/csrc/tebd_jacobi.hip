@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) void k_jacobi_rotate(const BondTask* __restric
 __global__ void k_jacobi_begin(const BondTask* __restrict__ tasks) {
   const BondTask t = tasks[blockIdx.x];
   const int nblk = 2 * t.P;
-  if (threadIdx.x < kCounters) t.counter[threadIdx.x] = threadIdx.x == 4 ? 1 : 0;
+  if (threadIdx.x < kCounters) t.counter[threadIdx.x] = 0;
   for (int e = threadIdx.x; e < nblk; e += blockDim.x) t.blkver[e] = 0u;
   for (int e = threadIdx.x; e < nblk * nblk; e += blockDim.x) t.pairseen[e] = ~0ull;
 }

@@ -55,9 +55,8 @@ __device__ __forceinline__ void rotate_rows(const zc (*Q)[JC + 1], zc* M, int ro
 }
 
 // The whole SVD of every task; every task of the batch has one pair of column blocks.  W and V (global
-// memory, tens of KB, in L2) are rotated in place.  counter[4] = sweeps run (0: not converged within
-// max_sweeps), counter[8 + s] = pairs rotated in sweep s (the last of kSweepBins entries: that sweep and
-// later ones).
+// memory, tens of KB, in L2) are rotated in place.  counter[2] = sweeps run, counter[3] = those that
+// rotated: all of them if the solve has not converged within max_sweeps.
 __global__ __launch_bounds__(kPairThreads) void k_jacobi_small(const BondTask* __restrict__ tasks, double tol_rel,
                                                                double tol_abs, int max_sweeps) {
   const BondTask& t = tasks[blockIdx.x];
@@ -117,12 +116,9 @@ __global__ __launch_bounds__(kPairThreads) void k_jacobi_small(const BondTask* _
     }
     if (sweep == max_sweeps) break;
   }
-  const int rots = done ? sweep - 1 : sweep;
-  if (tid < kSweepBins) t.counter[8 + tid] = tid < kSweepBins - 1 ? (tid < rots ? 1 : 0) : max(0, rots - tid);
   if (tid == 0) {
     t.counter[2] = sweep;
-    t.counter[3] = rots;
-    t.counter[4] = done ? sweep : 0;
+    t.counter[3] = done ? sweep - 1 : sweep;
   }
 }
 

@@ -295,7 +295,7 @@ constexpr int SORT_N = 4096;
 // one workgroup per task: bitonic sort of the squared norms (descending), kept rank,
 // lambda_c and truncerr.  Rule (FormLambda1): keep index < chi_max with
 // s^2/||theta||^2 > cutoff (cutoff >= 1e-30, i.e. |s| > 1e-15 after normalisation).
-// Nothing is written when a one-launch solve of the batch has not converged (its counter[4] is 0):
+// Nothing is written when a one-launch solve of the batch has not converged (every visit rotated):
 // the host learns of it only after this kernel, and lc_out may be the bond's lambda itself.
 __global__ __launch_bounds__(1024) void k_truncate(const BondTask* __restrict__ tasks, double cutoff) {
   const BondTask t = tasks[blockIdx.x];
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(1024) void k_truncate(const BondTask* __restrict__ 
   __shared__ int s_k;
   const int tid = threadIdx.x;
   int failed = 0;
-  for (int i = tid; i < (int)gridDim.x; i += 1024) failed |= tasks[i].small && tasks[i].counter[4] == 0;
+  for (int i = tid; i < (int)gridDim.x; i += 1024) failed |= tasks[i].small && tasks[i].counter[3] == tasks[i].counter[2];
   if (__syncthreads_or(failed)) return;
   int n2 = 1;
   while (n2 < t.Cpad) n2 <<= 1;
