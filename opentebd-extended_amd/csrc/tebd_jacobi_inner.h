@@ -11,12 +11,11 @@
 //     pairs forms that rotation at once, from the value in its registers;
 //   * the threads that do so sit in one wave, the others skip the rotation's code;
 //   * everything that depends only on the round and the thread (LDS offsets, signs, the next
-//     pair) comes from a table in LDS (read from global memory in every round it made each
-//     barrier wait for L2);
+//     pair) comes from a table, read one round ahead so that no barrier waits for L2;
 //   * only the upper triangle of A is kept, each entry is read by one lane, and the two lanes
 //     of a 2x2 block exchange their rows;
-//   * every LDS read of a round is issued before its first product, and the table's entries one
-//     round ahead, so a round waits for LDS once (1405 cycles without).
+//   * every LDS read of a round is issued before its first product, so a round waits for LDS once
+//     (1405 cycles without).
 #pragma once
 #include "tebd_device.h"
 
@@ -101,14 +100,6 @@ constexpr InnerTable<NR, NN> complete_table(InnerTable<NR, NN> t, const int (&fi
     }
   }
   return t;
-}
-
-// The table from constant memory to LDS, by all n threads of the workgroup.
-template <int NR, int NN>
-__device__ __forceinline__ void load_rounds(InnerRounds<NR, NN>& dst, const InnerRounds<NR, NN>& src, int tid, int n) {
-  unsigned* d = &dst.entry[0][0];
-  const unsigned* s = &src.entry[0][0];
-  for (int e = tid; e < (int)(sizeof(dst) / sizeof(unsigned)); e += n) d[e] = s[e];
 }
 
 // Lane moves inside rows of 16 lanes (`edge`: what a lane without a source gets): from the next

@@ -14,6 +14,9 @@
 //   * beside larger bonds the launch is one more step in sequence, while the rounds of one more task
 //     cost nothing: the same chains 8.7, 4.5 and 14.4 ms with all bonds sweep by sweep.
 //
+// The schedule is read from L2 one round ahead: its 34 KB in LDS left a CU one workgroup instead of two
+// (step of 1024 chains of 10 spins, chi = 8: 13.6 ms, 11.2).
+//
 // Every number is formed by the same operations in the same order as sweep by sweep with
 // BondTask::cyclic, so the results do not depend on the choice.
 #include "tebd_device.h"
@@ -61,14 +64,12 @@ __global__ __launch_bounds__(kPairThreads) void k_jacobi_small(const BondTask* _
                                                                double tol_abs, int max_sweeps) {
   const BondTask& t = tasks[blockIdx.x];
   __shared__ PairLds L;
-  __shared__ InnerRounds<kAllRounds, 2 * kInnerPairs> table;
   const int tid = threadIdx.x;
   zc* const W = t.W;
   zc* const V = t.V;
   const int R = t.R, NV = V ? t.NV : 0;
   const zc* Wi = W;
   const zc* Wj = W + (size_t)R * JB;
-  load_rounds(table, kRing.rounds, tid, kPairThreads);
   const double floor = tol_abs * sqrt(t.result[2]);  // of the largest column norm
   int sweep = 0;
   bool done = false;
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kPairThreads) void k_jacobi_small(const BondTask* _
     ++sweep;
     done = !L.need;
     if (done) break;
-    inner_solve(L, table, pt);
+    inner_solve(L, kRing.rounds, pt);
     asm volatile("" : "+v"(pt));
     {
       const int lane = pt & 63, wave = pt >> 6;
