@@ -198,7 +198,8 @@ int tebd_imag_time_prop(tebd_ctx* ctx, const double* H, int nh, double dtau, int
  * reference's rho2((i-1)d+j,(l-1)d+k)).  rho1 (host, or NULL): L matrices of d x d, element
  * i + d j (FormSingleSiteRho, :95-117).  Tr(O rho) gives any correlator or local value.
  * The environments of all right sites step together in a workspace of at most 4 GiB (or one
- * site's, if that is more), allocated on the first call and freed with the context. */
+ * site's, if that is more; less where memory is short), allocated on the first call and freed
+ * with the context. */
 int tebd_two_point_rdms(tebd_ctx* ctx, const double* phase, double* rho2, double* rho1);
 
 /* Singular-value cutoff on the normalised weight s^2/||theta||^2.  Default
@@ -244,7 +245,7 @@ int tebd_set_profiling(tebd_ctx* ctx, int on);
 int tebd_get_profile(tebd_ctx* ctx, double* out, int n);
 
 /* hipGraph replay of the one-sided Jacobi sweeps (no counterpart in the reference):
- * with on = 1 (the default) each sweep's launches of the large solves (sweep start, and the Gram /
+ * with on = 1 (the default) each sweep's launches of the sweep-by-sweep solves (sweep start, and the Gram /
  * eigenproblem and rotation kernels of its 2P-1 rounds) are captured once per launch
  * shape into an executable graph and replayed, instead of being launched one by one;
  * the convergence test between sweeps stays on the host.  Per-launch profiling
